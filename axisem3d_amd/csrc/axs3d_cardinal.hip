@@ -189,18 +189,13 @@ __device__ __forceinline__ void att_update(double *mvk, Real *dsk, int cs,
 // per block, the Fourier order fastest so that a row's consecutive orders
 // are written by consecutive lanes (CD_EMB = 16 orders: 128-byte runs in
 // FP32).
-// AX: the launch over the axial elements' element-modes (a.em_ax) that
-// forms the strain of their axis row (GLJ, L'Hospital terms) only; the
-// launch over all element-modes leaves those points out, which keeps the
-// axis code and its registers out of the kernel that does nearly all the
-// work.
 // PRT: elements with a particle relabelling transformation (an
 // axisymmetric undulation, one operand set for all slices) write the
 // undulated strain: the 9-component gradient, rotated to RTZ on spherical
 // meshes, through the inverse Jacobian.  The operands do not depend on
 // phi, so applying them to the Fourier coefficients equals applying them
 // slice by slice after the C2R (SolidElement.cpp:139-141).
-template <typename Real, bool ROT, bool AX, bool PRT>
+template <typename Real, bool ROT, bool PRT>
 __global__ __launch_bounds__(CD_EMB_THREADS) void k_cd_grad(CardArgs<Real> a,
                                                          int em0, int em1) {
     __shared__ cpx<Real> sU[CD_EMB][3][NPEM];
@@ -216,7 +211,7 @@ __global__ __launch_bounds__(CD_EMB_THREADS) void k_cd_grad(CardArgs<Real> a,
     int e = 0, alpha = 0;
     cpx<Real> u[3] = {{0, 0}, {0, 0}, {0, 0}};
     if (active) {
-        const EMItem it = (AX ? a.em_ax : s.em_list)[em];
+        const EMItem it = s.em_list[em];
         e = it.elem;
         alpha = it.alpha;
         const int p = s.elem_points[e * NPEM + ipnt];
@@ -232,7 +227,7 @@ __global__ __launch_bounds__(CD_EMB_THREADS) void k_cd_grad(CardArgs<Real> a,
     __syncthreads();
     if (!active) return;
     const bool axial = s.elem_axial[e] != 0;
-    if ((axial && i == 0) != AX) return;
+    const bool row0 = axial && i == 0;
     PointG<Real> G;
     load_point_g<Real>(sG, axial, i, j, G);
     PointOps<Real> g{}, q{};
@@ -240,7 +235,7 @@ __global__ __launch_bounds__(CD_EMB_THREADS) void k_cd_grad(CardArgs<Real> a,
     cpx<Real> eps[6];
     if (PRT && s.prt_idx[e] >= 0) {
         cpx<Real> g9[9];
-        grad9_point<Real>(sU[eml], u, (Real)alpha, AX, i, j, G, g, g9);
+        grad9_point<Real>(sU[eml], u, (Real)alpha, row0, i, j, G, g, g9);
         if (s.rot != nullptr) {
             const Real *r = s.rot + (size_t)e * 4 * NPEM + ipnt;
             rot9<cpx<Real>, Real>(g9, r[0], r[NPEM], r[2 * NPEM],
@@ -249,7 +244,7 @@ __global__ __launch_bounds__(CD_EMB_THREADS) void k_cd_grad(CardArgs<Real> a,
         prt_sph_to_und6<cpx<Real>, Real>(
             g9, s.prt + (size_t)s.prt_idx[e] * 8 * NPEM + ipnt, eps);
     } else {
-        grad6_point<Real>(sU[eml], u, (Real)alpha, AX, i, j, G, g, eps);
+        grad6_point<Real>(sU[eml], u, (Real)alpha, row0, i, j, G, g, eps);
         if (ROT) {
             const Real *r = s.rot + (size_t)e * 4 * NPEM + ipnt;
             rot_spz_rtz6<cpx<Real>, Real>(eps, r[0], r[NPEM], r[2 * NPEM],
@@ -511,21 +506,14 @@ void launch_cd_grad(hipStream_t st, const CardArgs<Real> &a,
     if (gem <= 0) return;
     const bool rot = bt.mtype != 0 && a.s.rot != nullptr;
     const bool prt = a.s.prt_idx != nullptr;
-#define AXS3D_CDG(ROT_, AX_, G_, B_, E_)                                      \
-    do {                                                                      \
-        if (prt)                                                              \
-            hipLaunchKernelGGL((k_cd_grad<Real, ROT_, AX_, true>), dim3(G_),  \
-                               dim3(CD_EMB_THREADS), 0, st, a, B_, E_);       \
-        else                                                                  \
-            hipLaunchKernelGGL((k_cd_grad<Real, ROT_, AX_, false>), dim3(G_), \
-                               dim3(CD_EMB_THREADS), 0, st, a, B_, E_);       \
-    } while (0)
-    if (rot) AXS3D_CDG(true, false, gem, bt.em_begin, bt.em_end);
-    else AXS3D_CDG(false, false, gem, bt.em_begin, bt.em_end);
-    const int gax = (bt.ax_end - bt.ax_begin + CD_EMB - 1) / CD_EMB;
-    if (gax <= 0) return;
-    if (rot) AXS3D_CDG(true, true, gax, bt.ax_begin, bt.ax_end);
-    else AXS3D_CDG(false, true, gax, bt.ax_begin, bt.ax_end);
+#define AXS3D_CDG(ROT_, PRT_)                                                 \
+    hipLaunchKernelGGL((k_cd_grad<Real, ROT_, PRT_>), dim3(gem),              \
+                       dim3(CD_EMB_THREADS), 0, st, a, bt.em_begin,           \
+                       bt.em_end)
+    if (rot && prt) AXS3D_CDG(true, true);
+    else if (rot) AXS3D_CDG(true, false);
+    else if (prt) AXS3D_CDG(false, true);
+    else AXS3D_CDG(false, false);
 #undef AXS3D_CDG
 }
 

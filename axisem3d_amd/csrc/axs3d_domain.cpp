@@ -858,16 +858,12 @@ void DomainBase::finalize() {
         eNu1[e] = nrmax / 2 + 1;
     }
     // Fourier-path element-modes grouped by material type (one launch per
-    // type), in element order within a group, the axial elements last
+    // type), in element order within a group
     for (int mt = 0; mt < 3; mt++) {
         mEMTypeBegin[mt] = (int)em.size();
-        for (int ax = 0; ax < 2; ax++) {
-            if (ax) mEMAxBegin[mt] = (int)em.size();
-            for (int e = 0; e < mNumElems; e++)
-                if (hElemKind[e] != 1 && hMType[e] == mt &&
-                    (hElemAxial[e] != 0) == (ax != 0))
-                    for (int a = 0; a < eNu1[e]; a++) em.push_back({e, a});
-        }
+        for (int e = 0; e < mNumElems; e++)
+            if (hElemKind[e] != 1 && hMType[e] == mt)
+                for (int a = 0; a < eNu1[e]; a++) em.push_back({e, a});
     }
     mEMTypeBegin[3] = (int)em.size();
     mNumEM = (int)em.size();
@@ -1677,7 +1673,6 @@ public:
         a.prt_idx = hPrtElems.empty() ? nullptr : dPrtIdx.as<int32_t>();
         a.prt = hPrtElems.empty() ? nullptr : dPrt.as<Real>();
         for (int k = 0; k < 4; k++) a.em_type_begin[k] = mEMTypeBegin[k];
-        for (int k = 0; k < 3; k++) a.em_ax_begin[k] = mEMAxBegin[k];
         a.point_off = dPointOff.as<uint32_t>();
         a.point_nu1 = dPointNu1.as<int32_t>();
         a.displ = dDispl.as<double>();
@@ -1697,7 +1692,6 @@ public:
         CardArgs<Real> c;
         c.s = stiffArgs();
         c.s.em_list = dEM3D.as<EMItem>();
-        c.em_ax = dEM3DAx.as<EMItem>();
         c.n3d = mNum3D;
         c.list3d = dList3D.as<int32_t>();
         c.elem_nr = dElemNr.as<int32_t>();
@@ -2493,13 +2487,11 @@ private:
     // budget.
     void planCardBatches(size_t bytes, std::vector<CardBatch> &batches,
                          std::vector<uint32_t> &scrOff,
-                         std::vector<EMItem> &em3d,
-                         std::vector<EMItem> &emAx, size_t &scrMax) const {
+                         std::vector<EMItem> &em3d, size_t &scrMax) const {
         const size_t budget =
             std::min(bytes / sizeof(cpx<Real>), (size_t)UINT32_MAX);
         scrOff.assign(mNumElems, 0u);
         em3d.clear();
-        emAx.clear();
         batches.clear();
         scrMax = 0;
         for (int mt = 0; mt < 3; mt++) {
@@ -2511,8 +2503,7 @@ private:
                 if (batches.empty() || batches.back().mtype != mt ||
                     used + need > budget) {
                     batches.push_back(
-                        {mt, w, w, (int)em3d.size(), (int)em3d.size(),
-                         (int)emAx.size(), (int)emAx.size()});
+                        {mt, w, w, (int)em3d.size(), (int)em3d.size()});
                     used = 0;
                 }
                 scrOff[e] = (uint32_t)used;
@@ -2520,11 +2511,8 @@ private:
                 batches.back().nr_max =
                     std::max(batches.back().nr_max, (int)hElemNr[e]);
                 for (int al = 0; al < nu1; al++) em3d.push_back({e, al});
-                if (hElemAxial[e])
-                    for (int al = 0; al < nu1; al++) emAx.push_back({e, al});
                 batches.back().end = w + 1;
                 batches.back().em_end = (int)em3d.size();
-                batches.back().ax_end = (int)emAx.size();
                 scrMax = std::max(scrMax, used);
             }
         }
@@ -2567,7 +2555,7 @@ private:
     // the largest scratch a single element needs; set up at finalize.
     void planStaticBatches() {
         std::vector<uint32_t> off;
-        std::vector<EMItem> em, ax;
+        std::vector<EMItem> em;
         size_t mx = 0;
         mStaticNeedMax = 0;
         for (int32_t e : hList3D)
@@ -2581,8 +2569,7 @@ private:
                                     scr_row(hFElemNr[e] / 2 + 1) *
                                     sizeof(cpx<Real>));
         if (mNum3D > 0) {
-            planCardBatches(STATIC_SCRATCH_BYTES, mCardBatchesS, off, em, ax,
-                            mx);
+            planCardBatches(STATIC_SCRATCH_BYTES, mCardBatchesS, off, em, mx);
             dScrOffS.alloc(off.size() * 4);
             dScrOffS.upload(off.data(), off.size() * 4, mStream);
         }
@@ -2596,17 +2583,13 @@ private:
 
     void buildCardBatches(size_t bytes) {
         std::vector<uint32_t> scrOff;
-        std::vector<EMItem> em3d, emAx;
+        std::vector<EMItem> em3d;
         size_t scrMax = 0;
-        planCardBatches(bytes, mCardBatches, scrOff, em3d, emAx, scrMax);
+        planCardBatches(bytes, mCardBatches, scrOff, em3d, scrMax);
         dScrOff.alloc(scrOff.size() * 4);
         dScrOff.upload(scrOff.data(), scrOff.size() * 4, mStream);
         dEM3D.alloc(em3d.size() * sizeof(EMItem));
         dEM3D.upload(em3d.data(), em3d.size() * sizeof(EMItem), mStream);
-        dEM3DAx.alloc(std::max<size_t>(emAx.size(), 1) * sizeof(EMItem));
-        if (!emAx.empty())
-            dEM3DAx.upload(emAx.data(), emAx.size() * sizeof(EMItem),
-                           mStream);
         scrMax = std::max(scrMax, mFCardScrMax);
         if (scrMax != mCardScrMax || dCardScratch.bytes() == 0) {
             mCardScrMax = scrMax;

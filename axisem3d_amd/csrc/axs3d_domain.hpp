@@ -260,7 +260,6 @@ protected:
     std::vector<int32_t> hPrtElems;     // elements with a PRT
     std::vector<double> hPrtX;          // [n][5][25] X0..X3, XJ
     int mEMTypeBegin[4] = {0, 0, 0, 0};
-    int mEMAxBegin[3] = {0, 0, 0};
     // fluid
     std::vector<int32_t> hFPointNr, hFElemPoints, hFAxial, hFSurf;
     std::vector<double> hFMass, hFElemGQ, hFElemK;
@@ -376,7 +375,6 @@ protected:
     DeviceBuffer dElemNr, dSliceOff, dPropOff, dList3D, dScrOff, dEM3D,
         dPosOff, dPosTab, dMass3DPts, dMass3DOff, dMass3DFlag, dInvMass3D,
         dOceanIdx, dOcean1D, dMass3DKOff, dMass3DK,
-        dEM3DAx,
         dFList3D, dFElemNr, dFK3D, dFK3DOff, dFScrOff, dFEM3D,
         dProp3D,
         dTwiddle,

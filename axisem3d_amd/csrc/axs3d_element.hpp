@@ -100,27 +100,12 @@ __device__ __forceinline__ void grad6_point(const cpx<Real> (*sU)[NPEM],
         eps[3] = cfma(a2, g.invs, eps[3]);
     } else {
         // axis: d/ds of the lower-order numerators (L'Hospital),
-        // computeGrad_1overS_setTo/addTo row 0, :426-437
-        cpx<Real> xa[3] = {{0, 0}, {0, 0}, {0, 0}};
-        cpx<Real> ya[3] = {{0, 0}, {0, 0}, {0, 0}};
-#pragma unroll
-        for (int k = 0; k < NPED; k++) {
-            const cpx<Real> uc0 = sU[0][k * NPED + j];
-            const cpx<Real> uc1 = sU[1][k * NPED + j];
-            const cpx<Real> uc2 = sU[2][k * NPED + j];
-            const cpx<Real> ur0 = sU[0][k];
-            const cpx<Real> ur1 = sU[1][k];
-            const cpx<Real> ur2 = sU[2][k];
-            xa[0] = cfma(csub(ialpha(ralpha, uc0), uc1), G.gxi_col[k], xa[0]);
-            xa[1] = cfma(cadd(ialpha(ralpha, uc1), uc0), G.gxi_col[k], xa[1]);
-            xa[2] = cfma(ialpha(ralpha, uc2), G.gxi_col[k], xa[2]);
-            ya[0] = cfma(csub(ialpha(ralpha, ur0), ur1), G.g_col[k], ya[0]);
-            ya[1] = cfma(cadd(ialpha(ralpha, ur1), ur0), G.g_col[k], ya[1]);
-            ya[2] = cfma(ialpha(ralpha, ur2), G.g_col[k], ya[2]);
-        }
-        eps[5] = cadd(eps[5], cadd(cmul(xa[0], g.dzdeta), cmul(ya[0], g.dzdxii)));
-        eps[1] = cadd(cmul(xa[1], g.dzdeta), cmul(ya[1], g.dzdxii));
-        eps[3] = cadd(eps[3], cadd(cmul(xa[2], g.dzdeta), cmul(ya[2], g.dzdxii)));
+        // computeGrad_1overS_setTo/addTo row 0, :426-437.  d/ds is linear
+        // and i alpha a constant of the order, so d/ds (i alpha u0 - u1) =
+        // i alpha dS[0] - dS[1] and so on: no contraction of its own.
+        eps[5] = cadd(eps[5], csub(ialpha(ralpha, dS[0]), dS[1]));
+        eps[1] = cadd(ialpha(ralpha, dS[1]), dS[0]);
+        eps[3] = cadd(eps[3], ialpha(ralpha, dS[2]));
     }
 }
 
@@ -152,26 +137,10 @@ __device__ __forceinline__ void grad9_point(const cpx<Real> (*sU)[NPEM],
         g9[4] = cmul(cadd(ialpha(ralpha, u[1]), u[0]), g.invs);
         g9[7] = cmul(ialpha(ralpha, u[2]), g.invs);
     } else {
-        cpx<Real> xa[3] = {{0, 0}, {0, 0}, {0, 0}};
-        cpx<Real> ya[3] = {{0, 0}, {0, 0}, {0, 0}};
-#pragma unroll
-        for (int k = 0; k < NPED; k++) {
-            const cpx<Real> uc0 = sU[0][k * NPED + j];
-            const cpx<Real> uc1 = sU[1][k * NPED + j];
-            const cpx<Real> uc2 = sU[2][k * NPED + j];
-            const cpx<Real> ur0 = sU[0][k];
-            const cpx<Real> ur1 = sU[1][k];
-            const cpx<Real> ur2 = sU[2][k];
-            xa[0] = cfma(csub(ialpha(ralpha, uc0), uc1), G.gxi_col[k], xa[0]);
-            xa[1] = cfma(cadd(ialpha(ralpha, uc1), uc0), G.gxi_col[k], xa[1]);
-            xa[2] = cfma(ialpha(ralpha, uc2), G.gxi_col[k], xa[2]);
-            ya[0] = cfma(csub(ialpha(ralpha, ur0), ur1), G.g_col[k], ya[0]);
-            ya[1] = cfma(cadd(ialpha(ralpha, ur1), ur0), G.g_col[k], ya[1]);
-            ya[2] = cfma(ialpha(ralpha, ur2), G.g_col[k], ya[2]);
-        }
-#pragma unroll
-        for (int c = 0; c < 3; c++)
-            g9[3 * c + 1] = cadd(cmul(xa[c], g.dzdeta), cmul(ya[c], g.dzdxii));
+        // L'Hospital, as in grad6_point
+        g9[1] = csub(ialpha(ralpha, g9[0]), g9[3]);
+        g9[4] = cadd(ialpha(ralpha, g9[3]), g9[0]);
+        g9[7] = ialpha(ralpha, g9[6]);
     }
 }
 

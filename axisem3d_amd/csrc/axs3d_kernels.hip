@@ -37,18 +37,13 @@ __device__ __forceinline__ int att_slot_fr(int p, int npa) {
 
 // MT: material type of the element-modes [em0, em1) of em_list (0
 // isotropic, 1 TI, 2 anisotropic); em_list is grouped by type.
-// AX: the element-modes [em0, em1) all belong to axial elements (GLJ in
-// xi, L'Hospital terms on the axis row) or all to non-axial ones; the
-// element-mode list keeps the axial elements of each type at its end, so
-// that the axis code and its registers stay out of the launch that does
-// nearly all the work.
 // PRT: some elements carry a particle relabelling transformation
 // (SolidElement::displToStiff, SolidElement.cpp:115-159): theirs take the
 // 9-component gradient, rotated to RTZ on spherical meshes whatever the
 // material, to the undulated strain (one operand set for all orders: the
 // undulation is axisymmetric), and the stress back through the transpose
 // and computeQuad9.
-template <typename Real, bool ATT, int MT, bool AX, bool PRT>
+template <typename Real, bool ATT, int MT, bool PRT>
 __global__ __launch_bounds__(STIFF_BLOCK) void k_solid_stiff_fr(
     StiffArgs<Real> a, int em0, int em1) {
     __shared__ cpx<Real> sU[EMB][3][NPEM];
@@ -76,7 +71,7 @@ __global__ __launch_bounds__(STIFF_BLOCK) void k_solid_stiff_fr(
         const int p = a.elem_points[e * NPEM + ipnt];
         nu1p = a.point_nu1[p];
         off = a.point_off[p];
-        axial = AX;
+        axial = a.elem_axial[e] != 0;
         if (alpha < nu1p) {
             const double *src = a.displ + (size_t)(off + alpha) * 6;
 #pragma unroll
@@ -724,40 +719,26 @@ void launch_solid_stiff_fr(hipStream_t st, const StiffArgs<Real> &a) {
     // one launch per material type present (em_list grouped by type)
     for (int mt = 0; mt < 3; mt++) {
         const int eb = a.em_type_begin[mt], ee = a.em_type_begin[mt + 1];
-        const int ea = a.em_ax_begin[mt];
         const bool att = a.nsls > 0;
-        for (int ax = 0; ax < 2; ax++) {
-            const int em0 = ax ? ea : eb, em1 = ax ? ee : ea;
-            if (em1 <= em0) continue;
-            const int grid = (em1 - em0 + EMB - 1) / EMB;
+        if (ee <= eb) continue;
+        const int grid = (ee - eb + EMB - 1) / EMB;
 #define AXS3D_FR2(ATT_, MT_, PRT_)                                            \
-    do {                                                                      \
-        if (ax)                                                               \
-            hipLaunchKernelGGL((k_solid_stiff_fr<Real, ATT_, MT_, true,       \
-                                                 PRT_>),                      \
-                               dim3(grid), dim3(STIFF_BLOCK), 0, st, a, em0,  \
-                               em1);                                          \
-        else                                                                  \
-            hipLaunchKernelGGL((k_solid_stiff_fr<Real, ATT_, MT_, false,      \
-                                                 PRT_>),                      \
-                               dim3(grid), dim3(STIFF_BLOCK), 0, st, a, em0,  \
-                               em1);                                          \
-    } while (0)
+    hipLaunchKernelGGL((k_solid_stiff_fr<Real, ATT_, MT_, PRT_>), dim3(grid), \
+                       dim3(STIFF_BLOCK), 0, st, a, eb, ee)
 #define AXS3D_FR(ATT_, MT_)                                                   \
     do {                                                                      \
         if (a.prt_idx != nullptr) AXS3D_FR2(ATT_, MT_, true);                 \
         else AXS3D_FR2(ATT_, MT_, false);                                     \
     } while (0)
-            if (mt == 0) {
-                if (att) AXS3D_FR(true, 0); else AXS3D_FR(false, 0);
-            } else if (mt == 1) {
-                if (att) AXS3D_FR(true, 1); else AXS3D_FR(false, 1);
-            } else {
-                if (att) AXS3D_FR(true, 2); else AXS3D_FR(false, 2);
-            }
+        if (mt == 0) {
+            if (att) AXS3D_FR(true, 0); else AXS3D_FR(false, 0);
+        } else if (mt == 1) {
+            if (att) AXS3D_FR(true, 1); else AXS3D_FR(false, 1);
+        } else {
+            if (att) AXS3D_FR(true, 2); else AXS3D_FR(false, 2);
+        }
 #undef AXS3D_FR
 #undef AXS3D_FR2
-        }
     }
 }
 

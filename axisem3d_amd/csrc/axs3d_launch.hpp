@@ -92,8 +92,6 @@ struct StiffArgs {
     const int32_t *prt_idx = nullptr;
     const Real *prt = nullptr;
     int em_type_begin[4];          // em_list grouped by material type
-    int em_ax_begin[3];            // within type t, the axial elements'
-                                   // element-modes from em_ax_begin[t]
     const uint32_t *point_off;
     const int32_t *point_nu1;
     const double *displ;
@@ -132,7 +130,6 @@ struct CardArgs {
     StiffArgs<Real> s;
     int n3d;                       // number of 3D elements; s.em_list is
                                    // their element-modes in list3d order
-    const EMItem *em_ax;           // the element-modes of the axial ones
     const int32_t *list3d;         // 3D elements grouped by material type,
                                    // each group heaviest first
     int type_begin[4];             // group boundaries in list3d
@@ -343,8 +340,6 @@ void launch_solid_stiff_fr(hipStream_t st, const StiffArgs<Real> &a);
 struct CardBatch {
     int mtype, begin, end;
     int em_begin, em_end;          // its element-modes in the 3D list
-    int ax_begin, ax_end;          // its axial elements' element-modes in
-                                   // the axial list
     int nr_max = 0;                // largest Nr of its elements
 };
 // Default scratch of one batch (bytes).
