@@ -196,8 +196,10 @@ __device__ __forceinline__ void att_update(double *mvk, Real *dsk, int cs,
 // phi, so applying them to the Fourier coefficients equals applying them
 // slice by slice after the C2R (SolidElement.cpp:139-141).
 template <typename Real, bool ROT, bool PRT>
-__global__ __launch_bounds__(CD_EMB_THREADS) void k_cd_grad(CardArgs<Real> a,
-                                                         int em0, int em1) {
+__global__ __launch_bounds__(CD_EMB_THREADS) void k_cd_grad(
+    CardArgs<Real> a, int em0, int em1, StepArgs h) {
+    __shared__ double red[CD_EMB_THREADS / 64][3];
+    if (step_head(h, red)) return;
     __shared__ cpx<Real> sU[CD_EMB][3][NPEM];
     __shared__ Real sG[2][NPEM];
     const StiffArgs<Real> &s = a.s;
@@ -205,7 +207,7 @@ __global__ __launch_bounds__(CD_EMB_THREADS) void k_cd_grad(CardArgs<Real> a,
     if (t < 2 * NPEM) sG[t / NPEM][t % NPEM] = s.gtab[t];
     const int eml = t % CD_EMB;
     const int ipnt = t < CD_EMB * NPEM ? t / CD_EMB : 0;
-    const int em = em0 + xcd_block() * CD_EMB + eml;
+    const int em = em0 + xcd_block(h.rec.nrec) * CD_EMB + eml;
     const bool active = t < CD_EMB * NPEM && em < em1;
     const int i = ipnt / NPED, j = ipnt - (ipnt / NPED) * NPED;
     int e = 0, alpha = 0;
@@ -330,6 +332,7 @@ __global__ __launch_bounds__(CD_EMB_THREADS) void k_cd_quad(CardArgs<Real> a,
                           sY[eml], ipnt, i, j, G, active, F);
     }
     if (active && alpha < s.point_nu1[s.elem_points[e * NPEM + ipnt]]) {
+        add_source(s.src, e, ipnt, alpha, F);
         Real *dst = s.eb + ((size_t)s.elem_eb_off[e] + (size_t)ipnt * nu1 +
                             alpha) * 6;
 #pragma unroll
@@ -501,20 +504,22 @@ static void launch_stress_mt(hipStream_t st, const CardArgs<Real> &a, int w0,
 // group heaviest first) whose strain and stress fit the scratch together.
 template <typename Real>
 void launch_cd_grad(hipStream_t st, const CardArgs<Real> &a,
-                    const CardBatch &bt) {
-    const int gem = (bt.em_end - bt.em_begin + CD_EMB - 1) / CD_EMB;
-    if (gem <= 0) return;
+                    const CardBatch &bt, StepArgs &h) {
+    const int gem =
+        h.rec.nrec + (bt.em_end - bt.em_begin + CD_EMB - 1) / CD_EMB;
+    if (bt.em_end <= bt.em_begin) return;
     const bool rot = bt.mtype != 0 && a.s.rot != nullptr;
     const bool prt = a.s.prt_idx != nullptr;
 #define AXS3D_CDG(ROT_, PRT_)                                                 \
     hipLaunchKernelGGL((k_cd_grad<Real, ROT_, PRT_>), dim3(gem),              \
                        dim3(CD_EMB_THREADS), 0, st, a, bt.em_begin,           \
-                       bt.em_end)
+                       bt.em_end, h)
     if (rot && prt) AXS3D_CDG(true, true);
     else if (rot) AXS3D_CDG(true, false);
     else if (prt) AXS3D_CDG(false, true);
     else AXS3D_CDG(false, false);
 #undef AXS3D_CDG
+    h = StepArgs();
 }
 
 template <typename Real>
@@ -886,9 +891,7 @@ __global__ __launch_bounds__(128) void k_mass3d(Mass3DArgs<Real> a,
             }
         }
     }
-    // bit 0: started from a non-finite displacement, bit 1: left one
-    if (MARCH && (bad0 || bad))
-        atomicOr(a.flag, (bad0 ? 1 : 0) | (bad ? 2 : 0));
+    if (MARCH) raise_flag(a.flag, a.note, bad0, bad);
 }
 
 template <typename Real>
@@ -1292,8 +1295,7 @@ __global__ __launch_bounds__(128) void k_fluid_defer(FluidDeferArgs<Real> a) {
         }
         fs[k] = zero;
     }
-    // bit 0: started from a non-finite potential, bit 1: left one
-    if (bad0 || bad) atomicOr(a.flag, (bad0 ? 1 : 0) | (bad ? 2 : 0));
+    raise_flag(a.flag, a.note, bad0, bad);
 }
 
 template <typename Real>
@@ -1428,7 +1430,7 @@ template int card_blocks_per_cu<float>(bool, int);
 template int card_blocks_per_cu<double>(bool, int);
 #define AXS3D_CD_INST(Real)                                                   \
     template void launch_cd_grad<Real>(hipStream_t, const CardArgs<Real> &, \
-                                       const CardBatch &);                  \
+                                       const CardBatch &, StepArgs &);      \
     template void launch_cd_stress<Real>(hipStream_t,                       \
                                          const CardArgs<Real> &,            \
                                          const CardBatch &);                \

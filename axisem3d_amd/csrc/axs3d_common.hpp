@@ -66,10 +66,11 @@ __device__ __forceinline__ void wave_sync() {
 // a work index such that every XCD takes one contiguous range of the work
 // (a bijection of [0, gridDim.x)): consecutive element-modes of one
 // element and their neighbours, which share GLL points, meet in one L2.
-__device__ __forceinline__ int xcd_block() {
+// first: leading blocks of the launch that do other work.
+__device__ __forceinline__ int xcd_block(int first = 0) {
     constexpr int NXCD = 8;
-    const int b = (int)blockIdx.x;
-    const int n = (int)gridDim.x;
+    const int b = (int)blockIdx.x - first;
+    const int n = (int)gridDim.x - first;
     const int q = n / NXCD, rem = n - q * NXCD;
     const int x = b % NXCD, r = b / NXCD;
     return x * q + (x < rem ? x : rem) + r;

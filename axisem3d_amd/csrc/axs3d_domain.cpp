@@ -1290,6 +1290,32 @@ void DomainBase::finalize() {
         up(dRecW, hRecW.data(), hRecW.size() * 8);
         up(dRecPhi, hRecPhi.data(), hRecPhi.size() * 8);
         if (!hRecRot.empty()) up(dRecRot, hRecRot.data(), hRecRot.size() * 8);
+        // the points with a weight, and the orders' phase factors
+        std::vector<RecPoint> pts((size_t)mNumRec * NPEM, RecPoint{0, 0, 0.});
+        std::vector<int32_t> npt(mNumRec, 0), rnu1(mNumRec);
+        std::vector<int64_t> coff(mNumRec);
+        std::vector<double2> cis;
+        for (int r = 0; r < mNumRec; r++) {
+            const int e = hRecElem[r];
+            for (int k = 0; k < NPEM; k++) {
+                const double w = hRecW[(size_t)r * NPEM + k];
+                if (std::fabs(w) < 2.220446049250313e-16) continue;
+                const int p = hElemPoints[(size_t)e * NPEM + k];
+                pts[(size_t)r * NPEM + npt[r]++] = {off[p], nu1[p], w};
+            }
+            rnu1[r] = eNu1[e];
+            coff[r] = (int64_t)cis.size();
+            for (int a = 0; a < eNu1[e]; a++) {
+                const double f = a == 0 ? 1. : 2.;
+                cis.push_back(make_double2(f * std::cos(a * hRecPhi[r]),
+                                           f * std::sin(a * hRecPhi[r])));
+            }
+        }
+        up(dRecPts, pts.data(), pts.size() * sizeof(RecPoint));
+        up(dRecNpt, npt.data(), npt.size() * 4);
+        up(dRecNu1, rnu1.data(), rnu1.size() * 4);
+        up(dRecCis, cis.data(), cis.size() * sizeof(double2));
+        up(dRecCisOff, coff.data(), coff.size() * 8);
         dSeismo.alloc((size_t)std::max(hMaxSamples, 1) * mNumRec * 3 * 8);
         dSeismo.zero(st);
     }
@@ -1346,9 +1372,7 @@ void DomainBase::finalize() {
         }
     }
     {
-        // [0] raised on a non-finite displacement, [1] the first step
-        // after which it was up
-        const int flag0[2] = {0, -1};
+        const int flag0[FLAG_WORDS] = {0, -1, 0};
         dFlag.alloc(sizeof(flag0));
         dFlag.upload(flag0, sizeof(flag0), st);
     }
@@ -1360,21 +1384,33 @@ void DomainBase::finalize() {
     autotune();
 }
 
-void DomainBase::recordOutput(int isample, bool dev) {
+// The receivers of a step: sample isample, or with dev the one the device
+// step counter gives; none outside the seismogram buffer.
+RecordArgs DomainBase::recordArgs(int isample, bool dev) const {
+    RecordArgs a;
+    if (mNumRec == 0 || (!dev && (isample < 0 || isample >= hMaxSamples)))
+        return a;
+    a.nrec = mNumRec;
+    a.pts = dRecPts.as<RecPoint>();
+    a.npt = dRecNpt.as<int32_t>();
+    a.nu1 = dRecNu1.as<int32_t>();
+    a.cis = dRecCis.as<double2>();
+    a.cis_off = dRecCisOff.as<int64_t>();
+    a.rot = hRecRot.empty() ? nullptr : dRecRot.as<double>();
+    a.displ = dDispl.as<double>();
+    a.out = dSeismo.as<double>() + (dev ? 0 : (size_t)isample * mNumRec * 3);
+    a.ctr = dev ? dStepCtr.as<int>() : nullptr;
+    a.max_samples = hMaxSamples;
+    return a;
+}
+
+void DomainBase::recordOutput(int isample) {
     requireFinalized("Domain::recordOutput");
     if (mNumRec == 0) return;
-    if (!dev && (isample < 0 || isample >= hMaxSamples))
+    if (isample < 0 || isample >= hMaxSamples)
         throw Error("Domain::recordOutput || Sample index out of range.");
     tick(AXS3D_KERNEL_RECORD);
-    launch_record(mStream, mNumRec, dRecElem.as<int32_t>(),
-                  dRecW.as<double>(), dRecPhi.as<double>(),
-                  dElemPoints.as<int32_t>(), dElemNu1.as<int32_t>(),
-                  dPointOff.as<uint32_t>(), dPointNu1.as<int32_t>(),
-                  dDispl.as<double>(),
-                  dSeismo.as<double>() +
-                      (dev ? 0 : (size_t)isample * mNumRec * 3),
-                  dev ? dStepCtr.as<int>() : nullptr, hMaxSamples,
-                  hRecRot.empty() ? nullptr : dRecRot.as<double>());
+    launch_record(mStream, recordArgs(isample, false));
     tock(AXS3D_KERNEL_RECORD);
 }
 
@@ -1733,6 +1769,8 @@ public:
         g.scheme = mScheme;
         g.sym_pi = mSymPi;
         g.sym_kappa = mSymKappa;
+        g.note = mNote;
+        g.ctr = mAdvance ? dStepCtr.as<int>() : nullptr;
         return g;
     }
     // absorbing boundaries: what the point kernels read, the terms' kernel
@@ -1821,6 +1859,7 @@ public:
         m.scheme = mScheme;
         m.sym_pi = mSymPi;
         m.sym_kappa = mSymKappa;
+        m.note = mNote;
         return m;
     }
     PointGeom fluidGeom() const {
@@ -1837,6 +1876,7 @@ public:
         g.scheme = mScheme;
         g.sym_pi = mSymPi;
         g.sym_kappa = mSymKappa;
+        g.note = mNote;
         return g;
     }
     FluidDeferArgs<Real> fluidDeferArgs() const {
@@ -1874,6 +1914,7 @@ public:
         f.scheme = mScheme;
         f.sym_pi = mSymPi;
         f.sym_kappa = mSymKappa;
+        f.note = mNote;
         return f;
     }
     CouplingGeom couplingGeom() const {
@@ -1929,18 +1970,60 @@ public:
         return c;
     }
 
+    // The moment sources of step tstep (with dev: of the step counter's).
+    SourceArgs<Real> sourceArgs(int tstep, bool dev) const {
+        SourceArgs<Real> s;
+        if (hSrcElem < 0) return s;
+        if (!dev && (tstep < 0 || tstep >= mStfSteps))
+            throw Error("Domain::applySources || Step outside the STF.");
+        s.idx = dSrcIdx.as<int32_t>();
+        s.force = dSrcForce.as<cpx<Real>>();
+        s.off = dSrcOff.as<int64_t>();
+        s.nu1 = dSrcNu1.as<int32_t>();
+        s.stf = dStf.as<double>();
+        s.nstf = mStfSteps;
+        s.ctr = dev ? dStepCtr.as<int>() : nullptr;
+        s.tstep = tstep;
+        return s;
+    }
+
     // Domain::applySources: the source force is subtracted from the point
     // stiffness (stage form).
     void applySources(int tstep) override {
         requireFinalized("Domain::applySources");
-        sourceKernel(tstep, false);
+        if (hSrcElem < 0) return;
+        StiffArgs<Real> sa = stiffArgs();
+        sa.src = sourceArgs(tstep, false);
+        tick(AXS3D_KERNEL_SOURCE);
+        for (size_t i = 0; i < hSrcElems.size(); i++)
+            launch_apply_source<Real>(mStream, sa, hSrcElems[i], (int)i,
+                                      mSrcNu1c[i], dStiff.as<Real>());
+        tock(AXS3D_KERNEL_SOURCE);
     }
 
-    void sourceKernel(int tstep, bool toElem, bool dev = false) {
+    // The forces of every source for a unit source time function.
+    void sourceForces() {
         if (hSrcElem < 0) return;
-        if (!dev && (tstep < 0 || tstep >= mStfSteps))
-            throw Error("Domain::applySources || Step outside the STF.");
-        tick(AXS3D_KERNEL_SOURCE);
+        std::vector<Real> pat(hSrcPattern.begin(), hSrcPattern.end());
+        DeviceBuffer pattern;
+        pattern.alloc(pat.size() * sizeof(Real));
+        pattern.upload(pat.data(), pat.size() * sizeof(Real), mStream);
+        std::vector<int32_t> idx(mNumElems, -1);
+        std::vector<int64_t> off;
+        int64_t total = 0;
+        for (size_t i = 0; i < hSrcElems.size(); i++) {
+            idx[hSrcElems[i]] = (int32_t)i;
+            off.push_back(total);
+            total += (int64_t)mSrcNu1c[i] * NPEM * 3;
+        }
+        dSrcIdx.alloc(idx.size() * 4);
+        dSrcIdx.upload(idx.data(), idx.size() * 4, mStream);
+        dSrcOff.alloc(off.size() * 8);
+        dSrcOff.upload(off.data(), off.size() * 8, mStream);
+        dSrcNu1.alloc(mSrcNu1c.size() * 4);
+        dSrcNu1.upload(mSrcNu1c.data(), mSrcNu1c.size() * 4, mStream);
+        dSrcForce.alloc((size_t)std::max<int64_t>(total, 1) *
+                        sizeof(cpx<Real>));
         const StiffArgs<Real> sa = stiffArgs();
         for (size_t i = 0; i < hSrcElems.size(); i++) {
             // the source element's PRT operands (X0..X3 unscaled), if any
@@ -1948,25 +2031,26 @@ public:
             for (size_t k = 0; k < hPrtElems.size(); k++)
                 if (hPrtElems[k] == hSrcElems[i])
                     prt_e = dPrt.as<Real>() + k * 8 * NPEM;
-            launch_moment_source<Real>(
-                mStream, toElem, sa, hSrcElems[i], mSrcNu1c[i],
-                dSrcPattern.as<Real>() + 2 * hSrcPatOff[i],
-                dStf.as<double>() + i * (size_t)mStfSteps, tstep, mStfSteps,
-                dev ? dStepCtr.as<int>() : nullptr, dStiff.as<Real>(), prt_e);
+            launch_source_forces<Real>(
+                mStream, sa, hSrcElems[i], mSrcNu1c[i],
+                pattern.as<Real>() + 2 * hSrcPatOff[i], prt_e,
+                dSrcForce.as<cpx<Real>>() + off[i]);
         }
-        tock(AXS3D_KERNEL_SOURCE);
+        hip_check(hipStreamSynchronize(mStream), "Domain::finalize");
     }
 
     // The cardinal path, batch by batch; with timing, each of the three
     // kernels is timed under its own id.
     void cardinalPath(bool timed) {
-        cardinalPathOn(cardArgs(), mCardBatches, timed);
+        StepArgs h;
+        cardinalPathOn(cardArgs(), mCardBatches, timed, h);
     }
     void cardinalPathOn(const CardArgs<Real> &c,
-                        const std::vector<CardBatch> &batches, bool timed) {
+                        const std::vector<CardBatch> &batches, bool timed,
+                        StepArgs &h) {
         for (const CardBatch &bt : batches) {
             if (timed) tick(AXS3D_KERNEL_CD_GRAD);
-            launch_cd_grad<Real>(mStream, c, bt);
+            launch_cd_grad<Real>(mStream, c, bt, h);
             if (timed) {
                 tock(AXS3D_KERNEL_CD_GRAD);
                 tick(AXS3D_KERNEL_CD_STRESS);
@@ -1982,23 +2066,27 @@ public:
     }
 
     // The element kernels; with stat, the cardinal paths run through the
-    // static scratch in the batches planned for it.
-    void elementKernel(bool stat = false) {
+    // static scratch in the batches planned for it.  In a bulk step h (the
+    // receivers and the step's number) rides on the first of them and src
+    // on those that write the source elements' forces.
+    void elementKernel(bool stat = false, StepArgs h = StepArgs(),
+                       const SourceArgs<Real> &src = SourceArgs<Real>()) {
         if (mNumEM > 0) {
             tick(AXS3D_KERNEL_STIFFNESS);
-            launch_solid_stiff_fr<Real>(mStream, stiffArgs());
+            StiffArgs<Real> sa = stiffArgs();
+            sa.src = src;
+            launch_solid_stiff_fr<Real>(mStream, sa, h);
             tock(AXS3D_KERNEL_STIFFNESS);
         }
         if (mNum3D > 0) {
             tick(AXS3D_KERNEL_STIFFNESS_3D);
+            CardArgs<Real> c = cardArgs();
+            c.s.src = src;
             if (stat) {
-                CardArgs<Real> c = cardArgs();
                 c.scratch = static_cast<Real *>(mStaticScratch);
                 c.scr_off = dScrOffS.as<uint32_t>();
-                cardinalPathOn(c, mCardBatchesS, true);
-            } else {
-                cardinalPath(true);
             }
+            cardinalPathOn(c, stat ? mCardBatchesS : mCardBatches, true, h);
             tock(AXS3D_KERNEL_STIFFNESS_3D);
         }
         if (mNumFEM > 0 || mNumF3D > 0) {
@@ -2159,39 +2247,54 @@ public:
     }
 
     // One Newmark step in its bulk form: the element kernels write the
-    // element-local forces, the source adds into its element's, the
-    // receivers sample u(t), then one fluid and one solid point kernel
-    // gather, couple, mask, divide by the mass and march.
+    // element-local forces (the source's among its element's) and sample
+    // the receivers from u(t), then one fluid and one solid point kernel
+    // gather, couple, mask, divide by the mass and march; the last of them
+    // advances the step counter.
     void step(int tstep, int isample, bool dev) override {
         const int all = PHASE_GATHER | PHASE_AXIAL | PHASE_MASS | PHASE_MARCH;
+        StepArgs h;
+        h.flag = dFlag.as<int>();
+        h.ctr = dev ? dStepCtr.as<int>() : nullptr;
+        h.tstep = tstep;
+        // bookkeeping of this step's point kernels only
+        struct Bulk {
+            bool &note, &advance;
+            ~Bulk() { note = advance = false; }
+        } bulk{mNote, mAdvance};
+        mNote = true;
         if (mScheme == 1) {
             // SymplecticTimeScheme::solve (SymplecticTimeScheme.cpp:30-
             // 103): record, source (into the first sub-step's forces),
             // launch, then four sub-steps of stiffness, boundaries, mass
             // and update
-            if (dev || isample >= 0) recordOutput(isample, dev);
+            const RecordArgs rec = recordArgs(isample, dev);
+            if (rec.nrec > 0) {
+                tick(AXS3D_KERNEL_RECORD);
+                launch_record(mStream, rec);
+                tock(AXS3D_KERNEL_RECORD);
+            }
             symplecticLaunch();
             for (int isub = 1; isub <= 4; isub++) {
-                elementKernel();
-                if (isub == 1) sourceKernel(tstep, true, dev);
+                if (isub == 1)
+                    elementKernel(false, h, sourceArgs(tstep, dev));
+                else
+                    elementKernel();
                 abcKernel();
                 mSymPi = symPi(isub);
                 mSymKappa = symKappa(isub);
                 fluidPoint(all | PHASE_COUPLE);
+                mAdvance = dev && isub == 4;
                 point(all | PHASE_COUPLE);
             }
         } else {
-            elementKernel();
-            sourceKernel(tstep, true, dev);
-            if (dev || isample >= 0) recordOutput(isample, dev);
+            h.rec = recordArgs(isample, dev);
+            elementKernel(false, h, sourceArgs(tstep, dev));
             abcKernel();
             fluidPoint(all | PHASE_COUPLE);
+            mAdvance = dev;
             point(all | PHASE_COUPLE);
         }
-        if (dev)
-            launch_step_advance(mStream, dStepCtr.as<int>(), dFlag.as<int>());
-        else
-            launch_flag_note(mStream, dFlag.as<int>(), tstep);
     }
 
     // Discrete adjoint of the bulk step (see axs3d_adjoint.hip for the
@@ -2367,8 +2470,9 @@ public:
                     cb.s.displ = su + (size_t)(n - n0) * nd;
                     cb.scratch = dAdjScrB.as<Real>();
                     for (const CardBatch &bt : mCardBatches) {
-                        launch_cd_grad<Real>(mStream, ca, bt);
-                        launch_cd_grad<Real>(mStream, cb, bt);
+                        StepArgs none;
+                        launch_cd_grad<Real>(mStream, ca, bt, none);
+                        launch_cd_grad<Real>(mStream, cb, bt, none);
                         launch_cd_sens<Real>(mStream, ca, cb.scratch, bt,
                                              dAdjGQ.as<double>(),
                                              dAdjKern3D.as<double>(), -dt2);
@@ -2977,11 +3081,7 @@ private:
         planStaticBatches();
         abcReal(mAbcS, mAbcSD);
         abcReal(mAbcF, mAbcFD);
-        if (hSrcElem >= 0) {
-            std::vector<Real> pat(hSrcPattern.begin(), hSrcPattern.end());
-            dSrcPattern.alloc(pat.size() * sizeof(Real));
-            dSrcPattern.upload(pat.data(), pat.size() * sizeof(Real), st);
-        }
+        sourceForces();
     }
 };
 

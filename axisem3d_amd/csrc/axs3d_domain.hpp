@@ -146,8 +146,7 @@ public:
     // on that scratch.
     virtual void computeStiffnessStatic() = 0;
     virtual void applyBC_BeforeAssemblingStiff() = 0;
-    // isample < 0 with dev: the sample follows the device step counter
-    void recordOutput(int isample, bool dev = false);
+    void recordOutput(int isample);
     virtual void applyBC_AfterAssemblingStiff() = 0;
     // Domain::applyBC_AfterComputingAccel (Domain.cpp:330-332): sponge
     virtual void applyBC_AfterComputingAccel() = 0;
@@ -398,7 +397,14 @@ protected:
         dFInvMass3D, dCpl3DSolid, dCpl3DNOff, dCpl3DNu, dCpl3DNam,
         dCpl3DCOff, dCplSolidPair3D, dCSolid3D;
     // device: source and receivers
-    DeviceBuffer dSrcPattern, dStf, dRecElem, dRecW, dRecPhi, dSeismo;
+    DeviceBuffer dSrcForce, dSrcIdx, dSrcOff, dSrcNu1, dStf, dRecElem, dRecW,
+        dRecPhi, dSeismo;
+    // receivers as the record kernels read them (RecordArgs)
+    DeviceBuffer dRecPts, dRecNpt, dRecNu1, dRecCis, dRecCisOff;
+    RecordArgs recordArgs(int isample, bool dev) const;
+    // step bookkeeping of the bulk kernels: whether blown-up steps are
+    // noted, and whether the next solid point kernel advances the counter
+    bool mNote = false, mAdvance = false;
     // station frames: [receiver][6] two rotations (axis, cos, sin)
     std::vector<double> hRecRot;
     DeviceBuffer dRecRot;
@@ -423,7 +429,7 @@ protected:
     // nrOf(p); w1 = 1D Clayton width
     int abcRecord(AbcHost &h, int npoints, int p, int w1);
     DeviceBuffer dPointDt;
-    DeviceBuffer dFlag;
+    DeviceBuffer dFlag;                 // FlagWord
     DeviceBuffer dStepCtr;              // [0] step, [1] first recorded step
     // adjoint: FP64 operators, densities, adjoint fields, checkpoints and
     // the forward fields of one segment

@@ -174,6 +174,7 @@ struct FluidPointArgs {
     AbcGeom abc;                   // Clayton and sponge terms (k_abc)
     int scheme;                    // 0 Newmark, 1 symplectic sub-step
     double sym_pi, sym_kappa;
+    bool note;                     // bulk step: see PointGeom
 };
 
 // Fluid point update, one thread per (point, order), phases as for the
@@ -271,7 +272,7 @@ __global__ __launch_bounds__(256) void k_fluid_point(
         const bool bad = !isfinite(ur) || !isfinite(ui);
         const bool bad0 = !isfinite(u0.x) || !isfinite(u0.y);
         if (!GATHER) stiff[(size_t)k * 2] = stiff[(size_t)k * 2 + 1] = 0;
-        if (bad0 || bad) atomicOr(a.flag, (bad0 ? 1 : 0) | (bad ? 2 : 0));
+        raise_flag(a.flag, a.note, bad0, bad);
         return;
     }
     // all three loaded (16-byte vectors) before anything is stored
@@ -286,8 +287,7 @@ __global__ __launch_bounds__(256) void k_fluid_point(
     const bool bad = !isfinite(ur) || !isfinite(ui);
     const bool bad0 = !isfinite(u0.x) || !isfinite(u0.y);
     if (!GATHER) stiff[(size_t)k * 2] = stiff[(size_t)k * 2 + 1] = 0;
-    // bit 0: started from a non-finite potential, bit 1: left one
-    if (bad0 || bad) atomicOr(a.flag, (bad0 ? 1 : 0) | (bad ? 2 : 0));
+    raise_flag(a.flag, a.note, bad0, bad);
 }
 
 template <typename Real>
@@ -337,6 +337,7 @@ void launch_fluid_point(hipStream_t st, int phases, const PointGeom &g,
     a.scheme = g.scheme;
     a.sym_pi = g.sym_pi;
     a.sym_kappa = g.sym_kappa;
+    a.note = g.note;
     if (cpl.n_pairs <= 0 && g.abc.idx == nullptr) phases &= ~PHASE_COUPLE;
     if (g.abc.idx == nullptr) phases &= ~PHASE_SPONGE;
     if (phases == 0) return;

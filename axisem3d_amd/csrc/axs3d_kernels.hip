@@ -45,7 +45,9 @@ __device__ __forceinline__ int att_slot_fr(int p, int npa) {
 // and computeQuad9.
 template <typename Real, bool ATT, int MT, bool PRT>
 __global__ __launch_bounds__(STIFF_BLOCK) void k_solid_stiff_fr(
-    StiffArgs<Real> a, int em0, int em1) {
+    StiffArgs<Real> a, int em0, int em1, StepArgs h) {
+    __shared__ double red[STIFF_BLOCK / 64][3];
+    if (step_head(h, red)) return;
     __shared__ cpx<Real> sU[EMB][3][NPEM];
     __shared__ cpx<Real> sX[EMB][3][NPEM];
     __shared__ cpx<Real> sY[EMB][3][NPEM];
@@ -55,7 +57,7 @@ __global__ __launch_bounds__(STIFF_BLOCK) void k_solid_stiff_fr(
     if (t < 2 * NPEM) sG[t / NPEM][t % NPEM] = a.gtab[t];
     const int eml = t / NPEM;
     const int ipnt = t - eml * NPEM;
-    const int em = em0 + xcd_block() * EMB + eml;
+    const int em = em0 + xcd_block(h.rec.nrec) * EMB + eml;
     const bool active = (eml < EMB) && (em < em1);
     const int i = ipnt / NPED, j = ipnt - (ipnt / NPED) * NPED;
     const int emx = active ? eml : 0;
@@ -199,6 +201,7 @@ __global__ __launch_bounds__(STIFF_BLOCK) void k_solid_stiff_fr(
                           i, j, G, active, F);
     }
     if (active && alpha < nu1p) {
+        add_source(a.src, e, ipnt, alpha, F);
         Real *dst = a.eb + ((size_t)a.elem_eb_off[e] +
                             (size_t)ipnt * a.elem_nu1[e] + alpha) * 6;
 #pragma unroll
@@ -209,48 +212,32 @@ __global__ __launch_bounds__(STIFF_BLOCK) void k_solid_stiff_fr(
     }
 }
 
-// Moment source: stress = -pattern * stf (SolidElement.cpp:279-280), then
-// computeQuad6_NoIntegration (GradientQuadrature.hpp:363-390) and the
-// subtracting scatter.  One thread per (alpha < nu1c, GLL point).  With
-// TO_ELEM the force is added to the source element's element-local force
-// (gathered later with the element stiffness), otherwise it is subtracted
-// from the point stiffness.  The points of one element are distinct, so
-// neither form races.
-template <typename Real, bool TO_ELEM>
-__global__ __launch_bounds__(STIFF_BLOCK) void k_moment_source(
-    int elem, int nu1c, const Real *__restrict__ pattern, const double *stf,
-    int tstep, int nstf, const int *__restrict__ step_ctr,
-    const int32_t *__restrict__ elem_points,
-    const uint8_t *__restrict__ elem_axial, const Real *__restrict__ elem_ops,
-    const uint32_t *__restrict__ point_off,
-    const int32_t *__restrict__ point_nu1, Real *__restrict__ stiff,
-    const uint32_t *__restrict__ elem_eb_off,
-    const int32_t *__restrict__ elem_nu1, Real *__restrict__ eb,
-    const Real *__restrict__ gtab, const Real *__restrict__ prt_e,
-    const Real *__restrict__ rot_e) {
+// Moment source for a unit source time function: stress = -pattern
+// (SolidElement.cpp:279-280), then computeQuad6_NoIntegration
+// (GradientQuadrature.hpp:363-390), into force [alpha][25][3].  One thread
+// per (alpha < nu1c, GLL point); runs once, at finalize.
+template <typename Real>
+__global__ __launch_bounds__(STIFF_BLOCK) void k_source_forces(
+    StiffArgs<Real> a, int elem, int nu1c, const Real *__restrict__ pattern,
+    const Real *__restrict__ prt_e, cpx<Real> *__restrict__ force) {
     __shared__ cpx<Real> sX[EMB][3][NPEM];
     __shared__ cpx<Real> sY[EMB][3][NPEM];
     __shared__ Real sG[2][NPEM];
-    // a replayed step takes its index from the device counter; outside
-    // the STF the whole block leaves before the first barrier
-    if (step_ctr) tstep = step_ctr[0];
-    if (tstep < 0 || tstep >= nstf) return;
     const int t = threadIdx.x;
-    if (t < 2 * NPEM) sG[t / NPEM][t % NPEM] = gtab[t];
+    if (t < 2 * NPEM) sG[t / NPEM][t % NPEM] = a.gtab[t];
     __syncthreads();
     const int eml = t / NPEM;
     const int ipnt = t - eml * NPEM;
     const int alpha = blockIdx.x * EMB + eml;
     const bool active = (eml < EMB) && (alpha < nu1c);
     const int i = ipnt / NPED, j = ipnt - (ipnt / NPED) * NPED;
-    const bool axial = elem_axial[elem] != 0;
+    const bool axial = a.elem_axial[elem] != 0;
     PointG<Real> G;
     load_point_g<Real>(sG, axial, i, j, G);
     PointOps<Real> q{};
     cpx<Real> sig[6];
-    const Real sv = (Real)stf[tstep];
     if (active) {
-        const Real *ops = elem_ops + (size_t)elem * ELEM_OPS * NPEM + ipnt;
+        const Real *ops = a.elem_ops + (size_t)elem * ELEM_OPS * NPEM + ipnt;
         q.dsdxii = ops[OP_DSDXII * NPEM];
         q.dsdeta = ops[OP_DSDETA * NPEM];
         q.dzdxii = ops[OP_DZDXII * NPEM];
@@ -258,11 +245,8 @@ __global__ __launch_bounds__(STIFF_BLOCK) void k_moment_source(
         q.invs = ops[OP_INVS * NPEM];
         const Real *pat = pattern + ((size_t)alpha * 6 * NPEM + ipnt) * 2;
 #pragma unroll
-        for (int k = 0; k < 6; k++) {
-            const Real re = pat[k * NPEM * 2] * sv;
-            const Real im = pat[k * NPEM * 2 + 1] * sv;
-            sig[k] = {-re, -im};
-        }
+        for (int k = 0; k < 6; k++)
+            sig[k] = {-pat[k * NPEM * 2], -pat[k * NPEM * 2 + 1]};
     }
     cpx<Real> F[3], L[3];
     const int emx = active ? eml : 0;
@@ -271,6 +255,8 @@ __global__ __launch_bounds__(STIFF_BLOCK) void k_moment_source(
         // strain rotation with doubled shears, to the spherical tensor with
         // the unscaled inverse Jacobian, back to SPZ, computeQuad9_
         // NoIntegration
+        const Real *rot_e =
+            a.rot != nullptr ? a.rot + (size_t)elem * 4 * NPEM : nullptr;
         Real rs1 = 0, rc1 = 1, rs2 = 0, rc2 = 1;
         if (rot_e != nullptr) {
             rs1 = rot_e[ipnt];
@@ -294,27 +280,33 @@ __global__ __launch_bounds__(STIFF_BLOCK) void k_moment_source(
                          sY[emx], ipnt, L);
     }
     __syncthreads();
-    if (active) quad6_finish<Real>(sX[emx], sY[emx], i, j, G, L, F);
-    if (active) {
-        const int p = elem_points[elem * NPEM + ipnt];
-        if (alpha < point_nu1[p]) {
-            if (TO_ELEM) {
-                Real *dst = eb + ((size_t)elem_eb_off[elem] +
-                                  (size_t)ipnt * elem_nu1[elem] + alpha) * 6;
+    if (!active) return;
+    quad6_finish<Real>(sX[emx], sY[emx], i, j, G, L, F);
+    cpx<Real> *dst = force + ((size_t)alpha * NPEM + ipnt) * 3;
 #pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    dst[2 * c] += F[c].re;
-                    dst[2 * c + 1] += F[c].im;
-                }
-            } else {
-                Real *dst = stiff + (size_t)(point_off[p] + alpha) * 6;
+    for (int c = 0; c < 3; c++) dst[c] = F[c];
+}
+
+// Domain::applySources (stage form): source src of element elem subtracted
+// from the point stiffness.  The points of one element are distinct, so
+// nothing races.
+template <typename Real>
+__global__ __launch_bounds__(256) void k_apply_source(
+    StiffArgs<Real> a, int elem, int src, int nu1c, Real *__restrict__ stiff) {
+    const int x = blockIdx.x * blockDim.x + threadIdx.x;
+    const int alpha = x / NPEM, ipnt = x - (x / NPEM) * NPEM;
+    const SourceArgs<Real> &s = a.src;
+    if (alpha >= nu1c || s.tstep < 0 || s.tstep >= s.nstf) return;
+    const int p = a.elem_points[elem * NPEM + ipnt];
+    if (alpha >= a.point_nu1[p]) return;
+    const Real v = (Real)s.stf[(size_t)src * s.nstf + s.tstep];
+    const cpx<Real> *f =
+        s.force + s.off[src] + ((size_t)alpha * NPEM + ipnt) * 3;
+    Real *dst = stiff + (size_t)(a.point_off[p] + alpha) * 6;
 #pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    dst[2 * c] -= F[c].re;
-                    dst[2 * c + 1] -= F[c].im;
-                }
-            }
-        }
+    for (int c = 0; c < 3; c++) {
+        dst[2 * c] -= f[c].re * v;
+        dst[2 * c + 1] -= f[c].im * v;
     }
 }
 
@@ -417,6 +409,8 @@ struct PointArgs {
     AbcGeom abc;
     int scheme;                   // 0 Newmark, 1 symplectic sub-step
     double sym_pi, sym_kappa;
+    bool note;                    // bulk step: see PointGeom
+    int *ctr;
 };
 
 //   COUPLE the Clayton-Enquist boundaries (AbsorbingBoundary::
@@ -434,6 +428,8 @@ __global__ __launch_bounds__(256) void k_point(PointArgs a,
                                                Real *__restrict__ stiff) {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= a.n_modes) return;
+    if (GATHER && a.ctr != nullptr && k == 0)
+        a.ctr[0] = a.flag[FLAG_STEP] + 1;
     const int p = a.mode_point[k];
     const int alpha = (int)(k - (int64_t)a.point_off[p]);
     const int ai = a.abc.idx != nullptr ? a.abc.idx[p] : -1;
@@ -585,7 +581,7 @@ __global__ __launch_bounds__(256) void k_point(PointArgs a,
 #pragma unroll
             for (int q = 0; q < 6; q++) stiff[(size_t)k * 6 + q] = 0;
         }
-        if (bad0 || bad) atomicOr(a.flag, (bad0 ? 1 : 0) | (bad ? 2 : 0));
+        raise_flag(a.flag, a.note, bad0, bad);
         return;
     }
 #pragma unroll
@@ -617,10 +613,7 @@ __global__ __launch_bounds__(256) void k_point(PointArgs a,
 #pragma unroll
         for (int q = 0; q < 6; q++) stiff[(size_t)k * 6 + q] = 0;
     }
-    // bit 0: the displacement this step started from was non-finite (what
-    // Domain::checkStability sees at the start of a step); bit 1: the one
-    // it leaves is
-    if (bad0 || bad) atomicOr(a.flag, (bad0 ? 1 : 0) | (bad ? 2 : 0));
+    raise_flag(a.flag, a.note, bad0, bad);
 }
 
 
@@ -640,91 +633,27 @@ void launch_sym_launch(hipStream_t st, double *u, const double *v, int64_t n,
                        dim3(256), 0, st, u, v, n, kdt);
 }
 
-// Receivers: one wave64 per station.  In-plane weighted sum over the
-// non-zero weights, then Re sum_alpha c_alpha x_alpha e^{i alpha phi}
-// with c_0 = 1 and c_alpha = 2 (Station.hpp:53-73, eigen_tools.hpp:79-106).
-__global__ __launch_bounds__(64) void k_record(
-    int nrec, const int32_t *__restrict__ rec_elem,
-    const double *__restrict__ rec_w, const double *__restrict__ rec_phi,
-    const int32_t *__restrict__ elem_points,
-    const int32_t *__restrict__ elem_nu1,
-    const uint32_t *__restrict__ point_off,
-    const int32_t *__restrict__ point_nu1, const double *__restrict__ displ,
-    double *__restrict__ out, const int *__restrict__ step_ctr,
-    int max_samples, const double *__restrict__ rec_rot) {
-    const int r = blockIdx.x;
-    if (r >= nrec) return;
-    // a replayed step: sample = step - first recorded step (counter words
-    // 0 and 1), nothing outside the seismogram buffer
-    if (step_ctr) {
-        const int isample = step_ctr[0] - step_ctr[1];
-        if (isample < 0 || isample >= max_samples) return;
-        out += (size_t)isample * nrec * 3;
-    }
-    const int lane = threadIdx.x;
-    const int e = rec_elem[r];
-    const int nu1 = elem_nu1[e];
-    const double phi = rec_phi[r];
-    double acc[3] = {0, 0, 0};
-    for (int alpha = lane; alpha < nu1; alpha += 64) {
-        double xr[3] = {0, 0, 0}, xi[3] = {0, 0, 0};
-        for (int p = 0; p < NPEM; p++) {
-            const double w = rec_w[r * NPEM + p];
-            if (fabs(w) < 2.220446049250313e-16) continue;
-            const int ip = elem_points[e * NPEM + p];
-            if (alpha >= point_nu1[ip]) continue;
-            const double *u = displ + (size_t)(point_off[ip] + alpha) * 6;
-#pragma unroll
-            for (int c = 0; c < 3; c++) {
-                xr[c] += u[2 * c] * w;
-                xi[c] += u[2 * c + 1] * w;
-            }
-        }
-        double sn, cs;
-        sincos((double)alpha * phi, &sn, &cs);
-        const double fac = alpha == 0 ? 1.0 : 2.0;
-#pragma unroll
-        for (int c = 0; c < 3; c++) acc[c] += fac * (xr[c] * cs - xi[c] * sn);
-    }
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        double v = acc[c];
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-        acc[c] = v;
-    }
-    if (lane == 0) {
-        // Station::rotateField (Station.hpp:79-118) as Station::rotate
-        // (Station.cpp:41-55): about axis k, v_i' = v_i c + v_j s, v_j' =
-        // -v_i s + v_j c with i = k + 1, j = k + 2 (mod 3)
-        if (rec_rot != nullptr) {
-            for (int slot = 0; slot < 2; slot++) {
-                const double *q = rec_rot + (size_t)r * 6 + 3 * slot;
-                const int k = (int)q[0];
-                if (k < 0) continue;
-                const int i = (k + 1) % 3, j = (k + 2) % 3;
-                const double vi = acc[i], vj = acc[j];
-                acc[i] = vi * q[1] + vj * q[2];
-                acc[j] = -vi * q[2] + vj * q[1];
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < 3; c++) out[r * 3 + c] = acc[c];
-    }
+// Receivers by themselves, one block each (the stage form, and the
+// symplectic step, which records before it moves the displacement).
+__global__ __launch_bounds__(256) void k_record(RecordArgs a) {
+    __shared__ double red[4][3];
+    record_receiver(a, blockIdx.x, red);
 }
 
 // ------------------------------------------------------------ launchers
 template <typename Real>
-void launch_solid_stiff_fr(hipStream_t st, const StiffArgs<Real> &a) {
+void launch_solid_stiff_fr(hipStream_t st, const StiffArgs<Real> &a,
+                           StepArgs &h) {
     if (a.n_em <= 0) return;
     // one launch per material type present (em_list grouped by type)
     for (int mt = 0; mt < 3; mt++) {
         const int eb = a.em_type_begin[mt], ee = a.em_type_begin[mt + 1];
         const bool att = a.nsls > 0;
         if (ee <= eb) continue;
-        const int grid = (ee - eb + EMB - 1) / EMB;
+        const int grid = h.rec.nrec + (ee - eb + EMB - 1) / EMB;
 #define AXS3D_FR2(ATT_, MT_, PRT_)                                            \
     hipLaunchKernelGGL((k_solid_stiff_fr<Real, ATT_, MT_, PRT_>), dim3(grid), \
-                       dim3(STIFF_BLOCK), 0, st, a, eb, ee)
+                       dim3(STIFF_BLOCK), 0, st, a, eb, ee, h)
 #define AXS3D_FR(ATT_, MT_)                                                   \
     do {                                                                      \
         if (a.prt_idx != nullptr) AXS3D_FR2(ATT_, MT_, true);                 \
@@ -739,30 +668,27 @@ void launch_solid_stiff_fr(hipStream_t st, const StiffArgs<Real> &a) {
         }
 #undef AXS3D_FR
 #undef AXS3D_FR2
+        h = StepArgs();
     }
 }
 
 template <typename Real>
-void launch_moment_source(hipStream_t st, bool to_elem,
-                          const StiffArgs<Real> &a, int elem, int nu1c,
-                          const Real *pattern, const double *stf, int tstep,
-                          int nstf, const int *step_ctr, Real *stiff,
-                          const Real *prt_e) {
+void launch_source_forces(hipStream_t st, const StiffArgs<Real> &a, int elem,
+                          int nu1c, const Real *pattern, const Real *prt_e,
+                          cpx<Real> *force) {
     if (nu1c <= 0) return;
-    const int grid = (nu1c + EMB - 1) / EMB;
-    const Real *rot_e = a.rot ? a.rot + (size_t)elem * 4 * NPEM : nullptr;
-    if (to_elem)
-        hipLaunchKernelGGL((k_moment_source<Real, true>), dim3(grid),
-                           dim3(STIFF_BLOCK), 0, st, elem, nu1c, pattern, stf,
-                           tstep, nstf, step_ctr, a.elem_points, a.elem_axial, a.elem_ops,
-                           a.point_off, a.point_nu1, stiff, a.elem_eb_off,
-                           a.elem_nu1, a.eb, a.gtab, prt_e, rot_e);
-    else
-        hipLaunchKernelGGL((k_moment_source<Real, false>), dim3(grid),
-                           dim3(STIFF_BLOCK), 0, st, elem, nu1c, pattern, stf,
-                           tstep, nstf, step_ctr, a.elem_points, a.elem_axial, a.elem_ops,
-                           a.point_off, a.point_nu1, stiff, a.elem_eb_off,
-                           a.elem_nu1, a.eb, a.gtab, prt_e, rot_e);
+    hipLaunchKernelGGL(k_source_forces<Real>, dim3((nu1c + EMB - 1) / EMB),
+                       dim3(STIFF_BLOCK), 0, st, a, elem, nu1c, pattern,
+                       prt_e, force);
+}
+
+template <typename Real>
+void launch_apply_source(hipStream_t st, const StiffArgs<Real> &a, int elem,
+                         int i, int nu1c, Real *stiff) {
+    if (nu1c <= 0) return;
+    hipLaunchKernelGGL(k_apply_source<Real>,
+                       dim3((nu1c * NPEM + 255) / 256), dim3(256), 0, st, a,
+                       elem, i, nu1c, stiff);
 }
 
 template <typename Real>
@@ -808,6 +734,8 @@ void launch_point(hipStream_t st, int phases, const PointGeom &g,
     a.scheme = g.scheme;
     a.sym_pi = g.sym_pi;
     a.sym_kappa = g.sym_kappa;
+    a.note = g.note;
+    a.ctr = g.ctr;
     if (cpl.n_pairs <= 0 && g.abc.idx == nullptr) phases &= ~PHASE_COUPLE;
     if (g.abc.idx == nullptr) phases &= ~PHASE_SPONGE;
     if (phases == 0) return;
@@ -832,17 +760,9 @@ void launch_point(hipStream_t st, int phases, const PointGeom &g,
 #undef AXS3D_POINT_CASE
 }
 
-void launch_record(hipStream_t st, int nrec, const int32_t *rec_elem,
-                   const double *rec_w, const double *rec_phi,
-                   const int32_t *elem_points, const int32_t *elem_nu1,
-                   const uint32_t *point_off, const int32_t *point_nu1,
-                   const double *displ, double *out, const int *step_ctr,
-                   int max_samples, const double *rec_rot) {
-    if (nrec <= 0) return;
-    hipLaunchKernelGGL(k_record, dim3(nrec), dim3(64), 0, st, nrec, rec_elem,
-                       rec_w, rec_phi, elem_points, elem_nu1, point_off,
-                       point_nu1, displ, out, step_ctr, max_samples,
-                       rec_rot);
+void launch_record(hipStream_t st, const RecordArgs &a) {
+    if (a.nrec <= 0) return;
+    hipLaunchKernelGGL(k_record, dim3(a.nrec), dim3(256), 0, st, a);
 }
 
 // The step counter of replayed steps: [0] the step, [1] the first
@@ -854,41 +774,19 @@ __global__ void k_step_set(int *ctr, int tstep, int record_step0) {
     }
 }
 
-// flag[0]: raised by the point kernels, bit 0 when a step started from a
-// non-finite displacement (what Domain::checkStability tests at the start
-// of a step), bit 1 when a step left one; flag[1]: the first step (from
-// 0) that started from one (-1: none yet).
-__global__ void k_step_advance(int *ctr, int *flag) {
-    if (threadIdx.x == 0) {
-        if ((flag[0] & 1) != 0 && flag[1] < 0) flag[1] = ctr[0];
-        ctr[0] += 1;
-    }
-}
-
-__global__ void k_flag_note(int *flag, int tstep) {
-    if (threadIdx.x == 0 && (flag[0] & 1) != 0 && flag[1] < 0)
-        flag[1] = tstep;
-}
-
 void launch_step_set(hipStream_t st, int *ctr, int tstep, int record_step0) {
     hipLaunchKernelGGL(k_step_set, dim3(1), dim3(64), 0, st, ctr, tstep,
                        record_step0);
 }
 
-void launch_step_advance(hipStream_t st, int *ctr, int *flag) {
-    hipLaunchKernelGGL(k_step_advance, dim3(1), dim3(64), 0, st, ctr, flag);
-}
-
-void launch_flag_note(hipStream_t st, int *flag, int tstep) {
-    hipLaunchKernelGGL(k_flag_note, dim3(1), dim3(64), 0, st, flag, tstep);
-}
-
 #define AXS3D_INSTANTIATE(Real)                                               \
-    template void launch_solid_stiff_fr<Real>(hipStream_t,                   \
-                                              const StiffArgs<Real> &);      \
-    template void launch_moment_source<Real>(                                 \
-        hipStream_t, bool, const StiffArgs<Real> &, int, int, const Real *,   \
-        const double *, int, int, const int *, Real *, const Real *);         \
+    template void launch_solid_stiff_fr<Real>(                                \
+        hipStream_t, const StiffArgs<Real> &, StepArgs &);                    \
+    template void launch_source_forces<Real>(                                 \
+        hipStream_t, const StiffArgs<Real> &, int, int, const Real *,         \
+        const Real *, cpx<Real> *);                                           \
+    template void launch_apply_source<Real>(                                  \
+        hipStream_t, const StiffArgs<Real> &, int, int, int, Real *);         \
     template void launch_assemble<Real>(hipStream_t, const PointGeom &,       \
                                         const Real *, Real *);                \
     template void launch_point<Real>(hipStream_t, int, const PointGeom &,     \

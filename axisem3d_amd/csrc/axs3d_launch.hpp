@@ -6,6 +6,7 @@
 
 #include "axs3d_common.hpp"
 #include "axs3d_fft.hpp"
+#include "axs3d_step.hpp"
 
 namespace axs3d {
 
@@ -107,6 +108,7 @@ struct StiffArgs {
     const Real *att1d;             // [e][2][npa] dlambda, dmu
     double *mv_fr;                 // [em][nsls][6][npa] complex, FP64
     Real *ds_fr;                   // [em][6][npa] complex
+    SourceArgs<Real> src;          // the step's moment sources
 };
 
 // Largest element Nr of the cardinal kernels (one padded complex series
@@ -209,6 +211,10 @@ struct PointGeom {
     // += sym_kappa dt v (SymplecticTimeScheme::update)
     int scheme = 0;
     double sym_pi = 0., sym_kappa = 0.;
+    // a bulk step: note the first blown-up step; its last point kernel
+    // advances the step counter ctr (null: none)
+    bool note = false;
+    int *ctr = nullptr;
 };
 
 // Absorbing boundaries (AbsorbingBoundary, src/core/boundary/ABC) of the
@@ -278,6 +284,7 @@ struct Mass3DArgs {
     AbcGeom abc;                   // sponge terms of the march
     int scheme = 0;                // the march as PointGeom's
     double sym_pi = 0., sym_kappa = 0.;
+    bool note = false;
 };
 
 // Fluid points whose update needs transforms over the azimuth: a 3D mass
@@ -320,6 +327,7 @@ struct FluidDeferArgs {
     AbcGeom abc;                   // sponge terms of the march
     int scheme = 0;                // the march as PointGeom's
     double sym_pi = 0., sym_kappa = 0.;
+    bool note = false;
 };
 template <typename Real>
 void launch_fluid_defer(hipStream_t st, int phases,
@@ -332,8 +340,11 @@ template <typename Real>
 void launch_mass3d(hipStream_t st, bool march, const Mass3DArgs<Real> &a,
                    Real *stiff);
 
+// h: the step's receivers and number, if this is its first element kernel
+// (taken: cleared by the launch that carries them)
 template <typename Real>
-void launch_solid_stiff_fr(hipStream_t st, const StiffArgs<Real> &a);
+void launch_solid_stiff_fr(hipStream_t st, const StiffArgs<Real> &a,
+                           StepArgs &h);
 
 // A batch of the cardinal path: list3d positions [begin, end), all of
 // material type mtype, whose strain and stress fit the scratch together.
@@ -349,7 +360,7 @@ constexpr size_t CARD_SCRATCH_BYTES = (size_t)4 << 30;
 // order on one stream.
 template <typename Real>
 void launch_cd_grad(hipStream_t st, const CardArgs<Real> &a,
-                    const CardBatch &bt);
+                    const CardBatch &bt, StepArgs &h);
 template <typename Real>
 void launch_cd_stress(hipStream_t st, const CardArgs<Real> &a,
                       const CardBatch &bt);
@@ -368,12 +379,18 @@ void launch_cdf_batch(hipStream_t st, const FluidCardArgs<Real> &a,
 template <typename Real>
 int card_blocks_per_cu(bool att, int nr_max);
 
+// The forces of moment source (elem, nu1c orders, pattern) for a unit
+// source time function, [alpha][25][3] complex; prt_e, the element's PRT
+// operands or null.
 template <typename Real>
-void launch_moment_source(hipStream_t st, bool to_elem,
-                          const StiffArgs<Real> &a, int elem, int nu1c,
-                          const Real *pattern, const double *stf, int tstep,
-                          int nstf, const int *step_ctr, Real *stiff,
-                          const Real *prt_e = nullptr);
+void launch_source_forces(hipStream_t st, const StiffArgs<Real> &a, int elem,
+                          int nu1c, const Real *pattern, const Real *prt_e,
+                          cpx<Real> *force);
+// The stage form of the sources (Domain::applySources): source i of a.src,
+// in element elem, subtracted from the point stiffness.
+template <typename Real>
+void launch_apply_source(hipStream_t st, const StiffArgs<Real> &a, int elem,
+                         int i, int nu1c, Real *stiff);
 
 template <typename Real>
 void launch_assemble(hipStream_t st, const PointGeom &g, const Real *eb,
@@ -403,12 +420,7 @@ void launch_fluid_point(hipStream_t st, int phases, const PointGeom &g,
 void launch_sym_launch(hipStream_t st, double *u, const double *v, int64_t n,
                        double kdt);
 
-void launch_record(hipStream_t st, int nrec, const int32_t *rec_elem,
-                   const double *rec_w, const double *rec_phi,
-                   const int32_t *elem_points, const int32_t *elem_nu1,
-                   const uint32_t *point_off, const int32_t *point_nu1,
-                   const double *displ, double *out, const int *step_ctr,
-                   int max_samples, const double *rec_rot = nullptr);
+void launch_record(hipStream_t st, const RecordArgs &a);
 
 // adjoint: sensitivity densities of one step, kern[e][k][3] += scale *
 // (lambda, mu, rho) densities of (psi, u, a); FP64 throughout
@@ -461,8 +473,4 @@ void launch_adjoint_source(hipStream_t st, int nrec, const int32_t *rec_elem,
 
 // step counter of a replayed (graph) step; see k_step_set
 void launch_step_set(hipStream_t st, int *ctr, int tstep, int record_step0);
-void launch_step_advance(hipStream_t st, int *ctr, int *flag);
-// eager steps: note tstep as the first blown-up step once flag[0] is up
-void launch_flag_note(hipStream_t st, int *flag, int tstep);
-
 }  // namespace axs3d
