@@ -874,17 +874,25 @@ __global__ __launch_bounds__(128) void k_mass3d(Mass3DArgs<Real> a,
             for (int ri = 0; ri < 2; ri++) {
                 const double u0 = a.displ[m6 + ri];
                 double vv, uu;
+                bool va = true;
                 if (a.scheme == 1) {
                     // SymplecticTimeScheme::update
                     vv = a.veloc[m6 + ri] + a.sym_pi * a.dt * an[ri];
                     uu = u0 + a.sym_kappa * a.dt * vv;
                 } else {
-                    vv = a.veloc[m6 + ri] +
-                         hdt * (a.accel[m6 + ri] + an[ri]);
-                    uu = u0 + (a.dt * vv + hdt2 * an[ri]);
-                    a.accel[m6 + ri] = an[ri];
+                    const bool fh = march_reads_half(a.march);
+                    vv = fh ? a.half[m6 + ri] : a.veloc[m6 + ri];
+                    uu = u0;
+                    newmark_march(a.march, a.dt, hdt, hdt2,
+                                  fh ? 0. : a.accel[m6 + ri], an[ri], uu, vv);
+                    if (a.march != MARCH_FULL) {
+                        a.half[m6 + ri] = vv;
+                        vv -= hdt * an[ri];
+                    }
+                    va = march_writes_va(a.march);
+                    if (va) a.accel[m6 + ri] = an[ri];
                 }
-                a.veloc[m6 + ri] = vv;
+                if (va) a.veloc[m6 + ri] = vv;
                 a.displ[m6 + ri] = uu;
                 bad |= !isfinite(uu);
                 bad0 |= !isfinite(u0);
@@ -1279,16 +1287,25 @@ __global__ __launch_bounds__(128) void k_fluid_defer(FluidDeferArgs<Real> a) {
         for (int ri = 0; ri < 2; ri++) {
             const double u0 = a.chi[m2 + ri];
             double vv, uu;
+            bool va = true;
             if (a.scheme == 1) {
                 // SymplecticTimeScheme::update
                 vv = a.chi_v[m2 + ri] + a.sym_pi * a.dt * an[ri];
                 uu = u0 + a.sym_kappa * a.dt * vv;
             } else {
-                vv = a.chi_v[m2 + ri] + hdt * (a.chi_a[m2 + ri] + an[ri]);
-                uu = u0 + (a.dt * vv + hdt2 * an[ri]);
-                a.chi_a[m2 + ri] = an[ri];
+                const bool fh = march_reads_half(a.march);
+                vv = fh ? a.half[m2 + ri] : a.chi_v[m2 + ri];
+                uu = u0;
+                newmark_march(a.march, a.dt, hdt, hdt2,
+                              fh ? 0. : a.chi_a[m2 + ri], an[ri], uu, vv);
+                if (a.march != MARCH_FULL) {
+                    a.half[m2 + ri] = vv;
+                    vv -= hdt * an[ri];
+                }
+                va = march_writes_va(a.march);
+                if (va) a.chi_a[m2 + ri] = an[ri];
             }
-            a.chi_v[m2 + ri] = vv;
+            if (va) a.chi_v[m2 + ri] = vv;
             a.chi[m2 + ri] = uu;
             bad |= !isfinite(uu);
             bad0 |= !isfinite(u0);

@@ -1285,6 +1285,11 @@ void DomainBase::finalize() {
     };
     abcUp(mAbcS, mAbcSD, mNumPoints, hPointNr);
     if (mNumFElems > 0) abcUp(mAbcF, mAbcFD, mNumFPoints, hFPointNr);
+    if (marchesHalf()) {
+        dHalf.alloc(fbytes);
+        if (mNumFElems > 0)
+            dFHalf.alloc((size_t)mNumFModes * 2 * sizeof(double));
+    }
     if (mNumRec > 0) {
         up(dRecElem, hRecElem.data(), hRecElem.size() * 4);
         up(dRecW, hRecW.data(), hRecW.size() * 8);
@@ -1437,43 +1442,71 @@ void DomainBase::checkStability(int tstep) {
 
 // NewmarkTimeScheme::solve (NewmarkTimeScheme.cpp:41-108).  Stability is
 // checked from the device flag at the end of the batch (the point kernel
-// raises it on any non-finite displacement).  By default the steps are
-// replays of one captured step graph, whose source and receiver kernels
-// read the step from the device counter set here; with profiling on, or
+// raises it on any non-finite displacement).  By default the steps that
+// march alike are replays of a captured graph, whose element kernels read
+// the step from the device counter set here; with profiling on, or
 // useGraph(false), every step is launched kernel by kernel.
 void DomainBase::solve(int step_begin, int nsteps) {
     requireFinalized("NewmarkTimeScheme::solve");
     if (nsteps > 0 && hSrcElem >= 0 &&
         (step_begin < 0 || step_begin + nsteps > mStfSteps))
         throw Error("Domain::applySources || Step outside the STF.");
+    struct Full {
+        int &march;
+        ~Full() { march = MARCH_FULL; }
+    } full{mMarch};
+    // the march of step i of the run (see MarchForm)
+    const bool half = marchesHalf();
+    const bool from = half && !mHalfValid;
+    auto form = [&](int i) {
+        if (!half) return (int)MARCH_FULL;
+        return MARCH_HALF | (i == 0 && from ? MARCH_FROM : 0) |
+               (i == nsteps - 1 ? MARCH_TO : 0);
+    };
+    mHalfValid = mHalfValid && nsteps <= 0;
     if (nsteps > 0 && mUseGraph && !mProfile) {
-        if (!mGraphExec) captureStep();
         launch_step_set(mStream, dStepCtr.as<int>(), step_begin,
                         mRecordStep0);
-        for (int i = 0; i < nsteps; i++)
-            hip_check(hipGraphLaunch(mGraphExec, mStream),
-                      "NewmarkTimeScheme::solve");
+        // the steps that march alike, in graphs of kGraphSteps; the others,
+        // and what is left, kernel by kernel
+        const int lo = from ? 1 : 0, hi = half ? nsteps - 1 : nsteps;
+        for (int i = 0; i < nsteps;) {
+            mMarch = form(i);
+            if (i >= lo && i + kGraphSteps <= hi) {
+                if (!mGraphExec) captureSteps(kGraphSteps);
+                hip_check(hipGraphLaunch(mGraphExec, mStream),
+                          "NewmarkTimeScheme::solve");
+                i += kGraphSteps;
+            } else {
+                step(step_begin + i, -1, true);
+                i++;
+            }
+        }
     } else {
-        for (int tstep = step_begin; tstep < step_begin + nsteps; tstep++) {
+        for (int i = 0; i < nsteps; i++) {
+            const int tstep = step_begin + i;
             int isample = -1;
             if (mNumRec > 0) {
                 isample = tstep - mRecordStep0;
                 if (isample < 0 || isample >= hMaxSamples) isample = -1;
             }
+            mMarch = form(i);
             step(tstep, isample, false);
         }
     }
+    if (nsteps > 0) mHalfValid = half;
     checkStability(step_begin + nsteps + 1);
 }
 
-// Captures one step in its device-counter form.  The captured kernels take
-// only device pointers fixed at finalize, the time step and the launch
-// shapes, so the graph stays valid until dt changes (setDt drops it).
-void DomainBase::captureStep() {
+// Captures n steps, of the march mMarch, in their device-counter form.  The
+// captured kernels take only device pointers fixed at finalize, the time
+// step and the launch shapes, so the graph stays valid until dt changes
+// (setDt drops it).
+void DomainBase::captureSteps(int n) {
     hip_check(hipStreamBeginCapture(mStream, hipStreamCaptureModeThreadLocal),
               "NewmarkTimeScheme::solve");
     try {
-        step(0, -1, true);
+        for (int i = 0; i < n; i++) step(0, -1, true);
     } catch (...) {
         hipGraph_t g = nullptr;
         (void)hipStreamEndCapture(mStream, &g);
@@ -1769,6 +1802,8 @@ public:
         g.scheme = mScheme;
         g.sym_pi = mSymPi;
         g.sym_kappa = mSymKappa;
+        g.half = dHalf.as<double>();
+        g.march = mMarch;
         g.note = mNote;
         g.ctr = mAdvance ? dStepCtr.as<int>() : nullptr;
         return g;
@@ -1859,6 +1894,8 @@ public:
         m.scheme = mScheme;
         m.sym_pi = mSymPi;
         m.sym_kappa = mSymKappa;
+        m.half = dHalf.as<double>();
+        m.march = mMarch;
         m.note = mNote;
         return m;
     }
@@ -1876,6 +1913,8 @@ public:
         g.scheme = mScheme;
         g.sym_pi = mSymPi;
         g.sym_kappa = mSymKappa;
+        g.half = dFHalf.as<double>();
+        g.march = mMarch;
         g.note = mNote;
         return g;
     }
@@ -1914,6 +1953,8 @@ public:
         f.scheme = mScheme;
         f.sym_pi = mSymPi;
         f.sym_kappa = mSymKappa;
+        f.half = dFHalf.as<double>();
+        f.march = mMarch;
         f.note = mNote;
         return f;
     }
@@ -2200,6 +2241,7 @@ public:
         if (mScheme != 0)
             throw Error("NewmarkTimeScheme::update || The domain marches "
                         "with the symplectic scheme.");
+        mHalfValid = false;
         point(PHASE_MARCH);
         fluidPoint(PHASE_MARCH);
     }
@@ -2331,6 +2373,7 @@ public:
                         "checkpoint interval must be positive.");
         if (hSrcElem >= 0 && nsteps > mStfSteps)
             throw Error("Domain::adjoint || Step outside the STF.");
+        mHalfValid = false;
         adjointOperands();
         const size_t nd = (size_t)mNumModes * 6;
         const size_t nf = nd * sizeof(double);
@@ -2542,6 +2585,8 @@ public:
         const int base = fl ? which - AXS3D_FIELD_FLUID_DISPL : which;
         const size_t n = fl ? (size_t)mNumFModes * 2 : (size_t)mNumModes * 6;
         if (n == 0) return;
+        if (base == AXS3D_FIELD_VELOC || base == AXS3D_FIELD_ACCEL)
+            mHalfValid = false;
         if (base == AXS3D_FIELD_STIFF) {
             std::vector<Real> tmp(in, in + n);
             hip_check(hipMemcpyAsync((fl ? dFStiff : dStiff).template as<Real>(),

@@ -231,11 +231,12 @@ protected:
     int mDevice = 0;
     int mPrecision = 0;
     hipStream_t mStream = nullptr;
-    // one step captured as a HIP graph (solve replays it)
+    // kGraphSteps steps captured as a HIP graph (solve replays it)
     bool mUseGraph = true;
     hipGraph_t mGraph = nullptr;
     hipGraphExec_t mGraphExec = nullptr;
-    void captureStep();
+    void captureSteps(int n);
+    static constexpr int kGraphSteps = 1;
     void dropGraph();
     bool mFinalized = false;
     double mDt = 0.;
@@ -405,6 +406,16 @@ protected:
     // step bookkeeping of the bulk kernels: whether blown-up steps are
     // noted, and whether the next solid point kernel advances the counter
     bool mNote = false, mAdvance = false;
+    // how the next Newmark step marches (MarchForm)
+    int mMarch = MARCH_FULL;
+    // w = v + dt/2 a of the last run (MarchForm); valid until something else
+    // changes the velocity or the acceleration
+    DeviceBuffer dHalf, dFHalf;
+    bool mHalfValid = false;
+    bool marchesHalf() const {
+        // absorbing boundaries need the velocity of every step
+        return mScheme == 0 && mAbcSD.n == 0 && mAbcFD.n == 0;
+    }
     // station frames: [receiver][6] two rotations (axis, cos, sin)
     std::vector<double> hRecRot;
     DeviceBuffer dRecRot;

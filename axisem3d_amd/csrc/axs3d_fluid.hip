@@ -174,6 +174,8 @@ struct FluidPointArgs {
     AbcGeom abc;                   // Clayton and sponge terms (k_abc)
     int scheme;                    // 0 Newmark, 1 symplectic sub-step
     double sym_pi, sym_kappa;
+    int march;                     // MarchForm
+    double *half;
     bool note;                     // bulk step: see PointGeom
 };
 
@@ -275,15 +277,25 @@ __global__ __launch_bounds__(256) void k_fluid_point(
         raise_flag(a.flag, a.note, bad0, bad);
         return;
     }
-    // all three loaded (16-byte vectors) before anything is stored
-    const double2 u0 = *up, v0 = *vp, a0 = *ap;
-    const double vr = v0.x + a.half_dt * (a0.x + s[0]);
-    const double vi = v0.y + a.half_dt * (a0.y + s[1]);
-    const double ur = u0.x + (a.dt * vr + a.half_dt_dt * s[0]);
-    const double ui = u0.y + (a.dt * vi + a.half_dt_dt * s[1]);
-    *vp = make_double2(vr, vi);
-    *ap = make_double2(s[0], s[1]);
+    // all of the state is loaded (16-byte vectors) before anything is stored
+    double2 *hp = reinterpret_cast<double2 *>(a.half + (size_t)k * 2);
+    const bool from_half = march_reads_half(a.march);
+    const double2 u0 = *up, v0 = from_half ? *hp : *vp;
+    double2 a0 = make_double2(0., 0.);
+    if (!from_half) a0 = *ap;
+    double vr = v0.x, vi = v0.y, ur = u0.x, ui = u0.y;
+    newmark_march(a.march, a.dt, a.half_dt, a.half_dt_dt, a0.x, s[0], ur, vr);
+    newmark_march(a.march, a.dt, a.half_dt, a.half_dt_dt, a0.y, s[1], ui, vi);
     *up = make_double2(ur, ui);
+    if (a.march != MARCH_FULL) {
+        *hp = make_double2(vr, vi);
+        vr -= a.half_dt * s[0];
+        vi -= a.half_dt * s[1];
+    }
+    if (march_writes_va(a.march)) {
+        *vp = make_double2(vr, vi);
+        *ap = make_double2(s[0], s[1]);
+    }
     const bool bad = !isfinite(ur) || !isfinite(ui);
     const bool bad0 = !isfinite(u0.x) || !isfinite(u0.y);
     if (!GATHER) stiff[(size_t)k * 2] = stiff[(size_t)k * 2 + 1] = 0;
@@ -337,6 +349,8 @@ void launch_fluid_point(hipStream_t st, int phases, const PointGeom &g,
     a.scheme = g.scheme;
     a.sym_pi = g.sym_pi;
     a.sym_kappa = g.sym_kappa;
+    a.march = g.march;
+    a.half = g.half;
     a.note = g.note;
     if (cpl.n_pairs <= 0 && g.abc.idx == nullptr) phases &= ~PHASE_COUPLE;
     if (g.abc.idx == nullptr) phases &= ~PHASE_SPONGE;

@@ -409,6 +409,8 @@ struct PointArgs {
     AbcGeom abc;
     int scheme;                   // 0 Newmark, 1 symplectic sub-step
     double sym_pi, sym_kappa;
+    int march;                    // MarchForm
+    double *half;
     bool note;                    // bulk step: see PointGeom
     int *ctr;
 };
@@ -544,8 +546,8 @@ __global__ __launch_bounds__(256) void k_point(PointArgs a,
 #pragma unroll
         for (int q = 0; q < 6; q++) a_new[q] = (double)s[q];
     }
-    // all of u, v, a are loaded (16-byte vectors) before anything is
-    // stored, so the nine loads are in flight together
+    // all of the state is loaded (16-byte vectors) before anything is
+    // stored, so the loads are in flight together
     double2 *up = reinterpret_cast<double2 *>(a.displ + (size_t)k * 6);
     double2 *vp = reinterpret_cast<double2 *>(a.veloc + (size_t)k * 6);
     double2 *ap = reinterpret_cast<double2 *>(a.accel + (size_t)k * 6);
@@ -584,30 +586,42 @@ __global__ __launch_bounds__(256) void k_point(PointArgs a,
         raise_flag(a.flag, a.note, bad0, bad);
         return;
     }
+    double2 *hp = reinterpret_cast<double2 *>(a.half + (size_t)k * 6);
+    const bool from_half = march_reads_half(a.march);
 #pragma unroll
     for (int c = 0; c < 3; c++) {
         u2[c] = up[c];
-        v2[c] = vp[c];
-        a2[c] = ap[c];
+        v2[c] = from_half ? hp[c] : vp[c];
+        a2[c] = make_double2(0., 0.);
     }
+    if (!from_half)
+#pragma unroll
+        for (int c = 0; c < 3; c++) a2[c] = ap[c];
 #pragma unroll
     for (int c = 0; c < 3; c++) {
         bad0 |= !isfinite(u2[c].x) || !isfinite(u2[c].y);
-        const double vr = v2[c].x + half_dt * (a2[c].x + a_new[2 * c]);
-        const double vi = v2[c].y + half_dt * (a2[c].y + a_new[2 * c + 1]);
-        const double ur = u2[c].x + (dt * vr + half_dt_dt * a_new[2 * c]);
-        const double ui =
-            u2[c].y + (dt * vi + half_dt_dt * a_new[2 * c + 1]);
-        v2[c] = make_double2(vr, vi);
-        a2[c] = make_double2(a_new[2 * c], a_new[2 * c + 1]);
-        u2[c] = make_double2(ur, ui);
-        bad |= !isfinite(ur) || !isfinite(ui);
+        newmark_march(a.march, dt, half_dt, half_dt_dt, a2[c].x,
+                      a_new[2 * c], u2[c].x, v2[c].x);
+        newmark_march(a.march, dt, half_dt, half_dt_dt, a2[c].y,
+                      a_new[2 * c + 1], u2[c].y, v2[c].y);
+        bad |= !isfinite(u2[c].x) || !isfinite(u2[c].y);
     }
 #pragma unroll
-    for (int c = 0; c < 3; c++) {
-        vp[c] = v2[c];
-        ap[c] = a2[c];
-        up[c] = u2[c];
+    for (int c = 0; c < 3; c++) up[c] = u2[c];
+    if (a.march != MARCH_FULL) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            hp[c] = v2[c];
+            v2[c].x -= half_dt * a_new[2 * c];
+            v2[c].y -= half_dt * a_new[2 * c + 1];
+        }
+    }
+    if (march_writes_va(a.march)) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            vp[c] = v2[c];
+            ap[c] = make_double2(a_new[2 * c], a_new[2 * c + 1]);
+        }
     }
     if (!GATHER) {
 #pragma unroll
@@ -734,6 +748,8 @@ void launch_point(hipStream_t st, int phases, const PointGeom &g,
     a.scheme = g.scheme;
     a.sym_pi = g.sym_pi;
     a.sym_kappa = g.sym_kappa;
+    a.march = g.march;
+    a.half = g.half;
     a.note = g.note;
     a.ctr = g.ctr;
     if (cpl.n_pairs <= 0 && g.abc.idx == nullptr) phases &= ~PHASE_COUPLE;

@@ -211,6 +211,8 @@ struct PointGeom {
     // += sym_kappa dt v (SymplecticTimeScheme::update)
     int scheme = 0;
     double sym_pi = 0., sym_kappa = 0.;
+    int march = MARCH_FULL;        // MarchForm, Newmark
+    double *half = nullptr;        // its w field
     // a bulk step: note the first blown-up step; its last point kernel
     // advances the step counter ctr (null: none)
     bool note = false;
@@ -284,6 +286,8 @@ struct Mass3DArgs {
     AbcGeom abc;                   // sponge terms of the march
     int scheme = 0;                // the march as PointGeom's
     double sym_pi = 0., sym_kappa = 0.;
+    int march = MARCH_FULL;
+    double *half = nullptr;
     bool note = false;
 };
 
@@ -327,6 +331,8 @@ struct FluidDeferArgs {
     AbcGeom abc;                   // sponge terms of the march
     int scheme = 0;                // the march as PointGeom's
     double sym_pi = 0., sym_kappa = 0.;
+    int march = MARCH_FULL;
+    double *half = nullptr;
     bool note = false;
 };
 template <typename Real>
