@@ -21,7 +21,8 @@ KERNEL_STIFFNESS, KERNEL_POINT, KERNEL_SOURCE, KERNEL_RECORD = 0, 1, 2, 3
 KERNEL_STIFFNESS_3D = 4
 KERNEL_FLUID_STIFFNESS, KERNEL_FLUID_POINT = 5, 6
 KERNEL_CD_GRAD, KERNEL_CD_STRESS, KERNEL_CD_QUAD = 7, 8, 9
-NUM_KERNELS = 10
+KERNEL_CD_FUSED = 10
+NUM_KERNELS = 11
 
 # every symbol declared in include/axs3d.h, with (restype, argtypes)
 _p = C.c_void_p

@@ -2080,8 +2080,8 @@ public:
         hip_check(hipStreamSynchronize(mStream), "Domain::finalize");
     }
 
-    // The cardinal path, batch by batch; with timing, each of the three
-    // kernels is timed under its own id.
+    // The cardinal path, batch by batch, then the elements of the
+    // one-kernel form; with timing, each kernel is timed under its own id.
     void cardinalPath(bool timed) {
         StepArgs h;
         cardinalPathOn(cardArgs(), mCardBatches, timed, h);
@@ -2103,6 +2103,11 @@ public:
             }
             launch_cd_quad<Real>(mStream, c, bt);
             if (timed) tock(AXS3D_KERNEL_CD_QUAD);
+        }
+        for (const FusedGroup &g : mFusedGroups) {
+            if (timed) tick(AXS3D_KERNEL_CD_FUSED);
+            launch_cd_fused<Real>(mStream, c, g, h);
+            if (timed) tock(AXS3D_KERNEL_CD_FUSED);
         }
     }
 
@@ -2375,6 +2380,9 @@ public:
             throw Error("Domain::adjoint || Step outside the STF.");
         mHalfValid = false;
         adjointOperands();
+        planAdjointBatches();
+        const bool own = !mAdjBatches.empty();
+        const size_t adjScr = own ? mAdjScrMax : mCardScrMax;
         const size_t nd = (size_t)mNumModes * 6;
         const size_t nf = nd * sizeof(double);
         const int nck = (nsteps + seg - 1) / seg;
@@ -2388,7 +2396,8 @@ public:
         const size_t ckBytes = 3 * nf + attBytes;
         const double need =
             (double)ckBytes * nck + (double)nf * (2.0 * seglen + 3.0) +
-            (double)attBytes + (double)mCardScrMax * sizeof(cpx<Real>) +
+            (double)attBytes +
+            (double)adjScr * (own ? 2 : 1) * sizeof(cpx<Real>) +
             (double)mPropTotal * sizeof(double);
         if (need > 0.9 * (double)freeb) {
             std::ostringstream ss;
@@ -2421,7 +2430,8 @@ public:
         if (mNum3D > 0) {
             dAdjKern3D.alloc(nk3 * sizeof(double));
             dAdjKern3D.zero(mStream);
-            dAdjScrB.alloc(mCardScrMax * sizeof(cpx<Real>));
+            if (own) dAdjScrA.alloc(adjScr * sizeof(cpx<Real>));
+            dAdjScrB.alloc(adjScr * sizeof(cpx<Real>));
         }
         const int all = PHASE_GATHER | PHASE_AXIAL | PHASE_MASS | PHASE_MARCH;
         char *ck = dAdjCkpt.as<char>();
@@ -2508,11 +2518,17 @@ public:
                 if (mNum3D > 0) {
                     // per-slice densities: strain rows of psi and u_n,
                     // batch by batch
-                    const CardArgs<Real> ca = cardArgs();
+                    CardArgs<Real> ca = cardArgs();
+                    if (own) {
+                        ca.s.em_list = dAdjEM3D.as<EMItem>();
+                        ca.scr_off = dAdjScrOff.as<uint32_t>();
+                        ca.scratch = dAdjScrA.as<Real>();
+                    }
                     CardArgs<Real> cb = ca;
                     cb.s.displ = su + (size_t)(n - n0) * nd;
                     cb.scratch = dAdjScrB.as<Real>();
-                    for (const CardBatch &bt : mCardBatches) {
+                    for (const CardBatch &bt : own ? mAdjBatches
+                                                   : mCardBatches) {
                         StepArgs none;
                         launch_cd_grad<Real>(mStream, ca, bt, none);
                         launch_cd_grad<Real>(mStream, cb, bt, none);
@@ -2553,6 +2569,7 @@ public:
         dAdjCkpt.reset();
         dAdjSegU.reset();
         dAdjSegA.reset();
+        dAdjScrA.reset();
         dAdjScrB.reset();
         for (int i = 0; i < 4; i++) dAdjAtt[i].reset();
     }
@@ -2633,10 +2650,12 @@ private:
     // Batches of the 3D solid elements for a scratch of `bytes`, their
     // elements' scratch offsets (complex values) and the largest batch
     // (complex values); the element-mode lists do not depend on the
-    // budget.
+    // budget.  Elements of the one-kernel form have no part in them, unless
+    // all is set (the adjoint's strain rows).
     void planCardBatches(size_t bytes, std::vector<CardBatch> &batches,
                          std::vector<uint32_t> &scrOff,
-                         std::vector<EMItem> &em3d, size_t &scrMax) const {
+                         std::vector<EMItem> &em3d, size_t &scrMax,
+                         bool all = false) const {
         const size_t budget =
             std::min(bytes / sizeof(cpx<Real>), (size_t)UINT32_MAX);
         scrOff.assign(mNumElems, 0u);
@@ -2645,7 +2664,8 @@ private:
         scrMax = 0;
         for (int mt = 0; mt < 3; mt++) {
             size_t used = 0;
-            for (int w = mTypeBegin3D[mt]; w < mTypeBegin3D[mt + 1]; w++) {
+            const int end = all ? mTypeBegin3D[mt + 1] : mFusedBegin[mt];
+            for (int w = mTypeBegin3D[mt]; w < end; w++) {
                 const int e = hList3D[w];
                 const int nu1 = hElemNr[e] / 2 + 1;
                 const size_t need = (size_t)6 * NPEM * scr_row(nu1);
@@ -2730,6 +2750,59 @@ private:
         }
     }
 
+    // The elements of the one-kernel form, and their launch groups: an
+    // element's LDS is sized by its group's largest, so a new group begins
+    // where twice as many would fit a CU, if both parts fill the chip.
+    void planFused() {
+        mFusedNrMax = 0;
+        if (hPrtElems.empty())
+            while (mFusedNrMax < FUSED_NR_CAP &&
+                   fused_lds_bytes<Real>(mFusedNrMax + 1) <= FUSED_LDS_MAX)
+                mFusedNrMax++;
+        mFusedGroups.clear();
+        mNumFused = 0;
+        // a launch of few blocks takes as long as one of them (about 25 us),
+        // where the same elements add 0.15 us each to launches that run
+        // anyway: next to larger elements it takes a chip of them
+        bool larger = false;
+        for (int w = 0; w < mNum3D; w++)
+            larger = larger || hElemNr[hList3D[w]] > mFusedNrMax;
+        for (int mt = 0; mt < 3; mt++) {
+            int w = mTypeBegin3D[mt];
+            const int end = mTypeBegin3D[mt + 1];
+            while (w < end && hElemNr[hList3D[w]] > mFusedNrMax) w++;
+            if (larger && end - w < FUSED_WITH_LARGER_MIN) w = end;
+            mFusedBegin[mt] = w;
+            mNumFused += end - w;
+            while (w < end) {
+                FusedGroup g{mt, w, w, hElemNr[hList3D[w]]};
+                const size_t lds = fused_lds_bytes<Real>(g.nr_max);
+                while (g.end < end &&
+                       (g.end - g.begin < FUSED_GROUP_MIN ||
+                        end - g.end < FUSED_GROUP_MIN ||
+                        2 * fused_lds_bytes<Real>(
+                                hElemNr[hList3D[g.end]]) > lds))
+                    g.end++;
+                mFusedGroups.push_back(g);
+                w = g.end;
+            }
+        }
+    }
+
+    // The adjoint's batches of all 3D elements.
+    void planAdjointBatches() {
+        if (mFusedGroups.empty() || !mAdjBatches.empty()) return;
+        std::vector<uint32_t> off;
+        std::vector<EMItem> em;
+        planCardBatches((size_t)(mScratchMiB * (1 << 20)), mAdjBatches, off,
+                        em, mAdjScrMax, true);
+        dAdjScrOff.alloc(off.size() * 4);
+        dAdjScrOff.upload(off.data(), off.size() * 4, mStream);
+        dAdjEM3D.alloc(em.size() * sizeof(EMItem));
+        dAdjEM3D.upload(em.data(), em.size() * sizeof(EMItem), mStream);
+        hip_check(hipStreamSynchronize(mStream), "Domain::adjoint");
+    }
+
     void buildCardBatches(size_t bytes) {
         std::vector<uint32_t> scrOff;
         std::vector<EMItem> em3d;
@@ -2738,7 +2811,8 @@ private:
         dScrOff.alloc(scrOff.size() * 4);
         dScrOff.upload(scrOff.data(), scrOff.size() * 4, mStream);
         dEM3D.alloc(em3d.size() * sizeof(EMItem));
-        dEM3D.upload(em3d.data(), em3d.size() * sizeof(EMItem), mStream);
+        if (!em3d.empty())
+            dEM3D.upload(em3d.data(), em3d.size() * sizeof(EMItem), mStream);
         scrMax = std::max(scrMax, mFCardScrMax);
         if (scrMax != mCardScrMax || dCardScratch.bytes() == 0) {
             mCardScrMax = scrMax;
@@ -2776,7 +2850,7 @@ private:
         if (env && env[0] == '0') return;
         mCardTuneMs = timeCardinalPass();
         mTuneTrials = 1;
-        if (!mScratchFixed) {
+        if (!mScratchFixed && !mCardBatches.empty()) {
             double best_mib = mScratchMiB;
             float best = (float)mCardTuneMs;
             for (const size_t mib : {(size_t)1024, (size_t)256}) {
@@ -3075,6 +3149,7 @@ private:
                     1.0, std::atof(env) * (double)((size_t)1 << 20));
                 mScratchFixed = true;
             }
+            planFused();
             buildCardBatches(budget);
             if (mNsls > 0) {
                 const int npa = mAttCG4 ? 4 : NPEM;

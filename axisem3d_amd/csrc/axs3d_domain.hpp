@@ -210,12 +210,15 @@ public:
     int precision() const { return mPrecision; }
     // every autotuner choice and timing: [0] cardinal pass ms, [1] scratch
     // MiB, [2] scratch sizes timed, [3] FFT largest radix, [4] radices
-    // timed, then (radix, ms) per radix timed; returns the count written
+    // timed, then (radix, ms) per radix timed, then the elements of the
+    // one-kernel form and its largest Nr; returns the count written
     int autotuneReport(double *out, int n) const {
         std::vector<double> v = {mCardTuneMs, mScratchMiB,
                                  (double)mTuneTrials, (double)mFftMaxRadix,
                                  (double)(mRadixMs.size() / 2)};
         v.insert(v.end(), mRadixMs.begin(), mRadixMs.end());
+        v.push_back(mNumFused);
+        v.push_back(mFusedNrMax);
         const int k = std::min(n, (int)v.size());
         for (int i = 0; i < k; i++) out[i] = v[i];
         return k;
@@ -344,6 +347,17 @@ protected:
     std::vector<double> hCpl3DNu, hCpl3DNa, hCpl3DNam;
     int mNumFDefer = 0, mNumCpl3D = 0;
     std::vector<CardBatch> mCardBatches;
+    // 3D elements that take the one-kernel form: the last ones of each
+    // type's part of list3d, from mFusedBegin[type], in launch groups
+    std::vector<FusedGroup> mFusedGroups;
+    int mFusedBegin[3] = {0, 0, 0};
+    int mFusedNrMax = 0;                // largest Nr that may take it
+    int mNumFused = 0;                  // how many take it
+    // batches of all 3D elements for the adjoint's strain rows, where some
+    // elements have none in mCardBatches
+    std::vector<CardBatch> mAdjBatches;
+    size_t mAdjScrMax = 0;
+    DeviceBuffer dAdjScrOff, dAdjEM3D, dAdjScrA;
     int mCardOcc = CARD_OCC;            // stress kernel waves per SIMD
     double mCardTuneMs = 0.;            // one cardinal pass at finalize
     double mScratchMiB = 0.;            // cardinal scratch budget in use

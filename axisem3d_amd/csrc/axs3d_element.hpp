@@ -61,17 +61,16 @@ __device__ __forceinline__ void load_point_g(const Real (*sG)[NPEM],
     }
 }
 
-// computeGrad6 at point (i, j) of one element-mode whose displacement
-// tile sU[3][25] is in LDS; u = this point's own displacement.  Voigt
-// strain [ss, pp, zz, pz, sz, sp] with engineering shears.
-template <typename Real>
-__device__ __forceinline__ void grad6_point(const cpx<Real> (*sU)[NPEM],
-                                            const cpx<Real> (&u)[3],
-                                            Real ralpha, bool axial_row0,
-                                            int i, int j,
-                                            const PointG<Real> &G,
-                                            const PointOps<Real> &g,
-                                            cpx<Real> (&eps)[6]) {
+// computeGrad6 at point (i, j) of one element-mode; U(c, p) the element's
+// displacement, u = this point's own; gx[k] = G_xi(k, i), gz[k] = G(k, j).
+// Voigt strain [ss, pp, zz, pz, sz, sp] with engineering shears.
+template <typename Real, typename Get>
+__device__ __forceinline__ void grad6_at(Get U, const cpx<Real> (&u)[3],
+                                         Real ralpha, bool axial_row0, int i,
+                                         int j, const Real (&gx)[NPED],
+                                         const Real (&gz)[NPED],
+                                         const PointOps<Real> &g,
+                                         cpx<Real> (&eps)[6]) {
     // higher-order terms (computeGrad_dSdZ, GradientQuadrature.hpp:405-418)
     cpx<Real> dS[3], dZ[3];
 #pragma unroll
@@ -79,8 +78,8 @@ __device__ __forceinline__ void grad6_point(const cpx<Real> (*sU)[NPEM],
         cpx<Real> x = {0, 0}, y = {0, 0};
 #pragma unroll
         for (int k = 0; k < NPED; k++) {
-            x = cfma(sU[c][k * NPED + j], G.gxi_col[k], x);
-            y = cfma(sU[c][i * NPED + k], G.g_col[k], y);
+            x = cfma(U(c, k * NPED + j), gx[k], x);
+            y = cfma(U(c, i * NPED + k), gz[k], y);
         }
         dS[c] = cadd(cmul(x, g.dzdeta), cmul(y, g.dzdxii));
         dZ[c] = cadd(cmul(x, g.dsdeta), cmul(y, g.dsdxii));
@@ -107,6 +106,19 @@ __device__ __forceinline__ void grad6_point(const cpx<Real> (*sU)[NPEM],
         eps[1] = cadd(ialpha(ralpha, dS[1]), dS[0]);
         eps[3] = cadd(eps[3], ialpha(ralpha, dS[2]));
     }
+}
+
+// The same from a displacement tile sU[3][25] in LDS.
+template <typename Real>
+__device__ __forceinline__ void grad6_point(const cpx<Real> (*sU)[NPEM],
+                                            const cpx<Real> (&u)[3],
+                                            Real ralpha, bool axial_row0,
+                                            int i, int j,
+                                            const PointG<Real> &G,
+                                            const PointOps<Real> &g,
+                                            cpx<Real> (&eps)[6]) {
+    grad6_at<Real>([&](int c, int p) { return sU[c][p]; }, u, ralpha,
+                   axial_row0, i, j, G.gxi_col, G.g_col, g, eps);
 }
 
 // computeGrad9 at point (i, j) (GradientQuadrature.hpp:181-201): the full
@@ -322,23 +334,33 @@ __device__ __forceinline__ void quad_xy(cpx<Real> dfds, cpx<Real> dfdz,
     Y = cadd(cmul(dfds, q.dzdxii), cmul(dfdz, q.dsdxii));
 }
 
-// Quadrature at this point, first half: forms X, Y from the six stress
+// Quadrature at this point, first half: X, Y from the six stress
 // components (with the axial L'Hospital corrections of
-// computeQuad_1overS_addTo, :493-497, folded into row 0 of X and Y), puts
-// them in the LDS tiles sX, sY, and returns the local 1/s term L
-// (GradientQuadrature.hpp:311-318).
+// computeQuad_1overS_addTo, :493-497, folded into row 0 of X and Y) and the
+// local 1/s term L (GradientQuadrature.hpp:311-318).
 template <typename Real>
-__device__ __forceinline__ void quad_prep_core(
-    const cpx<Real> (&X)[3], const cpx<Real> (&Y)[3], const cpx<Real> (&b)[3],
-    bool axial_row0, const PointOps<Real> &q, cpx<Real> (*sX)[NPEM],
-    cpx<Real> (*sY)[NPEM], int ipnt, cpx<Real> (&L)[3]);
+__device__ __forceinline__ void quad_xyl(const cpx<Real> (&b)[3],
+                                         bool axial_row0,
+                                         const PointOps<Real> &q,
+                                         cpx<Real> (&X)[3], cpx<Real> (&Y)[3],
+                                         cpx<Real> (&L)[3]) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        L[c] = cmul(b[c], -q.invs);
+        if (axial_row0) {
+            X[c] = csub(X[c], cmul(b[c], q.dzdeta));
+            Y[c] = csub(Y[c], cmul(b[c], q.dzdxii));
+        }
+    }
+}
 
 template <typename Real>
-__device__ __forceinline__ void quad6_prep(
-    const cpx<Real> (&sig)[6], Real alpha, bool axial_row0,
-    const PointOps<Real> &q, cpx<Real> (*sX)[NPEM], cpx<Real> (*sY)[NPEM],
-    int ipnt, cpx<Real> (&L)[3]) {
-    cpx<Real> X[3], Y[3];
+__device__ __forceinline__ void quad6_xyl(const cpx<Real> (&sig)[6],
+                                          Real alpha, bool axial_row0,
+                                          const PointOps<Real> &q,
+                                          cpx<Real> (&X)[3],
+                                          cpx<Real> (&Y)[3],
+                                          cpx<Real> (&L)[3]) {
     // (dFdS, dFdZ) per output component: (0,4), (5,3), (4,2)
     quad_xy(sig[0], sig[4], q, X[0], Y[0]);
     quad_xy(sig[5], sig[3], q, X[1], Y[1]);
@@ -347,7 +369,22 @@ __device__ __forceinline__ void quad6_prep(
     b[0] = csub(ialpha(alpha, sig[5]), sig[1]);
     b[1] = cadd(ialpha(alpha, sig[1]), sig[5]);
     b[2] = ialpha(alpha, sig[3]);
-    quad_prep_core<Real>(X, Y, b, axial_row0, q, sX, sY, ipnt, L);
+    quad_xyl<Real>(b, axial_row0, q, X, Y, L);
+}
+
+// The first half into the LDS tiles sX, sY.
+template <typename Real>
+__device__ __forceinline__ void quad6_prep(
+    const cpx<Real> (&sig)[6], Real alpha, bool axial_row0,
+    const PointOps<Real> &q, cpx<Real> (*sX)[NPEM], cpx<Real> (*sY)[NPEM],
+    int ipnt, cpx<Real> (&L)[3]) {
+    cpx<Real> X[3], Y[3];
+    quad6_xyl<Real>(sig, alpha, axial_row0, q, X, Y, L);
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        sX[c][ipnt] = X[c];
+        sY[c][ipnt] = Y[c];
+    }
 }
 
 // The same first half for a 9-component tensor f (computeQuad9,
@@ -366,24 +403,9 @@ __device__ __forceinline__ void quad9_prep(
     b[0] = csub(ialpha(alpha, f[1]), f[4]);
     b[1] = cadd(ialpha(alpha, f[4]), f[1]);
     b[2] = ialpha(alpha, f[7]);
-    quad_prep_core<Real>(X, Y, b, axial_row0, q, sX, sY, ipnt, L);
-}
-
-template <typename Real>
-__device__ __forceinline__ void quad_prep_core(
-    const cpx<Real> (&Xin)[3], const cpx<Real> (&Yin)[3],
-    const cpx<Real> (&b)[3], bool axial_row0, const PointOps<Real> &q,
-    cpx<Real> (*sX)[NPEM], cpx<Real> (*sY)[NPEM], int ipnt,
-    cpx<Real> (&L)[3]) {
-    cpx<Real> X[3] = {Xin[0], Xin[1], Xin[2]};
-    cpx<Real> Y[3] = {Yin[0], Yin[1], Yin[2]};
+    quad_xyl<Real>(b, axial_row0, q, X, Y, L);
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-        L[c] = cmul(b[c], -q.invs);
-        if (axial_row0) {
-            X[c] = csub(X[c], cmul(b[c], q.dzdeta));
-            Y[c] = csub(Y[c], cmul(b[c], q.dzdxii));
-        }
         sX[c][ipnt] = X[c];
         sY[c][ipnt] = Y[c];
     }

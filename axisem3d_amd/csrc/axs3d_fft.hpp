@@ -371,29 +371,36 @@ __host__ __device__ __forceinline__ int divm(int a, uint32_t mg) {
 
 // Plan words per Nr (FFT_PLAN_W of them): word 0 = number of passes |
 // (table length << 8); per pass p, in decimation-in-frequency order:
-// [1 + 3p] = radix | (m << 8), [2 + 3p] = ceil(2^32 / m) (0 for m = 1),
-// [3 + 3p] = offset of the pass's twiddles | (butterflies << 16).
+// [1 + 4p] = radix | (m << 8), [2 + 4p] = ceil(2^32 / m) (0 for m = 1),
+// [3 + 4p] = offset of the pass's twiddles | (butterflies << 16), [4 + 4p] =
+// ceil(2^32 / butterflies) (0 for one butterfly).
 constexpr int FFT_MAX_PASSES = 12;
-constexpr int FFT_PLAN_W = 1 + 3 * FFT_MAX_PASSES;
+constexpr int FFT_PLAN_W = 1 + 4 * FFT_MAX_PASSES;
 // Largest Nr (the longest lucky number Nr <= 2048 is 2048 itself).
 constexpr int FFT_NR_CAP = 2048;
 
-// One pass of radix R of the series buf by lanes lane, lane + nlanes, ...
+// One pass of radix R of ns series, stride apart from buf on, by lanes lane,
+// lane + nlanes, ...: the butterflies of all series in one count, so that
+// series of few butterflies still fill the lanes.
 template <typename Real, int R, bool INV>
 __host__ __device__ __forceinline__ void fft_pass(
-    cpx<Real> *buf, int nb, int m, uint32_t mg,
-    const cpx<Real> *__restrict__ tws, int lane, int nlanes) {
+    cpx<Real> *buf, int stride, int ns, int nb, uint32_t mgb, int m,
+    uint32_t mg, const cpx<Real> *__restrict__ tws, int lane, int nlanes) {
     const int L = m * R;
-    for (int b = lane; b < nb; b += nlanes) {
+    const int total = ns * nb;
+    for (int x = lane; x < total; x += nlanes) {
+        const int s = nb == 1 ? x : divm(x, mgb);
+        const int b = x - mul24(s, nb);
         const int blk = m == 1 ? b : divm(b, mg);
         const int j = b - mul24(blk, m);
         const int base = mul24(blk, L) + j;
+        cpx<Real> *bs = buf + mul24(s, stride);
         int ad[R];
         cpx<Real> v[R];
         fftc::sfor<R>([&](auto I) {
             constexpr int r = decltype(I)::value;
             ad[r] = pad(base + mul24(r, m));
-            v[r] = buf[ad[r]];
+            v[r] = bs[ad[r]];
         });
         const cpx<Real> *w = tws + mul24(j, R - 1);
         if (!INV && m > 1) {
@@ -416,7 +423,7 @@ __host__ __device__ __forceinline__ void fft_pass(
         }
         fftc::sfor<R>([&](auto I) {
             constexpr int r = decltype(I)::value;
-            buf[ad[r]] = v[r];
+            bs[ad[r]] = v[r];
         });
     }
 }
@@ -424,18 +431,20 @@ __host__ __device__ __forceinline__ void fft_pass(
 // Pass p of the plan (radix switch).
 template <typename Real, bool INV>
 __host__ __device__ __forceinline__ void fft_pass_p(
-    cpx<Real> *buf, const uint32_t *__restrict__ plan,
+    cpx<Real> *buf, int stride, int ns, const uint32_t *__restrict__ plan,
     const cpx<Real> *__restrict__ tw, int p, int lane, int nlanes) {
-    const uint32_t w0 = plan[1 + 3 * p];
-    const uint32_t mg = plan[2 + 3 * p];
-    const uint32_t w2 = plan[3 + 3 * p];
+    const uint32_t w0 = plan[1 + 4 * p];
+    const uint32_t mg = plan[2 + 4 * p];
+    const uint32_t w2 = plan[3 + 4 * p];
+    const uint32_t mgb = plan[4 + 4 * p];
     const int R = (int)(w0 & 255u), m = (int)(w0 >> 8);
     const int nb = (int)(w2 >> 16);
     const cpx<Real> *tws = tw + (w2 & 0xffffu);
     switch (R) {
 #define AXS3D_FFT_CASE(RR)                                                   \
     case RR:                                                                 \
-        fft_pass<Real, RR, INV>(buf, nb, m, mg, tws, lane, nlanes);          \
+        fft_pass<Real, RR, INV>(buf, stride, ns, nb, mgb, m, mg, tws, lane,  \
+                                nlanes);                                     \
         break;
         AXS3D_FFT_CASE(2)
         AXS3D_FFT_CASE(3)
@@ -457,26 +466,35 @@ __host__ __device__ __forceinline__ void fft_pass_p(
     }
 }
 
-// Whole transform of buf by one wave (lane = lane index in the wave).
-// The inverse takes the natural order and leaves slice k at pos[k]; the
-// forward takes that order and leaves the natural one.
+// Whole transforms of ns series, stride apart from buf on, by one wave (lane
+// = lane index in the wave).  The inverse takes the natural order and leaves
+// slice k at pos[k]; the forward takes that order and leaves the natural
+// one.
 template <typename Real>
-__device__ __forceinline__ void wave_fft(cpx<Real> *buf,
+__device__ __forceinline__ void wave_fft(cpx<Real> *buf, int stride, int ns,
                                          const uint32_t *__restrict__ plan,
                                          bool inv, const cpx<Real> *tw,
                                          int lane) {
     const int np = (int)(plan[0] & 255u);
     if (inv) {
         for (int p = 0; p < np; p++) {
-            fft_pass_p<Real, true>(buf, plan, tw, p, lane, 64);
+            fft_pass_p<Real, true>(buf, stride, ns, plan, tw, p, lane, 64);
             wave_sync();
         }
     } else {
         for (int p = np - 1; p >= 0; p--) {
-            fft_pass_p<Real, false>(buf, plan, tw, p, lane, 64);
+            fft_pass_p<Real, false>(buf, stride, ns, plan, tw, p, lane, 64);
             wave_sync();
         }
     }
+}
+// One series.
+template <typename Real>
+__device__ __forceinline__ void wave_fft(cpx<Real> *buf,
+                                         const uint32_t *__restrict__ plan,
+                                         bool inv, const cpx<Real> *tw,
+                                         int lane) {
+    wave_fft<Real>(buf, 0, 1, plan, inv, tw, lane);
 }
 
 // ---------------------------------------------------------- host side
@@ -491,9 +509,9 @@ inline void fft_host_run(cpx<Real> *buf, const uint32_t *plan, bool inv,
         const int p = inv ? i : np - 1 - i;
         for (int lane = 0; lane < 64; lane++) {
             if (inv)
-                fft_pass_p<Real, true>(buf, plan, tw, p, lane, 64);
+                fft_pass_p<Real, true>(buf, 0, 1, plan, tw, p, lane, 64);
             else
-                fft_pass_p<Real, false>(buf, plan, tw, p, lane, 64);
+                fft_pass_p<Real, false>(buf, 0, 1, plan, tw, p, lane, 64);
         }
     }
 }
@@ -558,10 +576,14 @@ inline void fft_build_plan(int nr, const std::vector<int> &rad,
     int span = nr, ntw = 0;
     for (size_t p = 0; p < rad.size(); p++) {
         const int R = rad[p], m = span / R;
-        words[1 + 3 * p] = (uint32_t)R | ((uint32_t)m << 8);
-        words[2 + 3 * p] =
-            m == 1 ? 0u : (uint32_t)((((uint64_t)1 << 32) + m - 1) / m);
-        words[3 + 3 * p] = (uint32_t)ntw | ((uint32_t)(nr / R) << 16);
+        auto magic = [](int d) {
+            return d == 1 ? 0u
+                          : (uint32_t)((((uint64_t)1 << 32) + d - 1) / d);
+        };
+        words[1 + 4 * p] = (uint32_t)R | ((uint32_t)m << 8);
+        words[2 + 4 * p] = magic(m);
+        words[3 + 4 * p] = (uint32_t)ntw | ((uint32_t)(nr / R) << 16);
+        words[4 + 4 * p] = magic(nr / R);
         for (int j = 0; j < m; j++)
             for (int q = 1; q < R; q++) {
                 const fftc::CS w = fftc::cs2pi(-(long)j * q, span);

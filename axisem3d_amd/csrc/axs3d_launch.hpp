@@ -367,6 +367,27 @@ constexpr size_t CARD_SCRATCH_BYTES = (size_t)4 << 30;
 template <typename Real>
 void launch_cd_grad(hipStream_t st, const CardArgs<Real> &a,
                     const CardBatch &bt, StepArgs &h);
+// A group of 3D elements for the one-kernel form (axs3d_fused.hip): list3d
+// positions [begin, end), all of material type mtype.
+struct FusedGroup {
+    int mtype, begin, end, nr_max;
+};
+// Largest Nr the one-kernel form can index.
+constexpr int FUSED_NR_CAP = 400;
+// Largest dynamic LDS the one-kernel form takes for an element (one block
+// per CU: faster than the three-kernel form up to there, 960 elements of Nr
+// 11 to 121 take 164 us a step without it, 134 with it up to Nr 90 and 98 up
+// to 121), the fewest elements of a launch group, and of a type next to
+// elements of larger Nr.
+constexpr size_t FUSED_LDS_MAX = (size_t)158 << 10;
+constexpr int FUSED_GROUP_MIN = 512;
+constexpr int FUSED_WITH_LARGER_MIN = 256;
+// Its dynamic LDS for an element of nr.
+template <typename Real>
+size_t fused_lds_bytes(int nr);
+template <typename Real>
+void launch_cd_fused(hipStream_t st, const CardArgs<Real> &a,
+                     const FusedGroup &g, StepArgs &h);
 template <typename Real>
 void launch_cd_stress(hipStream_t st, const CardArgs<Real> &a,
                       const CardBatch &bt);

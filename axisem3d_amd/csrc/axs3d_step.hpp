@@ -90,7 +90,7 @@ __device__ __forceinline__ void add_source(const SourceArgs<Real> &s, int e,
 // from a table and the points of a receiver (5 on an element edge) are
 // loaded without a branch between them, since the block is bound by the
 // latency of its loads.  Every thread of the block must call it; red holds
-// three values per wave (at most 8 waves).  The one-wave form with a
+// three values per wave.  The one-wave form with a
 // branch per point and sincos per order, in a launch of its own, took 7 us
 // a step at 3 orders and 87 us at 400 (32 receivers).
 __device__ __forceinline__ void record_receiver(const RecordArgs &a, int r,

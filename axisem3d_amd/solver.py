@@ -461,4 +461,6 @@ class GpuSolver:
                 "scratch_sizes_timed": int(ms[2]),
                 "fft_max_radix": int(r[3]),
                 "fft_radices_timed": {int(r[5 + 2 * i]): r[6 + 2 * i]
-                                      for i in range(int(r[4]))}}
+                                      for i in range(int(r[4]))},
+                "fused_elements": int(r[5 + 2 * int(r[4])]),
+                "fused_nr_max": int(r[6 + 2 * int(r[4])])}

@@ -134,7 +134,7 @@ def build_workload(name, nsteps):
     return spec, cfg
 
 
-def bytes_per_step(spec, real):
+def bytes_per_step(spec, real, fused_nr=0):
     """Algorithmic HBM bytes of one step, by kernel: every array touched
     once, intermediates (the cardinal scratch, the element-local forces'
     read by the point kernel aside) on chip.
@@ -148,8 +148,11 @@ def bytes_per_step(spec, real):
       and 6 Real memory stress, the last two read and written.
     cd_quad: element force write per point-mode of 3D elements, the 5
       integral-factor rows.
+    cd_fused: the same three of the 3D elements with Nr <= fused_nr,
+      which run as one kernel.
     point: element forces read, u, v, a read+written (FP64), per-point
-      data."""
+      data: the plain Newmark update's (a run of several steps marches two
+      fields and moves 96 B less)."""
     nupd = spec.n_updates_per_step()
     E, U = spec.n_solid_elements, spec.n_solid_points
     nr = spec.elem_nr.astype(np.int64)
@@ -158,28 +161,35 @@ def bytes_per_step(spec, real):
     mtype = getattr(spec, "elem_mtype", None)
     npar = np.full(E, 2) if mtype is None else \
         np.array([2, 5, 21])[np.asarray(mtype)]
+    att = getattr(spec, "att", None)
     # point-modes served by 3D elements, split by the elements' share of
     # each point (the 3D workloads are all-3D, so this is exact there)
-    frac3d = float(is3d.mean()) if E else 0.0
-    n3d = int(is3d.sum())
-    nupd3 = int(round(nupd * frac3d))
-    nupd1 = nupd - nupd3
-    fr = nupd1 * (48 + 6 * real) + (E - n3d) * (10 * 25 * real + 25 * 4 + 1
-                                               + 25 * real * 2)
-    grad = nupd3 * 48 + n3d * (5 * 25 * real + 25 * 4 + 1)
-    stress = int((nr[is3d] * npar[is3d]).sum()) * 25 * real
-    att = getattr(spec, "att", None)
-    if att is not None:
-        npa = 4 if att["cg4"] else 25
-        slices = int(nr[is3d].sum())
-        # moduli and memory stress in the working precision, memory
-        # variables FP64 (read and written)
-        stress += slices * npa * (real * (2 + 2 * 6) +
-                                  8 * 2 * 6 * att["nsls"])
-    quad = nupd3 * 6 * real + n3d * 5 * 25 * real
+    nu1 = nr // 2 + 1
+
+    def cardinal(sel):
+        n = int(sel.sum())
+        upd = int(round(nupd * float(nu1[sel].sum()) /
+                        max(float(nu1.sum()), 1.0)))
+        grad = upd * 48 + n * (5 * 25 * real + 25 * 4 + 1)
+        stress = int((nr[sel] * npar[sel]).sum()) * 25 * real
+        if att is not None:
+            npa = 4 if att["cg4"] else 25
+            # moduli and memory stress in the working precision, memory
+            # variables FP64 (read and written)
+            stress += int(nr[sel].sum()) * npa * (
+                real * (2 + 2 * 6) + 8 * 2 * 6 * att["nsls"])
+        return upd, grad, stress, upd * 6 * real + n * 5 * 25 * real
+
+    fused = is3d & (nr <= fused_nr)
+    updf, *f3 = cardinal(fused)
+    upd3, grad, stress, quad = cardinal(is3d & ~fused)
+    n1 = int((~is3d).sum())
+    fr = (nupd - updf - upd3) * (48 + 6 * real) + n1 * (
+        10 * 25 * real + 25 * 4 + 1 + 25 * real * 2)
     point = nupd * (6 * real + 6 * 48 + 4) + U * (4 + 4 + 4 + 1 + 8 + 16)
     return {"fr": int(fr), "cd_grad": int(grad), "cd_stress": int(stress),
-            "cd_quad": int(quad), "point": int(point)}
+            "cd_quad": int(quad), "cd_fused": int(sum(f3)),
+            "point": int(point)}
 
 
 def source_fingerprint():
@@ -528,18 +538,22 @@ def main():
 
     names = {capi.KERNEL_STIFFNESS: "solid stiffness, Fourier path",
              capi.KERNEL_STIFFNESS_3D: "solid stiffness, cardinal path "
-                                       "(all three kernels)",
+                                       "(all its kernels)",
              capi.KERNEL_CD_GRAD: "k_cd_grad",
              capi.KERNEL_CD_STRESS: "k_cd_stress",
              capi.KERNEL_CD_QUAD: "k_cd_quad",
+             capi.KERNEL_CD_FUSED: "k_cd_fused",
              capi.KERNEL_POINT: "k_point",
              capi.KERNEL_SOURCE: "moment source",
              capi.KERNEL_RECORD: "receivers"}
-    b = bytes_per_step(spec, 4)
+    tune32 = prof32.pop("autotune")
+    b = bytes_per_step(spec, 4, tune32["fused_nr_max"]
+                       if tune32["fused_elements"] else 0)
     # algorithmic bytes per step of each timed group
     byts = {capi.KERNEL_STIFFNESS: b["fr"],
             capi.KERNEL_STIFFNESS_3D: b["cd_grad"] + b["cd_stress"] +
-            b["cd_quad"],
+            b["cd_quad"] + b["cd_fused"],
+            capi.KERNEL_CD_FUSED: b["cd_fused"],
             capi.KERNEL_CD_GRAD: b["cd_grad"],
             capi.KERNEL_CD_STRESS: b["cd_stress"],
             capi.KERNEL_CD_QUAD: b["cd_quad"],
@@ -555,7 +569,6 @@ def main():
             "avg_us": ms / cnt * 1e3,
             "bytes_per_launch": byts[k] / per_step,
             "achieved_GBs": byts[k] / (ms / a.steps * 1e-3) / 1e9}
-    tune32 = prof32.pop("autotune")
     tg = prof32.pop("graph_s")
     if out_64 is not None:
         prof64.pop("autotune")

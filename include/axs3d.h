@@ -75,7 +75,8 @@ enum axs3d_kernel_id {
     AXS3D_KERNEL_CD_GRAD = 7,     /* cardinal path: gradient, per batch  */
     AXS3D_KERNEL_CD_STRESS = 8,   /* cardinal path: FFT, stress, FFT     */
     AXS3D_KERNEL_CD_QUAD = 9,     /* cardinal path: quadrature           */
-    AXS3D_NUM_KERNELS = 10
+    AXS3D_KERNEL_CD_FUSED = 10,  /* cardinal path of small Nr, one kernel */
+    AXS3D_NUM_KERNELS = 11
 };
 
 /* Context.  Replaces the construction of Domain + NewmarkTimeScheme in
@@ -537,7 +538,9 @@ int axs3d_autotune_info(const axs3d_ctx *ctx, int *cardinal_occupancy,
 /* Every choice the autotuner made at axs3d_finalize (no reference
  * counterpart): out[0] the chosen cardinal pass (ms), [1] the scratch
  * size (MiB), [2] scratch sizes timed, [3] the FFT plans' largest pass
- * radix, [4] radices timed, then (radix, pass ms) for each radix timed;
+ * radix, [4] radices timed, then (radix, pass ms) for each radix timed,
+ * then the number of 3D elements that take the one-kernel form and the
+ * largest Nr it takes;
  * at most n values, their count in *written. */
 int axs3d_autotune_report(const axs3d_ctx *ctx, double *out, int n,
                           int *written);

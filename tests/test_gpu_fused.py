@@ -1,0 +1,89 @@
+"""3D elements of small Nr in the one-kernel form of the cardinal path
+(displacement to element forces with the strain series of all GLL points in
+LDS) against the FP64 oracle: stage stiffness from a random state, twice, so
+that the SLS memory enters the second, and seismograms of a short run with
+the source inside such an element.
+
+Domains: a spherical sector of three by two elements, axial ones among them,
+with element Nr 1 to 5 (single butterflies, even and odd, orders that are
+mean or Nyquist only), a ramp of small Nr with points of fewer orders than
+their element, primes, and a ramp over the largest Nr that fits the LDS of
+either precision, so that neighbouring elements take the two forms; all
+media, with no, CG4 and FULL attenuation of 5 and of 3 solids.
+
+Tolerances as for the other element kernels: relative 1e-13 (FP64) and 1e-5
+(FP32+FP64) per stage, 1e-12 and 1e-4 over the run."""
+import numpy as np
+import pytest
+
+import oracle
+from axisem3d_amd import preloop
+
+pytestmark = pytest.mark.gpu
+STEPS = 30
+
+
+def _spec(nr0, nr1, mtype, att, nsls):
+    sp = preloop.spherical_regional(
+        ntheta=3, nrad=2, theta_max_deg=3.0, depth=100e3, nu_min=1, nu_max=1,
+        nsteps=STEPS, attenuation=att is not None, cg4=att == "cg4",
+        nsls=nsls, corr_len=40e3, bound_nr=False)
+    s_max = 6371e3 * np.sin(np.radians(3.0))
+    mesh = sp._mesh
+    _, prof = preloop.layered_profile(11, 6371e3, 6271e3)
+    field, a = sp._field, sp._att_in
+    sp = preloop.build_domain(
+        mesh, prof, lambda s, z: nr0 + (nr1 - nr0) * s / s_max, courant=0.5,
+        lucky=nr1 > 7, bound_nr=False)
+    sp._courant /= max(1.0, 0.4 * nr1)
+    E = sp.n_solid_elements
+    mt = {"iso": 0, "ti": 1, "aniso": 2}.get(mtype)
+    types = np.arange(E) % 3 if mt is None else np.full(E, mt)
+    preloop.make_media(sp, types.astype(np.uint8), field=field,
+                       mask3d=np.ones(E, bool), att=a, seed=4)
+    preloop.finish_regional(sp, STEPS, src_depth=30e3, f_peak=1.0,
+                            n_receivers=3, theta_max_deg=3.0)
+    return sp
+
+
+def _rel(a, b):
+    return np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300)
+
+
+CASES = [(1, 1, "iso", None, 0), (2, 2, "mixed", "cg4", 5),
+         (3, 3, "ti", "full", 3), (4, 4, "aniso", "cg4", 5),
+         (5, 5, "mixed", "full", 5), (4, 16, "mixed", "cg4", 5),
+         (9, 45, "mixed", "cg4", 3), (13, 13, "iso", None, 0),
+         (60, 91, "mixed", "full", 5), (70, 90, "ti", "cg4", 5),
+         (150, 190, "iso", "cg4", 5), (64, 64, "aniso", None, 0)]
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-13), ("fp32", 1e-5)])
+@pytest.mark.parametrize("nr0,nr1,mtype,att,nsls", CASES)
+def test_small_nr_matches_oracle(prec, tol, nr0, nr1, mtype, att, nsls):
+    from axisem3d_amd.solver import GpuSolver
+    sp = _spec(nr0, nr1, mtype, att, max(nsls, 1))
+    o = oracle.Oracle(sp)
+    g = GpuSolver(sp, prec)
+    rng = np.random.default_rng(21)
+    for k in range(2):
+        u = rng.standard_normal((o.nmodes, 3)) + 1j * rng.standard_normal(
+            (o.nmodes, 3))
+        g.set_field("displ", u)
+        g.set_field("stiff", np.zeros_like(u))
+        g.computeStiffness()
+        e = _rel(g.get_field("stiff"), o.stiffness(u))
+        print(f"Nr {nr0}..{nr1} {mtype} {att} {prec} pass {k}: {e:.2e}")
+        assert e < tol
+    g.close()
+    o = oracle.Oracle(sp)
+    ref = o.run(STEPS)
+    g = GpuSolver(sp, prec)
+    g.run(STEPS)
+    es, eu = _rel(g.seismograms(), ref), _rel(g.get_field("displ"), o.displ)
+    print(f"  run: seismograms {es:.2e}, field {eu:.2e}")
+    assert np.abs(o.displ).max() > 0
+    assert eu < (1e-12 if prec == "fp64" else 1e-4)
+    if np.abs(ref).max() > 0:
+        assert es < (1e-12 if prec == "fp64" else 1e-4)
+    g.close()
