@@ -144,12 +144,15 @@ __global__ __launch_bounds__(CD_EMB_THREADS) void k_cd_grad(
         const EMItem it = s.em_list[em];
         e = it.elem;
         alpha = it.alpha;
-        const int p = s.elem_points[e * NPEM + ipnt];
-        if (alpha < s.point_nu1[p]) {
-            const double *src = s.displ + (size_t)(s.point_off[p] + alpha) * 6;
+        const uint2 pm = s.elem_modes[e * NPEM + ipnt];
+        if (alpha < (int)pm.y) {
+            const double2 *src = reinterpret_cast<const double2 *>(
+                s.displ + (size_t)(pm.x + alpha) * 6);
 #pragma unroll
-            for (int c = 0; c < 3; c++)
-                u[c] = {(Real)src[2 * c], (Real)src[2 * c + 1]};
+            for (int c = 0; c < 3; c++) {
+                const double2 v = src[c];
+                u[c] = {(Real)v.x, (Real)v.y};
+            }
         }
 #pragma unroll
         for (int c = 0; c < 3; c++) sU[eml][c][ipnt] = u[c];
@@ -259,8 +262,8 @@ __global__ __launch_bounds__(CD_EMB_THREADS) void k_cd_quad(CardArgs<Real> a,
         quad6_point<Real>(sig, (Real)alpha, axial && i == 0, q, sX[eml],
                           sY[eml], ipnt, i, j, G, active, F);
     }
-    if (active && alpha < s.point_nu1[s.elem_points[e * NPEM + ipnt]]) {
-        add_source(s.src, e, ipnt, alpha, F);
+    if (active && alpha < (int)s.elem_modes[e * NPEM + ipnt].y) {
+        add_source(s.src, source_of(s.src, e), ipnt, alpha, F);
         Real *dst = s.eb + ((size_t)s.elem_eb_off[e] + (size_t)ipnt * nu1 +
                             alpha) * 6;
 #pragma unroll

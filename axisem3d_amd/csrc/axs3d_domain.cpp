@@ -1198,6 +1198,14 @@ void DomainBase::finalize() {
     up(dInvMass, inv.data(), inv.size() * 8);
     up(dModePoint, modePoint.data(), modePoint.size() * 4);
     up(dElemPoints, hElemPoints.data(), hElemPoints.size() * 4);
+    {
+        std::vector<uint2> em2(hElemPoints.size());
+        for (size_t k = 0; k < em2.size(); k++) {
+            const int p = hElemPoints[k];
+            em2[k] = make_uint2(off[p], (uint32_t)nu1[p]);
+        }
+        up(dElemModes, em2.data(), em2.size() * sizeof(uint2));
+    }
     up(dElemAxial, hElemAxial.data(), hElemAxial.size());
     up(dElemNu1, eNu1.data(), eNu1.size() * 4);
     up(dEMList, em.data(), em.size() * sizeof(EMItem));
@@ -1729,11 +1737,20 @@ class Domain final : public DomainBase {
 public:
     Domain(int device, int precision) : DomainBase(device, precision) {}
 
+    // groups of EMB element-modes of the Fourier path before those of
+    // material type t (the SLS state's order; each type begins a group)
+    int emGroup(int t) const {
+        int g = 0;
+        for (int k = 0; k < t; k++)
+            g += (mEMTypeBegin[k + 1] - mEMTypeBegin[k] + EMB - 1) / EMB;
+        return g;
+    }
     StiffArgs<Real> stiffArgs() const {
         StiffArgs<Real> a;
         a.n_em = mNumEM;
         a.em_list = dEMList.as<EMItem>();
         a.elem_points = dElemPoints.as<int32_t>();
+        a.elem_modes = dElemModes.as<uint2>();
         a.elem_axial = dElemAxial.as<uint8_t>();
         a.elem_ops = dElemOps.as<Real>();
         a.elem_mat = dElemMat.as<Real>();
@@ -1742,6 +1759,7 @@ public:
         a.prt_idx = hPrtElems.empty() ? nullptr : dPrtIdx.as<int32_t>();
         a.prt = hPrtElems.empty() ? nullptr : dPrt.as<Real>();
         for (int k = 0; k < 4; k++) a.em_type_begin[k] = mEMTypeBegin[k];
+        for (int k = 0; k < 3; k++) a.em_group_begin[k] = emGroup(k);
         a.point_off = dPointOff.as<uint32_t>();
         a.point_nu1 = dPointNu1.as<int32_t>();
         a.displ = dDispl.as<double>();
@@ -3093,10 +3111,11 @@ private:
             std::vector<Real> a1(hAtt1D.begin(), hAtt1D.end());
             dAtt1D.alloc(a1.size() * sizeof(Real));
             dAtt1D.upload(a1.data(), a1.size() * sizeof(Real), st);
-            dMemVarFR.alloc((size_t)mNumEM * mNsls * 6 * npa * 2 *
-                            sizeof(double));
+            // whole groups of EMB element-modes per material type
+            const size_t em = (size_t)emGroup(3) * EMB;
+            dMemVarFR.alloc(em * mNsls * 6 * npa * 2 * sizeof(double));
             dMemVarFR.zero(st);
-            dDStressFR.alloc((size_t)mNumEM * 6 * npa * 2 * sizeof(Real));
+            dDStressFR.alloc(em * 6 * npa * 2 * sizeof(Real));
             dDStressFR.zero(st);
         }
         if (!hTwTab.empty()) {

@@ -387,7 +387,7 @@ protected:
     // device: fields (FP64) and stiffness (Real)
     DeviceBuffer dDispl, dVeloc, dAccel, dStiff;
     // device: elements
-    DeviceBuffer dElemPoints, dElemAxial, dElemNu1, dElemOps, dElemMat,
+    DeviceBuffer dElemPoints, dElemModes, dElemAxial, dElemNu1, dElemOps, dElemMat,
         dMatOff, dRot, dEMList, dGTab, dElemEBOff, dEB, dAdj, dPrtIdx, dPrt;
     // device: cardinal path
     DeviceBuffer dElemNr, dSliceOff, dPropOff, dList3D, dScrOff, dEM3D,

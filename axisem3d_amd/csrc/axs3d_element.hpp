@@ -12,7 +12,6 @@
 
 namespace axs3d {
 
-constexpr int EMB = 10;          // element-modes per 256-thread block
 constexpr int STIFF_BLOCK = 256;
 
 template <typename Real>
@@ -123,23 +122,22 @@ __device__ __forceinline__ void grad6_point(const cpx<Real> (*sU)[NPEM],
 
 // computeGrad9 at point (i, j) (GradientQuadrature.hpp:181-201): the full
 // gradient g[3 c + d] = d u_c / d x_d, x = (s, phi, z), for the particle
-// relabelling path; the same contractions as grad6_point with the s-z and
-// phi pairs kept apart.
-template <typename Real>
-__device__ __forceinline__ void grad9_point(const cpx<Real> (*sU)[NPEM],
-                                            const cpx<Real> (&u)[3],
-                                            Real ralpha, bool axial_row0,
-                                            int i, int j,
-                                            const PointG<Real> &G,
-                                            const PointOps<Real> &g,
-                                            cpx<Real> (&g9)[9]) {
+// relabelling path; the same contractions as grad6_at with the s-z and phi
+// pairs kept apart.
+template <typename Real, typename Get>
+__device__ __forceinline__ void grad9_at(Get U, const cpx<Real> (&u)[3],
+                                         Real ralpha, bool axial_row0, int i,
+                                         int j, const Real (&gx)[NPED],
+                                         const Real (&gz)[NPED],
+                                         const PointOps<Real> &g,
+                                         cpx<Real> (&g9)[9]) {
 #pragma unroll
     for (int c = 0; c < 3; c++) {
         cpx<Real> x = {0, 0}, y = {0, 0};
 #pragma unroll
         for (int k = 0; k < NPED; k++) {
-            x = cfma(sU[c][k * NPED + j], G.gxi_col[k], x);
-            y = cfma(sU[c][i * NPED + k], G.g_col[k], y);
+            x = cfma(U(c, k * NPED + j), gx[k], x);
+            y = cfma(U(c, i * NPED + k), gz[k], y);
         }
         g9[3 * c] = cadd(cmul(x, g.dzdeta), cmul(y, g.dzdxii));
         g9[3 * c + 2] = cadd(cmul(x, g.dsdeta), cmul(y, g.dsdxii));
@@ -149,11 +147,24 @@ __device__ __forceinline__ void grad9_point(const cpx<Real> (*sU)[NPEM],
         g9[4] = cmul(cadd(ialpha(ralpha, u[1]), u[0]), g.invs);
         g9[7] = cmul(ialpha(ralpha, u[2]), g.invs);
     } else {
-        // L'Hospital, as in grad6_point
+        // L'Hospital, as in grad6_at
         g9[1] = csub(ialpha(ralpha, g9[0]), g9[3]);
         g9[4] = cadd(ialpha(ralpha, g9[3]), g9[0]);
         g9[7] = ialpha(ralpha, g9[6]);
     }
+}
+
+// The same from a displacement tile sU[3][25] in LDS.
+template <typename Real>
+__device__ __forceinline__ void grad9_point(const cpx<Real> (*sU)[NPEM],
+                                            const cpx<Real> (&u)[3],
+                                            Real ralpha, bool axial_row0,
+                                            int i, int j,
+                                            const PointG<Real> &G,
+                                            const PointOps<Real> &g,
+                                            cpx<Real> (&g9)[9]) {
+    grad9_at<Real>([&](int c, int p) { return sU[c][p]; }, u, ralpha,
+                   axial_row0, i, j, G.gxi_col, G.g_col, g, g9);
 }
 
 // A gradient-shaped tensor g -> Q g Q^T, Q the rotation by the colatitude
@@ -392,11 +403,12 @@ __device__ __forceinline__ void quad6_prep(
 // (f6, f8); lower-order numerators i alpha f1 - f4, i alpha f4 + f1,
 // i alpha f7.
 template <typename Real>
-__device__ __forceinline__ void quad9_prep(
-    const cpx<Real> (&f)[9], Real alpha, bool axial_row0,
-    const PointOps<Real> &q, cpx<Real> (*sX)[NPEM], cpx<Real> (*sY)[NPEM],
-    int ipnt, cpx<Real> (&L)[3]) {
-    cpx<Real> X[3], Y[3];
+__device__ __forceinline__ void quad9_xyl(const cpx<Real> (&f)[9],
+                                          Real alpha, bool axial_row0,
+                                          const PointOps<Real> &q,
+                                          cpx<Real> (&X)[3],
+                                          cpx<Real> (&Y)[3],
+                                          cpx<Real> (&L)[3]) {
 #pragma unroll
     for (int c = 0; c < 3; c++) quad_xy(f[3 * c], f[3 * c + 2], q, X[c], Y[c]);
     cpx<Real> b[3];
@@ -404,6 +416,15 @@ __device__ __forceinline__ void quad9_prep(
     b[1] = cadd(ialpha(alpha, f[4]), f[1]);
     b[2] = ialpha(alpha, f[7]);
     quad_xyl<Real>(b, axial_row0, q, X, Y, L);
+}
+
+template <typename Real>
+__device__ __forceinline__ void quad9_prep(
+    const cpx<Real> (&f)[9], Real alpha, bool axial_row0,
+    const PointOps<Real> &q, cpx<Real> (*sX)[NPEM], cpx<Real> (*sY)[NPEM],
+    int ipnt, cpx<Real> (&L)[3]) {
+    cpx<Real> X[3], Y[3];
+    quad9_xyl<Real>(f, alpha, axial_row0, q, X, Y, L);
 #pragma unroll
     for (int c = 0; c < 3; c++) {
         sX[c][ipnt] = X[c];

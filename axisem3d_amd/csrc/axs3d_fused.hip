@@ -74,6 +74,8 @@ __global__ __launch_bounds__(FusedBlock<Real>::value) void k_cd_fused(
     const int nw = T >> 6;
     const int e = a.list3d[w0 + (int)blockIdx.x - h.rec.nrec];
     const int nr = a.elem_nr[e];
+    const int src = source_of(s.src, e);
+    Real *ebe = s.eb + (size_t)s.elem_eb_off[e] * 6;
     const int nu1 = nr / 2 + 1;
     const int nyq = (nr & 1) ? -1 : nu1 - 1;
     const int stride = fused_stride(nr);
@@ -95,9 +97,9 @@ __global__ __launch_bounds__(FusedBlock<Real>::value) void k_cd_fused(
         for (int x = t; x < nr; x += T) pos[x] = pg[x];
     }
     if (t < NPEM) {
-        const int p = s.elem_points[e * NPEM + t];
-        pnu1[t] = s.point_nu1[p];
-        poff[t] = s.point_off[p];
+        const uint2 pm = s.elem_modes[e * NPEM + t];
+        poff[t] = pm.x;
+        pnu1[t] = (int)pm.y;
     }
     if (t < 2 * NPEM) sG[t / NPEM][t % NPEM] = s.gtab[t];
     if (NS != 0 && t < 3 * a.nsls) {
@@ -253,7 +255,6 @@ __global__ __launch_bounds__(FusedBlock<Real>::value) void k_cd_fused(
         }
     }
     __syncthreads();
-    Real *ebe = s.eb + (size_t)s.elem_eb_off[e] * 6;
     for (int x = t; x < items; x += T) {
         const int pt = div22(x, mgu), al = x - pt * nu1;
         if (al >= pnu1[pt]) continue;
@@ -279,7 +280,7 @@ __global__ __launch_bounds__(FusedBlock<Real>::value) void k_cd_fused(
             }
             F[c] = cadd(cadd(av, bv), U[c * items + x]);
         }
-        add_source(s.src, e, pt, al, F);
+        add_source(s.src, src, pt, al, F);
         cpx<Real> *dst = reinterpret_cast<cpx<Real> *>(ebe) + (size_t)x * 3;
 #pragma unroll
         for (int c = 0; c < 3; c++) dst[c] = F[c];

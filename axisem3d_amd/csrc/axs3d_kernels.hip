@@ -1,10 +1,11 @@
 // axs3d_kernels.hip -- CDNA4 (gfx950) kernels of the stiffness path.
 //
 // Fourier-path solid element stiffness (1D material, no PRT): one thread
-// per (element, Fourier order alpha, GLL point); ten element-modes per
-// 256-thread block (four wave64s).  The element-mode displacement tile and
-// the quadrature pre-products are staged in LDS so the two 5x5 GLL
-// contractions (gradient and quadrature) read neighbours from LDS instead
+// per (element, Fourier order alpha, GLL point); ten element-modes per block
+// of four waves, the element-mode fastest over the lanes.  The element-mode
+// displacement tile and the quadrature pre-products are staged in LDS so the
+// two 5x5 GLL contractions (gradient and quadrature) read neighbours from
+// LDS instead
 // of HBM.  The element kernel writes its element-local forces F (no
 // atomics); the point kernel then gathers, for every (point, mode), the
 // contributions of the elements sharing the point in ascending element
@@ -35,6 +36,61 @@ __device__ __forceinline__ int att_slot_fr(int p, int npa) {
     return p == 6 ? 0 : p == 8 ? 1 : p == 16 ? 2 : p == 18 ? 3 : -1;
 }
 
+// SLS memory per Fourier order with 1D moduli (AttenuationFull/CG4::apply,
+// AttenuationCG4.hpp:312-330, Attenuation.hpp:92-140): sigma -= sum_l m_l;
+// m_l = alpha_l m_l + beta_l ds_old; ds = iso(dlambda, dmu)(eps); m_l +=
+// gamma_l ds.  The memory variables and their recursion are FP64 (the stress
+// increments in the working precision); a block's state is one run of
+// memory, [l][d][qa][element-mode].
+template <typename Real>
+__device__ __forceinline__ cpx<double> sls_next(const StiffArgs<Real> &a,
+                                                int nsls, int l,
+                                                cpx<double> m,
+                                                cpx<double> dso,
+                                                cpx<double> dn) {
+    m = cmul(m, a.abg[l]);
+    m = cfma(dso, a.abg[nsls + l], m);
+    return cfma(dn, a.abg[2 * nsls + l], m);
+}
+
+// At an attenuation point by its own thread (group: the block's, eml: the
+// element-mode in it).
+template <typename Real>
+__device__ __forceinline__ void att_update_fr(const StiffArgs<Real> &a,
+                                              size_t group, int eml, int qa,
+                                              const cpx<Real> (&dsn)[6],
+                                              cpx<Real> (&sig)[6]) {
+    const int npa = a.npa, nsls = a.nsls;
+    const int step = npa * EMB, at = qa * EMB + eml;
+    cpx<double> *mv = reinterpret_cast<cpx<double> *>(a.mv_fr) +
+                      group * nsls * 6 * step + at;
+    cpx<Real> *ds =
+        reinterpret_cast<cpx<Real> *>(a.ds_fr) + group * 6 * step + at;
+#pragma unroll
+    for (int d = 0; d < 6; d++) {
+        const cpx<Real> o = ds[d * step];
+        const cpx<double> dso = {(double)o.re, (double)o.im};
+        const cpx<double> dn = {(double)dsn[d].re, (double)dsn[d].im};
+        cpx<double> sd = {(double)sig[d].re, (double)sig[d].im};
+        for (int l = 0; l < nsls; l++) {
+            cpx<double> &m = mv[(l * 6 + d) * step];
+            const cpx<double> m0 = m;
+            sd = csub(sd, m0);
+            m = sls_next(a, nsls, l, m0, dso, dn);
+        }
+        sig[d] = {(Real)sd.re, (Real)sd.im};
+        ds[d * step] = dsn[d];
+    }
+}
+
+// How a launch treats the SLS memory: none; at each attenuation point by
+// its thread; or CG4 with five solids, where only four points of 25 have
+// any, spread over the block (CG4_ITEMS threads, one per component, point
+// and element-mode, their loads issued before the gradient).
+enum AttForm { ATT_NONE = 0, ATT_POINT, ATT_SPREAD };
+constexpr int SPREAD_NS = 5;
+constexpr int CG4_ITEMS = 6 * 4 * EMB;
+
 // MT: material type of the element-modes [em0, em1) of em_list (0
 // isotropic, 1 TI, 2 anisotropic); em_list is grouped by type.
 // PRT: some elements carry a particle relabelling transformation
@@ -43,50 +99,81 @@ __device__ __forceinline__ int att_slot_fr(int p, int npa) {
 // material, to the undulated strain (one operand set for all orders: the
 // undulation is axisymmetric), and the stress back through the transpose
 // and computeQuad9.
-template <typename Real, bool ATT, int MT, bool PRT>
+// ATT: AttForm.
+// Bound by HBM (the displacement read, the forces written) where an element
+// has many orders, by LDS and VALU where it has few.  With the element-mode
+// fastest over the lanes a point's ten orders are one run of memory (480 B
+// of displacement, 240 B of FP32 forces) and LDS reads of one point fall on
+// consecutive banks.
+template <typename Real, int ATT, int MT, bool PRT>
 __global__ __launch_bounds__(STIFF_BLOCK) void k_solid_stiff_fr(
     StiffArgs<Real> a, int em0, int em1, StepArgs h) {
     __shared__ double red[STIFF_BLOCK / 64][3];
     if (step_head(h, red)) return;
-    __shared__ cpx<Real> sU[EMB][3][NPEM];
-    __shared__ cpx<Real> sX[EMB][3][NPEM];
-    __shared__ cpx<Real> sY[EMB][3][NPEM];
+    __shared__ cpx<Real> sX[3][NPEM][EMB];      // displacement, then X
+    __shared__ cpx<Real> sY[3][NPEM][EMB];
     __shared__ Real sG[2][NPEM];
+    // stress increments and memory sums of the spread form
+    __shared__ cpx<Real> sDn[ATT == ATT_SPREAD ? CG4_ITEMS : 1];
+    __shared__ cpx<double> sSum[ATT == ATT_SPREAD ? CG4_ITEMS : 1];
 
     const int t = threadIdx.x;
     if (t < 2 * NPEM) sG[t / NPEM][t % NPEM] = a.gtab[t];
-    const int eml = t / NPEM;
-    const int ipnt = t - eml * NPEM;
-    const int em = em0 + xcd_block(h.rec.nrec) * EMB + eml;
-    const bool active = (eml < EMB) && (em < em1);
+    const int eml = t % EMB;
+    const bool slot = t < EMB * NPEM;
+    const int ipnt = slot ? t / EMB : 0;
+    const int blk = xcd_block(h.rec.nrec);
+    const size_t group = (size_t)a.em_group_begin[MT] + blk;
+    const int em = em0 + blk * EMB + eml;
+    const bool active = slot && em < em1;
     const int i = ipnt / NPED, j = ipnt - (ipnt / NPED) * NPED;
-    const int emx = active ? eml : 0;
 
-    int e = 0, alpha = 0, nu1p = 0;
-    uint32_t off = 0;
+    // the block's share of the SLS state, one (d, qa, element-mode) per
+    // thread
+    cpx<double> m[ATT == ATT_SPREAD ? SPREAD_NS : 1];
+    cpx<double> dso = {0, 0};
+    cpx<double> *mv = nullptr;
+    cpx<Real> *ds = nullptr;
+    const bool item = ATT == ATT_SPREAD && t < CG4_ITEMS && em < em1;
+    if (ATT == ATT_SPREAD && item) {
+        mv = reinterpret_cast<cpx<double> *>(a.mv_fr) +
+             group * SPREAD_NS * CG4_ITEMS + t;
+        ds = reinterpret_cast<cpx<Real> *>(a.ds_fr) + group * CG4_ITEMS + t;
+#pragma unroll
+        for (int l = 0; l < SPREAD_NS; l++) m[l] = mv[l * CG4_ITEMS];
+        const cpx<Real> o = *ds;
+        dso = {(double)o.re, (double)o.im};
+    }
+
+    int e = 0, alpha = 0, nu1p = 0, src = -1;
+    size_t eb_at = 0;
     bool axial = false;
     cpx<Real> u[3] = {{0, 0}, {0, 0}, {0, 0}};
     if (active) {
         const EMItem it = a.em_list[em];
         e = it.elem;
         alpha = it.alpha;
-        const int p = a.elem_points[e * NPEM + ipnt];
-        nu1p = a.point_nu1[p];
-        off = a.point_off[p];
+        const uint2 pm = a.elem_modes[e * NPEM + ipnt];
+        nu1p = (int)pm.y;
         axial = a.elem_axial[e] != 0;
+        eb_at = (size_t)a.elem_eb_off[e] + (size_t)ipnt * a.elem_nu1[e];
+        src = source_of(a.src, e);
         if (alpha < nu1p) {
-            const double *src = a.displ + (size_t)(off + alpha) * 6;
+            const double2 *src = reinterpret_cast<const double2 *>(
+                a.displ + (size_t)(pm.x + alpha) * 6);
 #pragma unroll
-            for (int c = 0; c < 3; c++)
-                u[c] = {(Real)src[2 * c], (Real)src[2 * c + 1]};
+            for (int c = 0; c < 3; c++) {
+                const double2 v = src[c];
+                u[c] = {(Real)v.x, (Real)v.y};
+            }
         }
-#pragma unroll
-        for (int c = 0; c < 3; c++) sU[eml][c][ipnt] = u[c];
     }
+    if (slot)
+#pragma unroll
+        for (int c = 0; c < 3; c++) sX[c][ipnt][eml] = u[c];
     __syncthreads();
 
-    PointG<Real> G;
-    load_point_g<Real>(sG, axial, i, j, G);
+    const Real *Gxi = sG[axial ? 1 : 0];
     cpx<Real> sig[6];
     PointOps<Real> g{}, q{};
     const Real ralpha = (Real)alpha;
@@ -97,6 +184,13 @@ __global__ __launch_bounds__(STIFF_BLOCK) void k_solid_stiff_fr(
     Real rs1 = 0, rc1 = 1, rs2 = 0, rc2 = 1;
     if (active) {
         load_point_ops(a.elem_ops, e, ipnt, g, q);
+        Real gx[NPED], gz[NPED];
+#pragma unroll
+        for (int k = 0; k < NPED; k++) {
+            gx[k] = Gxi[k * NPED + i];
+            gz[k] = sG[0][k * NPED + j];
+        }
+        auto U = [&](int c, int p) { return sX[c][p][eml]; };
         cpx<Real> eps[6];
         const Real *mat = a.elem_mat + a.mat_off[e] + ipnt;
         // TI and anisotropic media work in RTZ on spherical meshes
@@ -111,12 +205,12 @@ __global__ __launch_bounds__(STIFF_BLOCK) void k_solid_stiff_fr(
         }
         if (PRT && xp != nullptr) {
             cpx<Real> g9[9];
-            grad9_point<Real>(sU[eml], u, ralpha, axial_row0, i, j, G, g, g9);
+            grad9_at<Real>(U, u, ralpha, axial_row0, i, j, gx, gz, g, g9);
             if (a.rot != nullptr)
                 rot9<cpx<Real>, Real>(g9, rs1, rc1, rs2, rc2);
             prt_sph_to_und6<cpx<Real>, Real>(g9, xp, eps);
         } else {
-            grad6_point<Real>(sU[eml], u, ralpha, axial_row0, i, j, G, g, eps);
+            grad6_at<Real>(U, u, ralpha, axial_row0, i, j, gx, gz, g, eps);
             if (rtz) rot_spz_rtz6<cpx<Real>, Real>(eps, rs1, rc1, rs2, rc2);
         }
         if constexpr (MT == 0) {
@@ -128,88 +222,85 @@ __global__ __launch_bounds__(STIFF_BLOCK) void k_solid_stiff_fr(
             aniso_hooke<cpx<Real>, Real>(
                 eps, [&](int k) { return mat[k * NPEM]; }, sig);
         }
-        if (ATT) {
-            // AttenuationFull/CG4::apply per Fourier order with 1D moduli
-            // (AttenuationCG4.hpp:312-330, Attenuation.hpp:92-140):
-            // sigma -= sum_l m_l; m_l = alpha_l m_l + beta_l ds_old;
-            // ds = iso(dlambda, dmu)(eps); m_l += gamma_l ds
-            const int npa = a.npa, nsls = a.nsls;
-            const int qa = att_slot_fr(ipnt, npa);
+        if constexpr (ATT != ATT_NONE) {
+            const int qa = att_slot_fr(ipnt, a.npa);
             if (qa >= 0) {
-                const Real *dlm = a.att1d + (size_t)e * 2 * npa + qa;
+                const Real *dlm = a.att1d + (size_t)e * 2 * a.npa + qa;
                 cpx<Real> dsn[6];
-                iso_hooke<Real>(eps, dlm[0], dlm[npa], dsn);
-                // the memory variables and their recursion in FP64 (the
-                // stress increments in the working precision)
-                cpx<double> *mv = reinterpret_cast<cpx<double> *>(a.mv_fr) +
-                                  (size_t)em * nsls * 6 * npa + qa;
-                cpx<Real> *ds = reinterpret_cast<cpx<Real> *>(a.ds_fr) +
-                                (size_t)em * 6 * npa + qa;
-                cpx<double> sd[6];
-#pragma unroll
-                for (int d = 0; d < 6; d++)
-                    sd[d] = {(double)sig[d].re, (double)sig[d].im};
-                for (int l = 0; l < nsls; l++)
+                iso_hooke<Real>(eps, dlm[0], dlm[a.npa], dsn);
+                if constexpr (ATT == ATT_SPREAD) {
 #pragma unroll
                     for (int d = 0; d < 6; d++)
-                        sd[d] = csub(sd[d], mv[(l * 6 + d) * npa]);
-#pragma unroll
-                for (int d = 0; d < 6; d++)
-                    sig[d] = {(Real)sd[d].re, (Real)sd[d].im};
-                cpx<double> dso[6], dn[6];
-#pragma unroll
-                for (int d = 0; d < 6; d++) {
-                    dso[d] = {(double)ds[d * npa].re, (double)ds[d * npa].im};
-                    dn[d] = {(double)dsn[d].re, (double)dsn[d].im};
+                        sDn[(d * 4 + qa) * EMB + eml] = dsn[d];
+                } else {
+                    att_update_fr<Real>(a, group, eml, qa, dsn, sig);
                 }
-                for (int l = 0; l < nsls; l++) {
-                    const double al = a.abg[l];
-                    const double be = a.abg[nsls + l];
-                    const double ga = a.abg[2 * nsls + l];
-#pragma unroll
-                    for (int d = 0; d < 6; d++) {
-                        cpx<double> &m = mv[(l * 6 + d) * npa];
-                        cpx<double> x = cmul(m, al);
-                        x = cfma(dso[d], be, x);
-                        m = cfma(dn[d], ga, x);
-                    }
-                }
-#pragma unroll
-                for (int d = 0; d < 6; d++) ds[d * npa] = dsn[d];
             }
         }
-        if (rtz) rot_rtz_spz6<cpx<Real>, Real>(sig, rs1, rc1, rs2, rc2);
     }
-    cpx<Real> F[3];
-    if (PRT) {
-        cpx<Real> L[3];
-        if (active && xp != nullptr) {
+    if constexpr (ATT == ATT_SPREAD) {
+        __syncthreads();
+        if (item) {
+            const cpx<Real> dsn = sDn[t];
+            const cpx<double> dn = {(double)dsn.re, (double)dsn.im};
+            cpx<double> sum = {0, 0};
+#pragma unroll
+            for (int l = 0; l < SPREAD_NS; l++) {
+                sum = cadd(sum, m[l]);
+                mv[l * CG4_ITEMS] = sls_next(a, SPREAD_NS, l, m[l], dso, dn);
+            }
+            sSum[t] = sum;
+            *ds = dsn;
+        }
+        __syncthreads();
+        const int qa = att_slot_fr(ipnt, 4);
+        if (active && qa >= 0)
+#pragma unroll
+            for (int d = 0; d < 6; d++) {
+                const cpx<double> r = sSum[(d * 4 + qa) * EMB + eml];
+                sig[d] = {(Real)((double)sig[d].re - r.re),
+                          (Real)((double)sig[d].im - r.im)};
+            }
+    }
+    if (active && MT != 0 && a.rot != nullptr && xp == nullptr)
+        rot_rtz_spz6<cpx<Real>, Real>(sig, rs1, rc1, rs2, rc2);
+    __syncthreads();                 // the displacement has been read
+    cpx<Real> L[3];
+    if (active) {
+        cpx<Real> X[3], Y[3];
+        if (PRT && xp != nullptr) {
             cpx<Real> f9[9];
             prt_und_to_sph9<cpx<Real>, Real>(sig, xp + 4 * NPEM, f9);
             if (a.rot != nullptr)
                 rot9<cpx<Real>, Real>(f9, -rs1, rc1, -rs2, rc2);
-            quad9_prep<Real>(f9, ralpha, axial_row0, q, sX[emx], sY[emx],
-                             ipnt, L);
-        } else if (active) {
-            quad6_prep<Real>(sig, ralpha, axial_row0, q, sX[emx], sY[emx],
-                             ipnt, L);
+            quad9_xyl<Real>(f9, ralpha, axial_row0, q, X, Y, L);
+        } else {
+            quad6_xyl<Real>(sig, ralpha, axial_row0, q, X, Y, L);
         }
-        __syncthreads();
-        if (active) quad6_finish<Real>(sX[emx], sY[emx], i, j, G, L, F);
-    } else {
-        quad6_point<Real>(sig, ralpha, axial_row0, q, sX[emx], sY[emx], ipnt,
-                          i, j, G, active, F);
-    }
-    if (active && alpha < nu1p) {
-        add_source(a.src, e, ipnt, alpha, F);
-        Real *dst = a.eb + ((size_t)a.elem_eb_off[e] +
-                            (size_t)ipnt * a.elem_nu1[e] + alpha) * 6;
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            dst[2 * c] = F[c].re;
-            dst[2 * c + 1] = F[c].im;
+            sX[c][ipnt][eml] = X[c];
+            sY[c][ipnt][eml] = Y[c];
         }
     }
+    __syncthreads();
+    if (!active || alpha >= nu1p) return;
+    cpx<Real> F[3];
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        cpx<Real> av = {0, 0}, bv = {0, 0};
+#pragma unroll
+        for (int k = 0; k < NPED; k++) {
+            av = cfma(sX[c][k * NPED + j][eml], Gxi[i * NPED + k], av);
+            bv = cfma(sY[c][i * NPED + k][eml], sG[0][j * NPED + k], bv);
+        }
+        F[c] = cadd(cadd(av, bv), L[c]);
+    }
+    add_source(a.src, src, ipnt, alpha, F);
+    cpx<Real> *dst = reinterpret_cast<cpx<Real> *>(a.eb) +
+                     (eb_at + alpha) * 3;
+#pragma unroll
+    for (int c = 0; c < 3; c++) dst[c] = F[c];
 }
 
 // Moment source for a unit source time function: stress = -pattern
@@ -662,24 +753,28 @@ void launch_solid_stiff_fr(hipStream_t st, const StiffArgs<Real> &a,
     // one launch per material type present (em_list grouped by type)
     for (int mt = 0; mt < 3; mt++) {
         const int eb = a.em_type_begin[mt], ee = a.em_type_begin[mt + 1];
-        const bool att = a.nsls > 0;
         if (ee <= eb) continue;
         const int grid = h.rec.nrec + (ee - eb + EMB - 1) / EMB;
+        const bool spread = a.nsls == SPREAD_NS && a.npa == 4;
 #define AXS3D_FR2(ATT_, MT_, PRT_)                                            \
     hipLaunchKernelGGL((k_solid_stiff_fr<Real, ATT_, MT_, PRT_>), dim3(grid), \
                        dim3(STIFF_BLOCK), 0, st, a, eb, ee, h)
-#define AXS3D_FR(ATT_, MT_)                                                   \
+#define AXS3D_FR(MT_)                                                         \
     do {                                                                      \
-        if (a.prt_idx != nullptr) AXS3D_FR2(ATT_, MT_, true);                 \
-        else AXS3D_FR2(ATT_, MT_, false);                                     \
+        if (a.prt_idx != nullptr) {                                           \
+            if (a.nsls > 0) AXS3D_FR2(ATT_POINT, MT_, true);                  \
+            else AXS3D_FR2(ATT_NONE, MT_, true);                              \
+        } else if (spread) {                                                  \
+            AXS3D_FR2(ATT_SPREAD, MT_, false);                                \
+        } else if (a.nsls > 0) {                                              \
+            AXS3D_FR2(ATT_POINT, MT_, false);                                 \
+        } else {                                                              \
+            AXS3D_FR2(ATT_NONE, MT_, false);                                  \
+        }                                                                     \
     } while (0)
-        if (mt == 0) {
-            if (att) AXS3D_FR(true, 0); else AXS3D_FR(false, 0);
-        } else if (mt == 1) {
-            if (att) AXS3D_FR(true, 1); else AXS3D_FR(false, 1);
-        } else {
-            if (att) AXS3D_FR(true, 2); else AXS3D_FR(false, 2);
-        }
+        if (mt == 0) AXS3D_FR(0);
+        else if (mt == 1) AXS3D_FR(1);
+        else AXS3D_FR(2);
 #undef AXS3D_FR
 #undef AXS3D_FR2
         h = StepArgs();

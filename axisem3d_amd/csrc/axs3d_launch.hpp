@@ -82,6 +82,9 @@ struct StiffArgs {
     int n_em;
     const EMItem *em_list;
     const int32_t *elem_points;
+    // [e][25] (mode offset, orders) of the element's points: one load on the
+    // way to the displacement instead of two that wait for each other
+    const uint2 *elem_modes;
     const uint8_t *elem_axial;
     const Real *elem_ops;
     const Real *elem_mat;          // 1D material, packed per element
@@ -93,6 +96,7 @@ struct StiffArgs {
     const int32_t *prt_idx = nullptr;
     const Real *prt = nullptr;
     int em_type_begin[4];          // em_list grouped by material type
+    int em_group_begin[3];         // groups of EMB of them before a type's
     const uint32_t *point_off;
     const int32_t *point_nu1;
     const double *displ;
@@ -100,14 +104,14 @@ struct StiffArgs {
     const int32_t *elem_nu1;
     Real *eb;                      // element-local forces
     const Real *gtab;
-    // attenuation of the Fourier-path (1D-material) elements, per element
-    // mode em of em_list (nsls = 0: none)
+    // attenuation of the Fourier-path (1D-material) elements, in groups of
+    // EMB element-modes (nsls = 0: none)
     int nsls;
     int npa;                       // 4 (CG4) or 25 (FULL)
     const double *abg;             // [3][nsls] alpha, beta, gamma
     const Real *att1d;             // [e][2][npa] dlambda, dmu
-    double *mv_fr;                 // [em][nsls][6][npa] complex, FP64
-    Real *ds_fr;                   // [em][6][npa] complex
+    double *mv_fr;                 // [group][nsls][6][npa][EMB] complex, FP64
+    Real *ds_fr;                   // [group][6][npa][EMB] complex
     SourceArgs<Real> src;          // the step's moment sources
 };
 

@@ -68,12 +68,16 @@ struct SourceArgs {
     int tstep = 0;
 };
 
+// The source in element e, or -1; loaded with the element's other operands.
 template <typename Real>
-__device__ __forceinline__ void add_source(const SourceArgs<Real> &s, int e,
+__device__ __forceinline__ int source_of(const SourceArgs<Real> &s, int e) {
+    return s.idx != nullptr ? s.idx[e] : -1;
+}
+
+template <typename Real>
+__device__ __forceinline__ void add_source(const SourceArgs<Real> &s, int i,
                                            int ipnt, int alpha,
                                            cpx<Real> (&F)[3]) {
-    if (s.idx == nullptr) return;
-    const int i = s.idx[e];
     if (i < 0 || alpha >= s.nu1[i]) return;
     const int ts = s.ctr != nullptr ? s.ctr[0] : s.tstep;
     if (ts < 0 || ts >= s.nstf) return;
@@ -86,13 +90,13 @@ __device__ __forceinline__ void add_source(const SourceArgs<Real> &s, int e,
 // One receiver by one block (StationSolid.cpp:59-66): in-plane weighted
 // sum, then Re sum_alpha c_alpha x_alpha e^{i alpha phi} with c_0 = 1 and
 // c_alpha = 2 (Station.hpp:53-73, eigen_tools.hpp:79-106), FP64.  The
-// orders are spread over the block's whole waves; the phase factors come
-// from a table and the points of a receiver (5 on an element edge) are
-// loaded without a branch between them, since the block is bound by the
-// latency of its loads.  Every thread of the block must call it; red holds
-// three values per wave.  The one-wave form with a
-// branch per point and sincos per order, in a launch of its own, took 7 us
-// a step at 3 orders and 87 us at 400 (32 receivers).
+// (point, order) pairs of the points with a weight (5 on an element edge)
+// are spread over the block's whole waves, so that all their loads are in
+// flight together and a thread needs few registers (it shares its kernel
+// with the elements); the phase factors come from a table.  Every thread of
+// the block must call it; red holds three values per wave.  The one-wave
+// form with a branch per point and sincos per order, in a launch of its own,
+// took 7 us a step at 3 orders and 87 us at 400 (32 receivers).
 __device__ __forceinline__ void record_receiver(const RecordArgs &a, int r,
                                                 double (*red)[3]) {
     double *out = a.out;
@@ -111,24 +115,16 @@ __device__ __forceinline__ void record_receiver(const RecordArgs &a, int r,
     const double2 *cis = a.cis + a.cis_off[r];
     double acc[3] = {0, 0, 0};
     if (t < nw * 64) {
-        for (int alpha = t; alpha < nu1; alpha += nw * 64) {
-            double xr[3] = {0, 0, 0}, xi[3] = {0, 0, 0};
-#pragma unroll 3
-            for (int p = 0; p < npt; p++) {
-                const RecPoint q = pts[p];
-                const bool in = alpha < q.nu1;
-                const double2 *u = reinterpret_cast<const double2 *>(
-                    a.displ + ((size_t)q.off + (in ? alpha : 0)) * 6);
-#pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    const double2 v = u[c];
-                    xr[c] += (in ? v.x : 0.) * q.w;
-                    xi[c] += (in ? v.y : 0.) * q.w;
-                }
-            }
+        for (int x = t; x < npt * nu1; x += nw * 64) {
+            const int p = x / nu1, alpha = x - p * nu1;
+            const RecPoint q = pts[p];
+            if (alpha >= q.nu1) continue;
+            const double2 *u = reinterpret_cast<const double2 *>(
+                a.displ + ((size_t)q.off + alpha) * 6);
             const double2 cs = cis[alpha];
 #pragma unroll
-            for (int c = 0; c < 3; c++) acc[c] += xr[c] * cs.x - xi[c] * cs.y;
+            for (int c = 0; c < 3; c++)
+                acc[c] += (u[c].x * cs.x - u[c].y * cs.y) * q.w;
         }
 #pragma unroll
         for (int c = 0; c < 3; c++) {
