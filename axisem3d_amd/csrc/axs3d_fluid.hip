@@ -16,6 +16,14 @@
 // order, GLL point), ten element-modes per 256-thread block, LDS tiles
 // for the two 5x5 contractions, element-local forces [e][ipnt][alpha]
 // gathered by the point kernel in ascending element order.
+//
+// The potential is contracted in FP64 in both precision modes: it is large
+// and smooth next to its differences between GLL points, and what an FP32
+// potential loses there enters the normal force on the solid boundary whole.
+// (Error of the displacement there against an FP64 run after 400 steps of 24
+// x 18 elements, the largest over its root mean square, in six wavefields:
+// 0.8 to 2.2e-4 with an FP32 potential, 0.8 to 2.1e-5 now.  The kernel waits
+// on memory either way: 54.7 us a step before, 55.0 now.)
 #include "axs3d_common.hpp"
 #include "axs3d_element.hpp"
 #include "axs3d_launch.hpp"
@@ -25,7 +33,7 @@ namespace axs3d {
 template <typename Real>
 __global__ __launch_bounds__(STIFF_BLOCK) void k_fluid_stiff_fr(
     FluidArgs<Real> a) {
-    __shared__ cpx<Real> sP[EMB][NPEM];
+    __shared__ cpx<double> sP[EMB][NPEM];
     __shared__ cpx<Real> sX[EMB][NPEM];
     __shared__ cpx<Real> sY[EMB][NPEM];
     __shared__ Real sG[2][NPEM];
@@ -42,7 +50,7 @@ __global__ __launch_bounds__(STIFF_BLOCK) void k_fluid_stiff_fr(
     int e = 0, alpha = 0, nu1p = 0;
     uint32_t off = 0;
     bool axial = false;
-    cpx<Real> p = {0, 0};
+    cpx<double> p = {0, 0};
     if (active) {
         const EMItem it = a.em_list[em];
         e = it.elem;
@@ -53,7 +61,7 @@ __global__ __launch_bounds__(STIFF_BLOCK) void k_fluid_stiff_fr(
         axial = a.elem_axial[e] != 0;
         if (alpha < nu1p) {
             const double *src = a.chi + (size_t)(off + alpha) * 2;
-            p = {(Real)src[0], (Real)src[1]};
+            p = {src[0], src[1]};
         }
         sP[eml][ipnt] = p;
     }
@@ -69,16 +77,19 @@ __global__ __launch_bounds__(STIFF_BLOCK) void k_fluid_stiff_fr(
         load_point_ops(a.elem_ops, e, ipnt, g, q);
         // computeGrad3: dp/ds, dp/dz from the two contractions; i alpha p
         // / s, on the axis row its L'Hospital limit i alpha dp/ds
-        cpx<Real> x = {0, 0}, y = {0, 0};
+        cpx<double> xd = {0, 0}, yd = {0, 0};
 #pragma unroll
         for (int k = 0; k < NPED; k++) {
-            x = cfma(sP[eml][k * NPED + j], G.gxi_col[k], x);
-            y = cfma(sP[eml][i * NPED + k], G.g_col[k], y);
+            xd = cfma(sP[eml][k * NPED + j], (double)G.gxi_col[k], xd);
+            yd = cfma(sP[eml][i * NPED + k], (double)G.g_col[k], yd);
         }
+        const cpx<Real> x = {(Real)xd.re, (Real)xd.im};
+        const cpx<Real> y = {(Real)yd.re, (Real)yd.im};
         const cpx<Real> dpds = cadd(cmul(x, g.dzdeta), cmul(y, g.dzdxii));
         const cpx<Real> dpdz = cadd(cmul(x, g.dsdeta), cmul(y, g.dsdxii));
+        const cpx<Real> pr = {(Real)p.re, (Real)p.im};
         const cpx<Real> ps = axial_row0 ? ialpha(ralpha, dpds)
-                                        : cmul(ialpha(ralpha, p), g.invs);
+                                        : cmul(ialpha(ralpha, pr), g.invs);
         // Acoustic: stress = K strain
         const Real K = a.elem_k[(size_t)e * NPEM + ipnt];
         const cpx<Real> q0 = cmul(dpds, K), q1 = cmul(ps, K);
