@@ -19,11 +19,11 @@
 //  A. gradient: one thread per (element-mode, GLL point) as on the
 //     Fourier path, strain (rotated to RTZ where the medium works there)
 //     to the scratch.
-//  B. stress: one GLL point per block of three waves.  Each wave packs
-//     one of the point's three strain pairs as x + i y into its own LDS
-//     buffer and transforms it in place (axs3d_fft.hpp: passes of radix 2
-//     to 16 with compile-time DFTs and a table of every twiddle power;
-//     plans, tables and the digit reversal per Nr, in LDS sized per
+//  B. stress: one to five GLL points per block of three waves.  Each wave
+//     packs one of the points' three strain pairs as x + i y into its own
+//     LDS buffers and transforms them in place (axs3d_fft.hpp: passes of
+//     radix 2 to 16 with compile-time DFTs and a table of every twiddle
+//     power; plans, tables and the digit reversal per Nr, in LDS sized per
 //     launch).  The three waves then form the stress slice by slice from
 //     all six strains (3D moduli, SLS memory variables) and transform back
 //     into the scratch.  One FFT call site for both directions keeps the
@@ -59,53 +59,74 @@ __device__ __forceinline__ void fft_load_tables(
 
 constexpr int CD_EMB = 16;             // gradient/quadrature: element-modes
 constexpr int CD_EMB_THREADS = CD_EMB * NPEM;  // per block
-constexpr int CD_PW = 3;               // stress kernel: waves per point
+constexpr int CD_PW = 3;               // stress kernel: waves (strain pairs)
 constexpr int CD_PT = CD_PW * 64;      // threads per stress block
+
+// Two consecutive orders of a scratch row, one 16-byte access in FP32 (rows
+// start on 128-byte lines and hold a multiple of 16 orders).
+template <typename Real>
+struct alignas(16) cpx2 {
+    cpx<Real> v[2];
+};
 
 // C2R input of the strain pair (X, Y) = rows (2q, 2q+1) of a point:
 // buf[k] = Xfull[k] + i Yfull[k], with Xfull the Hermitian extension under
 // SolverFFTW's C2R rules (Nyquist doubled, Im of mean and Nyquist
-// ignored).
+// ignored).  Each entry is read once, two orders a lane, and written to its
+// own place and its mirror's: the kernel is bound by the memory accesses it
+// has in flight, so few wide ones.
 template <typename Real>
 __device__ __forceinline__ void pack_pair(cpx<Real> *buf,
                                           const cpx<Real> *__restrict__ X,
                                           const cpx<Real> *__restrict__ Y,
                                           int nr, int nu1, bool even,
                                           int lane) {
-    // branch-free: slice k takes row entry kk = k (k < nu1) or nr - k
-    // (conjugated); the mean and an even Nr's Nyquist entry are real,
-    // the latter doubled.  (Reading each entry once and writing its mirror
-    // too measured 2% slower on the regional workload.)
     const int nyq = even ? nu1 - 1 : -1;
-#pragma unroll 4
-    for (int k = lane; k < nr; k += 64) {
-        const bool lo = k < nu1;
-        const int kk = lo ? k : nr - k;
-        const cpx<Real> x = X[kk], y = Y[kk];
-        const bool real_only = k == 0 || k == nyq;
-        const Real sc = k == nyq ? (Real)2 : (Real)1;
-        const Real sim = real_only ? (Real)0 : (lo ? (Real)1 : (Real)-1);
-        // xf = (sc x.re, sim x.im), yf likewise; buf = xf + i yf
-        buf[pad(k)] = {sc * x.re - sim * y.im, sim * x.im + sc * y.re};
+#pragma unroll 2
+    for (int k0 = 2 * lane; k0 < nu1; k0 += 128) {
+        const cpx2<Real> x2 = *reinterpret_cast<const cpx2<Real> *>(X + k0);
+        const cpx2<Real> y2 = *reinterpret_cast<const cpx2<Real> *>(Y + k0);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int k = k0 + i;
+            if (k >= nu1) break;
+            const cpx<Real> x = x2.v[i], y = y2.v[i];
+            if (k == 0) {
+                buf[0] = {x.re, y.re};
+            } else if (k == nyq) {
+                buf[pad(k)] = {(Real)2 * x.re, (Real)2 * y.re};
+            } else {
+                buf[pad(k)] = {x.re - y.im, x.im + y.re};
+                buf[pad(nr - k)] = {x.re + y.im, y.re - x.im};
+            }
+        }
     }
     wave_sync();
 }
 
 // R2C output: X_k = (Z_k + conj Z_{N-k}) / 2N, Y_k = (Z_k - conj Z_{N-k})
-// / 2iN, Nyquist row halved; written to rows (2q, 2q+1).
+// / 2iN, Nyquist row halved; written to rows (2q, 2q+1), two orders a lane
+// (the one past the last falls on the row's padding).
 template <typename Real>
 __device__ __forceinline__ void unpack_pair(const cpx<Real> *buf,
                                             cpx<Real> *__restrict__ X,
                                             cpx<Real> *__restrict__ Y, int nr,
                                             int nu1, bool even, int lane) {
     const Real h0 = (Real)0.5 / (Real)nr;
-#pragma unroll 4
-    for (int k = lane; k < nu1; k += 64) {
-        const cpx<Real> zk = buf[pad(k)];
-        const cpx<Real> zn = buf[pad(k == 0 ? 0 : nr - k)];
-        const Real h = (even && k == nu1 - 1) ? h0 * (Real)0.5 : h0;
-        X[k] = {(zk.re + zn.re) * h, (zk.im - zn.im) * h};
-        Y[k] = {(zk.im + zn.im) * h, (zn.re - zk.re) * h};
+#pragma unroll 2
+    for (int k0 = 2 * lane; k0 < nu1; k0 += 128) {
+        cpx2<Real> x2, y2;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int k = min(k0 + i, nu1 - 1);
+            const cpx<Real> zk = buf[pad(k)];
+            const cpx<Real> zn = buf[pad(k == 0 ? 0 : nr - k)];
+            const Real h = (even && k == nu1 - 1) ? h0 * (Real)0.5 : h0;
+            x2.v[i] = {(zk.re + zn.re) * h, (zk.im - zn.im) * h};
+            y2.v[i] = {(zk.im + zn.im) * h, (zn.re - zk.re) * h};
+        }
+        *reinterpret_cast<cpx2<Real> *>(X + k0) = x2;
+        *reinterpret_cast<cpx2<Real> *>(Y + k0) = y2;
     }
     wave_sync();
 }
@@ -274,123 +295,107 @@ __global__ __launch_bounds__(CD_EMB_THREADS) void k_cd_quad(CardArgs<Real> a,
     }
 }
 
-// B: stress of one GLL point of one element per block of three waves.
-// Wave q packs strain pair q (rows 2q, 2q+1: (ss, pp), (zz, pz), (sz, sp))
-// as x + i y into its own LDS buffer and inverse-transforms it; after a
-// block barrier the three waves form the stress slice by slice from all
-// six strains (Isotropic::strainToStress, Isotropic.hpp:155-172;
-// TransverselyIsotropic::strainToStress, TransverselyIsotropic.hpp:161-
-// 180; Anisotropic::strainToStress, Anisotropic.hpp:203-274) with the SLS
-// memory update, write it back in place, and after a second barrier each
-// wave forward-transforms its pair and unpacks it into the scratch rows.
-// Between the transforms slice k sits at buffer position pos[k] (the
-// digit reversal of the in-place FFT); the slice loop runs over slices so
-// its global accesses stay consecutive.
-template <typename Real, int NS, int MT>
-__device__ __forceinline__ void cd_stress_slices(const CardArgs<Real> &a,
-                                                 cpx<Real> *b0, cpx<Real> *b1,
-                                                 cpx<Real> *b2,
-                                                 const uint16_t *pos,
-                                                 const SliceMat<Real> &M,
-                                                 const double *abg, bool att,
-                                                 int nr, int t) {
-    // two slices in flight without attenuation; with it the memory
-    // variables of one slice already fill the registers
-    constexpr int UNR = NS != 0 ? 1 : 2;
-#pragma unroll UNR
-    for (int k = t; k < nr; k += CD_PT) {
-        const int p = pad(pos[k]);
-        const cpx<Real> z01 = b0[p], z23 = b1[p], z45 = b2[p];
-        const Real e[6] = {z01.re, z01.im, z23.re, z23.im, z45.re, z45.im};
-        Real sv[6];
-        slice_stress<Real, NS, MT>(e, M, k, att, a.nsls, abg, sv);
-        b0[p] = {sv[0], sv[1]};
-        b1[p] = {sv[2], sv[3]};
-        b2[p] = {sv[4], sv[5]};
-    }
-}
-
+// B: stress of a few GLL points of one element per block of three waves.
+// Wave q packs strain pair q (rows 2q, 2q+1: (ss, pp), (zz, pz), (sz, sp)) of
+// each point as x + i y into its own LDS buffers and inverse-transforms them
+// together; after a block barrier the three waves form the stress slice by
+// slice from all six strains with the SLS memory update (slice_stress),
+// write it back in place, and after a second barrier each wave
+// forward-transforms its pairs and unpacks them into the scratch rows.
+// Between the transforms slice k sits at buffer position pos[k] (the digit
+// reversal of the in-place FFT); the slice loop runs over slices so its
+// global accesses stay consecutive.
 // B kernel.  MT = material type of the batch's elements (0 isotropic, 1
 // TI, 2 anisotropic); NS = number of SLS (0: no attenuation, -1: taken
-// from the arguments).  25 blocks per element of the batch list3d[w0 ..),
-// one per GLL point.
+// from the arguments).  One block per item of the batch's work list.
 template <typename Real, int NS, int MT>
 __global__ __launch_bounds__(CD_PT, CardOcc<Real>::value) void k_cd_stress(
-    CardArgs<Real> a, int w0) {
+    CardArgs<Real> a, int work0) {
     __shared__ double abg[3 * CD_MAX_SLS];    // SLS alpha, beta, gamma
     const int t = threadIdx.x;
     const int lane = t & 63;
     // the wave index is uniform across the wave: keep it (and all that is
     // derived from it) in scalar registers
     const int q = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int w = w0 + (int)blockIdx.x / NPEM;
-    const int pp = (int)blockIdx.x % NPEM;
-    const int e = a.list3d[w];
+    const StressItem it = a.work[work0 + (int)blockIdx.x];
+    const int pp = it.point, np = it.count;
+    const int e = a.list3d[it.w];
     const int nu1 = a.s.elem_nu1[e];
     const int nr = a.elem_nr[e];
     const uint32_t *plan = a.plan + (size_t)nr * CARD_PLAN_W;
     FftLds<Real> L;
-    L.carve(fft_lds, nr, CD_PW);
+    L.carve(fft_lds, nr, CD_PW * np);
     fft_load_tables<Real>(L, a.twiddle, a.tw_off, a.slice_pos, a.pos_off,
                           plan, nr, t, CD_PT);
     if (NS != 0 && t < 3 * a.nsls) {
         const int c = t / a.nsls, l = t - c * a.nsls;
         abg[c * CD_MAX_SLS + l] = a.abg[t];
     }
-    __syncthreads();
     const bool even = (nr & 1) == 0;
-    const size_t rs = (size_t)NPEM * scr_row(nu1);
+    const int row = scr_row(nu1);
+    const size_t rs = (size_t)NPEM * row;
     cpx<Real> *r0 = reinterpret_cast<cpx<Real> *>(a.scratch) + a.scr_off[e] +
-                    (size_t)pp * scr_row(nu1);
-    cpx<Real> *b = L.buf(q);
-    pack_pair<Real>(b, r0 + 2 * q * rs, r0 + (2 * q + 1) * rs, nr, nu1, even,
-                    lane);
+                    (size_t)pp * row + 2 * q * rs;
+    // buffer of point p of this wave's pair: b + p stride
+    const int stride = L.buf_bytes / (int)sizeof(cpx<Real>);
+    cpx<Real> *b = L.buf(q * np);
+    for (int p = 0; p < np; p++)
+        pack_pair<Real>(b + p * stride, r0 + (size_t)p * row,
+                        r0 + rs + (size_t)p * row, nr, nu1, even, lane);
+    __syncthreads();
     // both transforms from one call site (the inverse, the stress, then
     // the forward transform), which halves the FFT's code
 #pragma unroll 1
     for (int pass = 0; pass < 2; pass++) {
-        wave_fft<Real>(b, plan, pass == 0, L.tw, lane);
+        wave_fft<Real>(b, stride, np, plan, pass == 0, L.tw, lane);
         if (pass == 1) break;
         __syncthreads();
-    {
         SliceMat<Real> M;
-        M.ps = (size_t)NPEM * nr;
-        M.par = a.prop3d + a.prop_off[e] + (size_t)pp * nr;
-        const int ip4 = NS != 0 ? att_slot(pp, a.npa) : -1;
-        const bool att = NS != 0 && ip4 >= 0;
-        if (NS != 0 && att) {
-            const int64_t sl0 = a.slice_off[e];
-            const int npa = a.npa;
-            M.cs = (size_t)npa * nr;
-            M.dl = a.att3d + (size_t)sl0 * 2 * npa + (size_t)ip4 * nr;
-            M.dm = M.dl + M.cs;
-            M.mv = a.memvar + (size_t)sl0 * a.nsls * 6 * npa +
-                   (size_t)ip4 * nr;
-            M.ds = a.dstress + (size_t)sl0 * 6 * npa + (size_t)ip4 * nr;
+        M.element(a.prop3d + a.prop_off[e], a.att3d, a.memvar, a.dstress,
+                  a.slice_off[e], nr, a.npa, a.nsls);
+        for (int p = 0; p < np; p++) {
+            const int ip4 = NS != 0 ? att_slot(pp + p, a.npa) : -1;
+            cpx<Real> *b0 = L.buf(p), *b1 = L.buf(np + p);
+            cpx<Real> *b2 = L.buf(2 * np + p);
+            // two slices in flight without attenuation; with it the memory
+            // variables of one slice already fill the registers
+            constexpr int UNR = NS != 0 ? 1 : 2;
+#pragma unroll UNR
+            for (int k = t; k < nr; k += CD_PT) {
+                const int x = pad(L.pos[k]);
+                const cpx<Real> z01 = b0[x], z23 = b1[x], z45 = b2[x];
+                const Real ev[6] = {z01.re, z01.im, z23.re,
+                                    z23.im, z45.re, z45.im};
+                Real sv[6];
+                slice_stress<Real, NS, MT>(ev, M, (pp + p) * nr + k,
+                                           ip4 < 0 ? -1 : ip4 * nr + k,
+                                           a.nsls, abg, sv);
+                b0[x] = {sv[0], sv[1]};
+                b1[x] = {sv[2], sv[3]};
+                b2[x] = {sv[4], sv[5]};
+            }
         }
-        cd_stress_slices<Real, NS, MT>(a, L.buf(0), L.buf(1), L.buf(2),
-                                        L.pos, M, abg, att, nr, t);
-    }
         __syncthreads();
     }
-    unpack_pair<Real>(b, r0 + 2 * q * rs, r0 + (2 * q + 1) * rs, nr, nu1,
-                      even, lane);
+    for (int p = 0; p < np; p++)
+        unpack_pair<Real>(b + p * stride, r0 + (size_t)p * row,
+                          r0 + rs + (size_t)p * row, nr, nu1, even, lane);
 }
 
 template <typename Real, int MT>
-static void launch_stress_mt(hipStream_t st, const CardArgs<Real> &a, int w0,
-                             int n, int nr_max) {
-    const dim3 grid(n * NPEM), block(CD_PT);
-    const size_t lds = fft_lds_bytes<Real>(nr_max, CD_PW);
+static void launch_stress_mt(hipStream_t st, const CardArgs<Real> &a,
+                             const CardBatch &bt) {
+    const dim3 grid(bt.work_end - bt.work_begin), block(CD_PT);
+    const size_t lds = bt.stress_lds;
     if (a.nsls == 0)
         hipLaunchKernelGGL((k_cd_stress<Real, 0, MT>), grid, block, lds, st,
-                           a, w0);
+                           a, bt.work_begin);
     else if (a.nsls == 5)
         hipLaunchKernelGGL((k_cd_stress<Real, 5, MT>), grid, block, lds, st,
-                           a, w0);
+                           a, bt.work_begin);
     else
         hipLaunchKernelGGL((k_cd_stress<Real, -1, MT>), grid, block, lds, st,
-                           a, w0);
+                           a, bt.work_begin);
 }
 
 // The three launches of a batch (gradient, stress, quadrature); batches
@@ -419,15 +424,13 @@ void launch_cd_grad(hipStream_t st, const CardArgs<Real> &a,
 template <typename Real>
 void launch_cd_stress(hipStream_t st, const CardArgs<Real> &a,
                       const CardBatch &bt) {
-    const int n = bt.end - bt.begin;
-    if (n <= 0) return;
-    switch (bt.mtype) {
-        case 0: launch_stress_mt<Real, 0>(st, a, bt.begin, n, bt.nr_max); break;
-        case 1: launch_stress_mt<Real, 1>(st, a, bt.begin, n, bt.nr_max); break;
-        default:
-            launch_stress_mt<Real, 2>(st, a, bt.begin, n, bt.nr_max);
-            break;
-    }
+    if (bt.work_end <= bt.work_begin) return;
+    if (bt.mtype == 0)
+        launch_stress_mt<Real, 0>(st, a, bt);
+    else if (bt.mtype == 1)
+        launch_stress_mt<Real, 1>(st, a, bt);
+    else
+        launch_stress_mt<Real, 2>(st, a, bt);
 }
 
 template <typename Real>
@@ -1327,7 +1330,8 @@ void launch_cd_sens(hipStream_t st, const CardArgs<Real> &a, const Real *scrb,
 template <typename Real>
 int card_blocks_per_cu(bool att, int nr_max) {
     int n = 0;
-    const size_t lds = fft_lds_bytes<Real>(nr_max, CD_PW);
+    const size_t lds =
+        stress_lds_bytes<Real>(nr_max, stress_points<Real>(nr_max));
     const hipError_t r =
         att ? hipOccupancyMaxActiveBlocksPerMultiprocessor(
                   &n, k_cd_stress<Real, 5, 0>, CD_PT, lds)

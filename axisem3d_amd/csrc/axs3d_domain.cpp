@@ -1791,6 +1791,7 @@ public:
         c.plan = dPlan.as<uint32_t>();
         c.slice_pos = dPosTab.as<uint16_t>();
         c.pos_off = dPosOff.as<int64_t>();
+        c.work = dStressWork.as<StressItem>();
         c.scratch = dCardScratch.as<Real>();
         c.scr_off = dScrOff.as<uint32_t>();
         c.nsls = mNsls;
@@ -2703,6 +2704,40 @@ private:
                 scrMax = std::max(scrMax, used);
             }
         }
+        if (all) return;
+        for (CardBatch &b : batches) {
+            b.work_begin = hWorkOff[b.begin];
+            b.work_end = hWorkOff[b.end - 1] + workCount(b.end - 1);
+            for (int w = b.begin; w < b.end; w++) {
+                const int nr = hElemNr[hList3D[w]];
+                b.stress_lds = std::max(
+                    b.stress_lds,
+                    stress_lds_bytes<Real>(nr, stress_points<Real>(nr)));
+            }
+        }
+    }
+
+    // The stress kernel's blocks of the elements that take the three-kernel
+    // form, in list order.
+    int workCount(int w) const {
+        const int n = stress_points<Real>(hElemNr[hList3D[w]]);
+        return (NPEM + n - 1) / n;
+    }
+    void planStressWork() {
+        std::vector<StressItem> work;
+        hWorkOff.assign(mNum3D, 0);
+        for (int mt = 0; mt < 3; mt++)
+            for (int w = mTypeBegin3D[mt]; w < mFusedBegin[mt]; w++) {
+                const int n = stress_points<Real>(hElemNr[hList3D[w]]);
+                hWorkOff[w] = (int)work.size();
+                for (int p = 0; p < NPEM; p += n)
+                    work.push_back({w, (int16_t)p,
+                                    (int16_t)std::min(n, NPEM - p)});
+            }
+        dStressWork.alloc(work.size() * sizeof(StressItem));
+        if (!work.empty())
+            dStressWork.upload(work.data(), work.size() * sizeof(StressItem),
+                               mStream);
     }
 
     // Batches of the 3D fluid elements ([3][25][nu1] rows each) for a
@@ -3169,6 +3204,7 @@ private:
                 mScratchFixed = true;
             }
             planFused();
+            planStressWork();
             buildCardBatches(budget);
             if (mNsls > 0) {
                 const int npa = mAttCG4 ? 4 : NPEM;

@@ -358,6 +358,9 @@ protected:
     std::vector<CardBatch> mAdjBatches;
     size_t mAdjScrMax = 0;
     DeviceBuffer dAdjScrOff, dAdjEM3D, dAdjScrA;
+    // stress blocks (StressItem), and the first one of each list3d position
+    DeviceBuffer dStressWork;
+    std::vector<int32_t> hWorkOff;
     int mCardOcc = CARD_OCC;            // stress kernel waves per SIMD
     double mCardTuneMs = 0.;            // one cardinal pass at finalize
     double mScratchMiB = 0.;            // cardinal scratch budget in use

@@ -527,12 +527,13 @@ inline double fft_butterfly_cost(int R) {
 
 // Fixed cost of a pass in the same units (loop set-up, the wave's
 // barrier, the LDS latency that a pass of few butterflies cannot hide).
-constexpr double kFftPassCost = 40.0;
+constexpr double kFftPassCost = 20.0;
 
 // Pass radices of Nr (prime factors <= 13), each <= max_radix (or a
 // prime), minimising
-// the modelled cost sum_p ceil((Nr / R_p) / 64) cost(R_p) (a pass has Nr /
-// R_p butterflies whatever its place); descending order.  Empty if Nr has
+// the modelled cost sum_p (Nr / R_p) / 64 cost(R_p) (a pass has Nr / R_p
+// butterflies whatever its place, which a wave counts together with those
+// of its other series); descending order.  Empty if Nr has
 // a prime factor above 13.
 inline std::vector<int> fft_choose_radices(int nr, int max_radix) {
     std::vector<int> divs;
@@ -552,7 +553,7 @@ inline std::vector<int> fft_choose_radices(int nr, int max_radix) {
             if (d % R != 0 || best[d / R] >= 1e299) continue;
             const int nb = nr / R;
             const double c = best[d / R] + kFftPassCost +
-                             (double)((nb + 63) / 64) * fft_butterfly_cost(R);
+                             (double)nb / 64.0 * fft_butterfly_cost(R);
             if (c < best[d]) {
                 best[d] = c;
                 choice[d] = R;

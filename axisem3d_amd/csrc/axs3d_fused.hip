@@ -182,29 +182,18 @@ __global__ __launch_bounds__(FusedBlock<Real>::value) void k_cd_fused(
         __syncthreads();
         if (pass == 1) break;
         SliceMat<Real> M;
-        M.ps = (size_t)NPEM * nr;
-        const Real *par = a.prop3d + a.prop_off[e];
-        const int npa = a.npa;
-        const int64_t sl0 = a.slice_off[e];
-        M.cs = (size_t)npa * nr;
+        M.element(a.prop3d + a.prop_off[e], a.att3d, a.memvar, a.dstress,
+                  a.slice_off[e], nr, a.npa, a.nsls);
         for (int x = t; x < NPEM * nr; x += T) {
             const int pt = div22(x, mgr), k = x - pt * nr;
-            const int ip4 = NS != 0 ? att_slot(pt, npa) : -1;
-            const bool att = NS != 0 && ip4 >= 0;
-            M.par = par + pt * nr;
-            if (att) {
-                const size_t at = (size_t)ip4 * nr;
-                M.dl = a.att3d + (size_t)sl0 * 2 * npa + at;
-                M.dm = M.dl + M.cs;
-                M.mv = a.memvar + (size_t)sl0 * a.nsls * 6 * npa + at;
-                M.ds = a.dstress + (size_t)sl0 * 6 * npa + at;
-            }
+            const int ip4 = NS != 0 ? att_slot(pt, a.npa) : -1;
+            const int att = ip4 < 0 ? -1 : ip4 * nr + k;
             cpx<Real> *b0 = S + 3 * pt * stride + pad(pos[k]);
             cpx<Real> *b1 = b0 + stride, *b2 = b1 + stride;
             const cpx<Real> z0 = *b0, z1 = *b1, z2 = *b2;
             const Real ev[6] = {z0.re, z0.im, z1.re, z1.im, z2.re, z2.im};
             Real sv[6];
-            slice_stress<Real, NS, MT>(ev, M, k, att, a.nsls, abg, sv);
+            slice_stress<Real, NS, MT>(ev, M, x, att, a.nsls, abg, sv);
             *b0 = {sv[0], sv[1]};
             *b1 = {sv[2], sv[3]};
             *b2 = {sv[4], sv[5]};

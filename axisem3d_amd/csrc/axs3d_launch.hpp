@@ -119,14 +119,40 @@ struct StiffArgs {
 // of Nr per wave in LDS, sized per launch).
 constexpr int CARD_NR_CAP = FFT_NR_CAP;
 // Minimum waves per SIMD the stress kernel's register allocation allows:
-// five in FP32; in FP64 the LDS of an Nr of several hundred holds at most
-// two or three blocks per CU anyway, and three waves leave the radix-16
-// passes their registers.
-constexpr int CARD_OCC = 5;
+// four in FP32 (five spill the two components' memory variables that are in
+// flight: 2227 against 1792 us a step of 2114 elements); in FP64 the LDS
+// holds fewer blocks anyway, and three waves leave the radix-16 passes their
+// registers.
+constexpr int CARD_OCC = 4;
 template <typename Real>
 struct CardOcc {
     static constexpr int value = sizeof(Real) == 4 ? CARD_OCC : 3;
 };
+// Work item of the stress kernel: position w of list3d, its first GLL point
+// and the number of points (the block's series: that many per strain pair).
+struct StressItem {
+    int32_t w;
+    int16_t point, count;
+};
+// LDS of a stress block of `count` points of Nr nr.
+template <typename Real>
+inline size_t stress_lds_bytes(int nr, int count) {
+    return fft_lds_bytes<Real>(nr, 3 * count);
+}
+// Points per block of an element of Nr nr.  A pass over one series of Nr has
+// Nr / R butterflies, 25 of radix 16 at Nr = 400, for 64 lanes; a wave that
+// owns the same strain pair of several points counts their butterflies
+// together.  As many (up to five, which divide the 25) as leave five blocks'
+// LDS per CU (fifteen waves of the sixteen the registers allow; in FP64 four
+// blocks, twelve waves).
+template <typename Real>
+inline int stress_points(int nr) {
+    const size_t budget = sizeof(Real) == 4 ? (size_t)32 << 10
+                                            : (size_t)40 << 10;
+    int n = 1;
+    while (n < 5 && stress_lds_bytes<Real>(nr, n + 1) <= budget) n++;
+    return n;
+}
 // FFT plan words per Nr (see axs3d_fft.hpp).
 constexpr int CARD_PLAN_W = FFT_PLAN_W;
 
@@ -150,6 +176,7 @@ struct CardArgs {
     const uint32_t *plan;          // [Nr][CARD_PLAN_W] FFT passes
     const uint16_t *slice_pos;     // buffer position of each slice after
     const int64_t *pos_off;        // the inverse transform, per Nr
+    const StressItem *work;        // the stress kernel's blocks
     Real *scratch;                 // batch scratch, complex
     const uint32_t *scr_off;       // [element] its part of its batch's
                                    // scratch ([150][nu1] complex), in
@@ -362,6 +389,8 @@ struct CardBatch {
     int mtype, begin, end;
     int em_begin, em_end;          // its element-modes in the 3D list
     int nr_max = 0;                // largest Nr of its elements
+    int work_begin = 0, work_end = 0;  // its stress blocks
+    size_t stress_lds = 0;         // the largest one's LDS
 };
 // Default scratch of one batch (bytes).
 constexpr size_t CARD_SCRATCH_BYTES = (size_t)4 << 30;

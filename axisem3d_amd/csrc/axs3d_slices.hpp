@@ -14,82 +14,118 @@ __device__ __forceinline__ int att_slot(int p, int npa) {
     return p == 6 ? 0 : p == 8 ? 1 : p == 16 ? 2 : p == 18 ? 3 : -1;
 }
 
-// Per-slice operands of one GLL point: pointers at slice 0 of element e;
-// parameter c of slice k sits at par[c * ps + k], attenuation component
-// d of slice k at [d * cs + k].
+// Per-slice operands of an element: its base addresses, the same for the
+// whole block (they stay in scalar registers), and the lane's place in a
+// component's row: parameter c of slice k at point p sits at par[c * ps + p
+// Nr + k], attenuation component d at slot q at [d * cs + q Nr + k].
 template <typename Real>
 struct SliceMat {
-    const Real *par;             // this point's parameter 0
-    size_t ps;                   // parameter step, 25 Nr
-    const Real *dl, *dm;         // moduli of its attenuation slot
-    double *mv;                  // memory variables [nsls][6] of the slot
-    Real *ds;                    // memory stress [6] of the slot
-    size_t cs;                   // component step of mv, ds: npa Nr
-    __device__ Real p(int c, int k) const { return par[c * ps + k]; }
+    const Real *par;
+    int ps;                      // parameter step, 25 Nr
+    const Real *dl, *dm;         // attenuation moduli
+    double *mv;                  // memory variables, [nsls][6] rows
+    Real *ds;                    // memory stress, [6] rows
+    int cs;                      // component step of these, npa Nr
+    __device__ void element(const Real *prop, const Real *att3d,
+                            double *memvar, Real *dstress, int64_t slice0,
+                            int nr, int npa, int nsls) {
+        par = prop;
+        ps = NPEM * nr;
+        cs = npa * nr;
+        dl = att3d + slice0 * 2 * npa;
+        dm = dl + cs;
+        mv = memvar + slice0 * nsls * 6 * npa;
+        ds = dstress + slice0 * 6 * npa;
+    }
+    __device__ Real p(int c, int at) const { return par[c * ps + at]; }
 };
 
-// SLS memory of stress component d at slice k (Attenuation::updateMem*,
-// AttenuationFull/CG4::apply): sigma -= sum_l m_l; m_l = alpha_l m_l +
-// beta_l ds_old + gamma_l ds_new; ds_old = ds_new, where dsn = ds_new is
-// the (dlambda, dmu) isotropic stress of the strain in the frame the
-// stress is formed in.  mvk, dsk point at slice k of the slot's memory
-// variables and memory stress; abg = alpha, beta, gamma in the working
-// precision (LDS, [3][CD_MAX_SLS]).  The solids go four at a time so
-// their loads are in flight together.
+// SLS memory of the six stress components at slice k (Attenuation::
+// updateMem*, AttenuationFull/CG4::apply): sigma -= sum_l m_l; m_l = alpha_l
+// m_l + beta_l ds_old + gamma_l ds_new; ds_old = ds_new, where dsn = ds_new
+// is the (dlambda, dmu) isotropic stress of the strain in the frame the
+// stress is formed in.  at = the slot's place of slice k; abg = alpha, beta,
+// gamma (LDS, [3][CD_MAX_SLS]).  The memory variables and the recursion are
+// FP64 in both precision modes (the stress increments stay in the working
+// precision).
+// The update is bound by the latency of its loads, which no store may pass:
+// with a fixed count of solids two components' are issued together, then
+// their stores.
 constexpr int CD_MAX_SLS = 16;
-// The memory variables and the recursion are FP64 in both precision
-// modes (the stress increments stay in the working precision).
 template <typename Real, int NS>
-__device__ __forceinline__ void att_update(double *mvk, Real *dsk, int cs,
+__device__ __forceinline__ void att_update(const SliceMat<Real> &M, int at,
                                            int nsls, const double *abg,
-                                           int d, Real dsn, Real &sig) {
-    const int od = d * cs;
-    const int ls = 6 * cs;
-    const double dso = (double)dsk[od];
-    const double dn = (double)dsn;
-    double sd = (double)sig;
+                                           const Real (&dsn)[6],
+                                           Real (&sv)[6]) {
+    const int cs = M.cs, ls = 6 * cs;
+    double *mv = M.mv;
+    Real *ds = M.ds;
+    auto next = [&](double m, int l, double dso, double dn) {
+        return abg[l] * m + abg[CD_MAX_SLS + l] * dso +
+               abg[2 * CD_MAX_SLS + l] * dn;
+    };
     if constexpr (NS > 0) {
-        // the common five-solid case (or any fixed count): unrolled
-        double m[NS];
+        constexpr int DB = 2;
 #pragma unroll
-        for (int l = 0; l < NS; l++) m[l] = mvk[od + l * ls];
+        for (int d0 = 0; d0 < 6; d0 += DB) {
+            double m[DB][NS], dso[DB];
 #pragma unroll
-        for (int l = 0; l < NS; l++) sd -= m[l];
+            for (int d = 0; d < DB; d++) {
+                dso[d] = (double)ds[(d0 + d) * cs + at];
 #pragma unroll
-        for (int l = 0; l < NS; l++)
-            mvk[od + l * ls] = abg[l] * m[l] + abg[CD_MAX_SLS + l] * dso +
-                               abg[2 * CD_MAX_SLS + l] * dn;
-    } else {
-        for (int l0 = 0; l0 < nsls; l0 += 4) {
-            double m[4];
+                for (int l = 0; l < NS; l++)
+                    m[d][l] = mv[((d0 + d) * cs + l * ls) + at];
+            }
 #pragma unroll
-            for (int q = 0; q < 4; q++)
-                m[q] = l0 + q < nsls ? mvk[od + (l0 + q) * ls] : 0.;
+            for (int d = 0; d < DB; d++) {
+                const double dn = (double)dsn[d0 + d];
+                double sd = (double)sv[d0 + d];
 #pragma unroll
-            for (int q = 0; q < 4; q++) sd -= m[q];
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int l = l0 + q;
-                if (l < nsls)
-                    mvk[od + l * ls] = abg[l] * m[q] +
-                                       abg[CD_MAX_SLS + l] * dso +
-                                       abg[2 * CD_MAX_SLS + l] * dn;
+                for (int l = 0; l < NS; l++) {
+                    sd -= m[d][l];
+                    mv[((d0 + d) * cs + l * ls) + at] =
+                        next(m[d][l], l, dso[d], dn);
+                }
+                sv[d0 + d] = (Real)sd;
+                ds[(d0 + d) * cs + at] = dsn[d0 + d];
             }
         }
+    } else {
+#pragma unroll
+        for (int d = 0; d < 6; d++) {
+            const int od = d * cs;
+            const double dso = (double)ds[od + at];
+            const double dn = (double)dsn[d];
+            double sd = (double)sv[d];
+            for (int l0 = 0; l0 < nsls; l0 += 4) {
+                double m[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    m[q] = l0 + q < nsls ? mv[(od + (l0 + q) * ls) + at] : 0.;
+#pragma unroll
+                for (int q = 0; q < 4; q++) sd -= m[q];
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    if (l0 + q < nsls)
+                        mv[(od + (l0 + q) * ls) + at] =
+                            next(m[q], l0 + q, dso, dn);
+            }
+            sv[d] = (Real)sd;
+            ds[od + at] = dsn[d];
+        }
     }
-    sig = (Real)sd;
-    dsk[od] = dsn;
 }
 
 // Stress sv of the strain e at slice k (Isotropic::strainToStress,
 // Isotropic.hpp:155-172; TransverselyIsotropic::strainToStress,
 // TransverselyIsotropic.hpp:161-180; Anisotropic::strainToStress,
 // Anisotropic.hpp:203-274) with the SLS memory update at an attenuation
-// point (att).
+// point (att: the slot's place of this slice, or -1); k: the point's place
+// of this slice.
 template <typename Real, int NS, int MT>
 __device__ __forceinline__ void slice_stress(const Real (&e)[6],
                                              const SliceMat<Real> &M, int k,
-                                             bool att, int nsls,
+                                             int att, int nsls,
                                              const double *abg,
                                              Real (&sv)[6]) {
     if constexpr (MT == 0) {
@@ -117,18 +153,15 @@ __device__ __forceinline__ void slice_stress(const Real (&e)[6],
     } else {
         aniso_hooke<Real, Real>(e, [&](int c) { return M.p(c, k); }, sv);
     }
-    if (NS != 0 && att) {
-        const Real dl = M.dl[k], dm = M.dm[k];
+    if (NS != 0 && att >= 0) {
+        const Real dl = M.dl[att], dm = M.dm[att];
         const Real dm2 = dm * (Real)2;
         const Real tr = e[0] + e[1] + e[2];
-        double *mvk = M.mv + k;
-        Real *dsk = M.ds + k;
-        const int cs = (int)M.cs;
+        Real dsn[6];
 #pragma unroll
         for (int d = 0; d < 6; d++)
-            att_update<Real, NS>(mvk, dsk, cs, nsls, abg, d,
-                                 d < 3 ? tr * dl + e[d] * dm2 : e[d] * dm,
-                                 sv[d]);
+            dsn[d] = d < 3 ? tr * dl + e[d] * dm2 : e[d] * dm;
+        att_update<Real, NS>(M, att, nsls, abg, dsn, sv);
     }
 }
 
