@@ -1012,11 +1012,9 @@ void DomainBase::finalize() {
     }
     // receivers
     mNumRec = (int)hRecElem.size();
-    mRecNu1Max = 0;
     for (int32_t e : hRecElem) {
         if (e < 0 || e >= mNumElems)
             throw Error("Domain::finalize || Receiver element out of range.");
-        mRecNu1Max = std::max(mRecNu1Max, eNu1[e]);
     }
 
     // fluid points, elements, boundaries and the solid-fluid coupling
@@ -1299,9 +1297,7 @@ void DomainBase::finalize() {
             dFHalf.alloc((size_t)mNumFModes * 2 * sizeof(double));
     }
     if (mNumRec > 0) {
-        up(dRecElem, hRecElem.data(), hRecElem.size() * 4);
         up(dRecW, hRecW.data(), hRecW.size() * 8);
-        up(dRecPhi, hRecPhi.data(), hRecPhi.size() * 8);
         if (!hRecRot.empty()) up(dRecRot, hRecRot.data(), hRecRot.size() * 8);
         // the points with a weight, and the orders' phase factors
         std::vector<RecPoint> pts((size_t)mNumRec * NPEM, RecPoint{0, 0, 0.});
@@ -1641,6 +1637,43 @@ void DomainBase::adjointDensity(const double *psi, const double *u,
                              hipMemcpyDeviceToHost, mStream),
               "Domain::adjointDensity");
     hip_check(hipStreamSynchronize(mStream), "Domain::adjointDensity");
+}
+
+// The receivers grouped by element, as the adjoint force takes them.
+AdjSourceArgs DomainBase::adjSourceArgs() {
+    AdjSourceArgs a;
+    if (mNumRec == 0) return a;
+    if (dAdjRec.bytes() == 0) {
+        std::vector<int32_t> rec(mNumRec), elem, first;
+        for (int r = 0; r < mNumRec; r++) rec[r] = r;
+        std::stable_sort(rec.begin(), rec.end(), [&](int x, int y) {
+            return hRecElem[x] < hRecElem[y];
+        });
+        for (int k = 0; k < mNumRec; k++)
+            if (k == 0 || hRecElem[rec[k]] != hRecElem[rec[k - 1]]) {
+                elem.push_back(hRecElem[rec[k]]);
+                first.push_back(k);
+            }
+        first.push_back(mNumRec);
+        auto up = [&](DeviceBuffer &b, const std::vector<int32_t> &v) {
+            b.alloc(v.size() * 4);
+            b.upload(v.data(), v.size() * 4, mStream);
+        };
+        up(dAdjRecElem, elem);
+        up(dAdjRecFirst, first);
+        up(dAdjRec, rec);
+    }
+    a.n = (int)(dAdjRecElem.bytes() / 4);
+    a.elem = dAdjRecElem.as<int32_t>();
+    a.first = dAdjRecFirst.as<int32_t>();
+    a.rec = dAdjRec.as<int32_t>();
+    a.w = dRecW.as<double>();
+    a.cis = dRecCis.as<double2>();
+    a.cis_off = dRecCisOff.as<int64_t>();
+    a.elem_modes = dElemModes.as<uint2>();
+    a.elem_nu1 = dElemNu1.as<int32_t>();
+    a.elem_eb_off = dElemEBOff.as<uint32_t>();
+    return a;
 }
 
 void DomainBase::swapAdjointFields() {
@@ -2510,6 +2543,7 @@ public:
         dAdjA.zero(mStream);
         for (int i = 0; i < 4; i++) dAdjAtt[i].zero(mStream);
         const double dt2 = mDt * mDt;
+        const AdjSourceArgs adjSource = adjSourceArgs();
         double *su = dAdjSegU.as<double>(), *sa = dAdjSegA.as<double>();
         for (int s = nck - 1; s >= 0; s--) {
             const int n0 = s * seg, n1 = std::min(n0 + seg, nsteps);
@@ -2558,12 +2592,9 @@ public:
                 }
                 elementKernel();
                 launch_adjoint_source<Real>(
-                    mStream, mNumRec, dRecElem.as<int32_t>(),
-                    dRecW.as<double>(), dRecPhi.as<double>(),
+                    mStream, adjSource,
                     dAdjG.as<double>() + (size_t)n * mNumRec * 3, 1.0 / dt2,
-                    mRecNu1Max, dElemPoints.as<int32_t>(),
-                    dElemNu1.as<int32_t>(), dPointNu1.as<int32_t>(),
-                    dElemEBOff.as<uint32_t>(), dEB.as<Real>());
+                    dEB.as<Real>());
                 point(all);
             }
             swapAdjointFields();

@@ -419,8 +419,7 @@ protected:
         dFInvMass3D, dCpl3DSolid, dCpl3DNOff, dCpl3DNu, dCpl3DNam,
         dCpl3DCOff, dCplSolidPair3D, dCSolid3D;
     // device: source and receivers
-    DeviceBuffer dSrcForce, dSrcIdx, dSrcOff, dSrcNu1, dStf, dRecElem, dRecW,
-        dRecPhi, dSeismo;
+    DeviceBuffer dSrcForce, dSrcIdx, dSrcOff, dSrcNu1, dStf, dRecW, dSeismo;
     // receivers as the record kernels read them (RecordArgs)
     DeviceBuffer dRecPts, dRecNpt, dRecNu1, dRecCis, dRecCisOff;
     RecordArgs recordArgs(int isample, bool dev) const;
@@ -474,7 +473,6 @@ protected:
         DeviceBuffer *b[4] = {&dMemVar, &dDStress, &dMemVarFR, &dDStressFR};
         return b[i];
     }
-    int mRecNu1Max = 0;
     void adjointCheck(bool media = false) const;
     // media form of the adjoint: offsets of each element's parameters in
     // the packed output, their total, the types and FP64 rotations
@@ -485,6 +483,8 @@ protected:
     SensArgs sensArgs(const double *psi, const double *u, const double *a,
                       double *kern, double scale) const;
     void swapAdjointFields();
+    DeviceBuffer dAdjRecElem, dAdjRecFirst, dAdjRec;
+    AdjSourceArgs adjSourceArgs();
 
     virtual void uploadReal() = 0;   // precision-specific operand upload
     virtual void autotune() = 0;     // pick kernel variants by timing

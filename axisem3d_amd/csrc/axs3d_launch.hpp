@@ -522,14 +522,20 @@ void launch_cd_sens(hipStream_t st, const CardArgs<Real> &a, const Real *scrb,
                     double scale);
 
 // adjoint force R^* g * scale into the receivers' element-local forces
+struct AdjSourceArgs {
+    int n = 0;                     // elements with receivers
+    const int32_t *elem = nullptr, *first = nullptr;  // [n], [n + 1]
+    const int32_t *rec = nullptr;  // receivers by element, ascending
+    const double *w = nullptr;     // [receiver][25]
+    const double2 *cis = nullptr;  // RecordArgs::cis
+    const int64_t *cis_off = nullptr;
+    const uint2 *elem_modes = nullptr;
+    const int32_t *elem_nu1 = nullptr;
+    const uint32_t *elem_eb_off = nullptr;
+};
 template <typename Real>
-void launch_adjoint_source(hipStream_t st, int nrec, const int32_t *rec_elem,
-                           const double *rec_w, const double *rec_phi,
-                           const double *g, double scale, int nu1max,
-                           const int32_t *elem_points,
-                           const int32_t *elem_nu1,
-                           const int32_t *point_nu1,
-                           const uint32_t *elem_eb_off, Real *eb);
+void launch_adjoint_source(hipStream_t st, const AdjSourceArgs &a,
+                           const double *g, double scale, Real *eb);
 
 // step counter of a replayed (graph) step; see k_step_set
 void launch_step_set(hipStream_t st, int *ctr, int tstep, int record_step0);
