@@ -134,7 +134,7 @@ __device__ __forceinline__ void unpack_pair(const cpx<Real> *buf,
 // A: gradient of the element-modes [em0, em1) of the 3D element-mode list
 // into the scratch rows [d*25 + ipnt][alpha] of each element, rotated to
 // RTZ for TI and anisotropic media on spherical meshes (SolidElement.cpp:
-// 177-193).  One thread per (element-mode, GLL point), ten element-modes
+// 177-193).  One thread per (element-mode, GLL point), sixteen element-modes
 // per block, the Fourier order fastest so that a row's consecutive orders
 // are written by consecutive lanes (CD_EMB = 16 orders: 128-byte runs in
 // FP32).
