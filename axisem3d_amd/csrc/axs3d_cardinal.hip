@@ -783,14 +783,18 @@ __global__ __launch_bounds__(128) void k_mass3d(Mass3DArgs<Real> a,
                     vv = a.veloc[m6 + ri] + a.sym_pi * a.dt * an[ri];
                     uu = u0 + a.sym_kappa * a.dt * vv;
                 } else {
-                    const bool fh = march_reads_half(a.march);
-                    vv = fh ? a.half[m6 + ri] : a.veloc[m6 + ri];
                     uu = u0;
-                    newmark_march(a.march, a.dt, hdt, hdt2,
-                                  fh ? 0. : a.accel[m6 + ri], an[ri], uu, vv);
                     if (a.march != MARCH_FULL) {
-                        a.half[m6 + ri] = vv;
-                        vv -= hdt * an[ri];
+                        double w = march_reads_half(a.march)
+                                       ? a.half[m6 + ri]
+                                       : half_of(hdt, a.veloc[m6 + ri],
+                                                 a.accel[m6 + ri]);
+                        vv = newmark_half(a.dt, hdt, an[ri], uu, w);
+                        a.half[m6 + ri] = w;
+                    } else {
+                        vv = a.veloc[m6 + ri];
+                        newmark_full(a.dt, hdt, hdt2, a.accel[m6 + ri],
+                                     an[ri], uu, vv);
                     }
                     va = march_writes_va(a.march);
                     if (va) a.accel[m6 + ri] = an[ri];
@@ -1196,14 +1200,18 @@ __global__ __launch_bounds__(128) void k_fluid_defer(FluidDeferArgs<Real> a) {
                 vv = a.chi_v[m2 + ri] + a.sym_pi * a.dt * an[ri];
                 uu = u0 + a.sym_kappa * a.dt * vv;
             } else {
-                const bool fh = march_reads_half(a.march);
-                vv = fh ? a.half[m2 + ri] : a.chi_v[m2 + ri];
                 uu = u0;
-                newmark_march(a.march, a.dt, hdt, hdt2,
-                              fh ? 0. : a.chi_a[m2 + ri], an[ri], uu, vv);
                 if (a.march != MARCH_FULL) {
-                    a.half[m2 + ri] = vv;
-                    vv -= hdt * an[ri];
+                    double w = march_reads_half(a.march)
+                                   ? a.half[m2 + ri]
+                                   : half_of(hdt, a.chi_v[m2 + ri],
+                                             a.chi_a[m2 + ri]);
+                    vv = newmark_half(a.dt, hdt, an[ri], uu, w);
+                    a.half[m2 + ri] = w;
+                } else {
+                    vv = a.chi_v[m2 + ri];
+                    newmark_full(a.dt, hdt, hdt2, a.chi_a[m2 + ri], an[ri],
+                                 uu, vv);
                 }
                 va = march_writes_va(a.march);
                 if (va) a.chi_a[m2 + ri] = an[ri];

@@ -289,26 +289,34 @@ __global__ __launch_bounds__(256) void k_fluid_point(
         return;
     }
     // all of the state is loaded (16-byte vectors) before anything is stored
-    double2 *hp = reinterpret_cast<double2 *>(a.half + (size_t)k * 2);
-    const bool from_half = march_reads_half(a.march);
-    const double2 u0 = *up, v0 = from_half ? *hp : *vp;
-    double2 a0 = make_double2(0., 0.);
-    if (!from_half) a0 = *ap;
-    double vr = v0.x, vi = v0.y, ur = u0.x, ui = u0.y;
-    newmark_march(a.march, a.dt, a.half_dt, a.half_dt_dt, a0.x, s[0], ur, vr);
-    newmark_march(a.march, a.dt, a.half_dt, a.half_dt_dt, a0.y, s[1], ui, vi);
-    *up = make_double2(ur, ui);
+    double2 u = *up;
+    const bool bad0 = !isfinite(u.x) || !isfinite(u.y);
+    double2 v;
     if (a.march != MARCH_FULL) {
-        *hp = make_double2(vr, vi);
-        vr -= a.half_dt * s[0];
-        vi -= a.half_dt * s[1];
+        double2 *hp = reinterpret_cast<double2 *>(a.half + (size_t)k * 2);
+        double2 w;
+        if (march_reads_half(a.march)) {
+            w = *hp;
+        } else {
+            const double2 v0 = *vp, a0 = *ap;
+            w = make_double2(half_of(a.half_dt, v0.x, a0.x),
+                             half_of(a.half_dt, v0.y, a0.y));
+        }
+        v.x = newmark_half(a.dt, a.half_dt, s[0], u.x, w.x);
+        v.y = newmark_half(a.dt, a.half_dt, s[1], u.y, w.y);
+        *hp = w;
+    } else {
+        const double2 a0 = *ap;
+        v = *vp;
+        newmark_full(a.dt, a.half_dt, a.half_dt_dt, a0.x, s[0], u.x, v.x);
+        newmark_full(a.dt, a.half_dt, a.half_dt_dt, a0.y, s[1], u.y, v.y);
     }
+    *up = u;
     if (march_writes_va(a.march)) {
-        *vp = make_double2(vr, vi);
+        *vp = v;
         *ap = make_double2(s[0], s[1]);
     }
-    const bool bad = !isfinite(ur) || !isfinite(ui);
-    const bool bad0 = !isfinite(u0.x) || !isfinite(u0.y);
+    const bool bad = !isfinite(u.x) || !isfinite(u.y);
     if (!GATHER) stiff[(size_t)k * 2] = stiff[(size_t)k * 2 + 1] = 0;
     raise_flag(a.flag, a.note, bad0, bad);
 }

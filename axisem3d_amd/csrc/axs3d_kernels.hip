@@ -677,41 +677,55 @@ __global__ __launch_bounds__(256) void k_point(PointArgs a,
         raise_flag(a.flag, a.note, bad0, bad);
         return;
     }
-    double2 *hp = reinterpret_cast<double2 *>(a.half + (size_t)k * 6);
-    const bool from_half = march_reads_half(a.march);
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        u2[c] = up[c];
-        v2[c] = from_half ? hp[c] : vp[c];
-        a2[c] = make_double2(0., 0.);
-    }
-    if (!from_half)
-#pragma unroll
-        for (int c = 0; c < 3; c++) a2[c] = ap[c];
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        bad0 |= !isfinite(u2[c].x) || !isfinite(u2[c].y);
-        newmark_march(a.march, dt, half_dt, half_dt_dt, a2[c].x,
-                      a_new[2 * c], u2[c].x, v2[c].x);
-        newmark_march(a.march, dt, half_dt, half_dt_dt, a2[c].y,
-                      a_new[2 * c + 1], u2[c].y, v2[c].y);
-        bad |= !isfinite(u2[c].x) || !isfinite(u2[c].y);
-    }
-#pragma unroll
-    for (int c = 0; c < 3; c++) up[c] = u2[c];
     if (a.march != MARCH_FULL) {
+        double2 *hp = reinterpret_cast<double2 *>(a.half + (size_t)k * 6);
+        const bool from_half = march_reads_half(a.march);
+        const bool to_va = march_writes_va(a.march);
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            hp[c] = v2[c];
-            v2[c].x -= half_dt * a_new[2 * c];
-            v2[c].y -= half_dt * a_new[2 * c + 1];
+            u2[c] = up[c];
+            v2[c] = from_half ? hp[c] : vp[c];
         }
-    }
-    if (march_writes_va(a.march)) {
+        if (!from_half)
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                const double2 a0 = ap[c];
+                v2[c] = make_double2(half_of(half_dt, v2[c].x, a0.x),
+                                     half_of(half_dt, v2[c].y, a0.y));
+            }
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            vp[c] = v2[c];
+            double2 u = u2[c], w = v2[c], v;
+            bad0 |= !isfinite(u.x) || !isfinite(u.y);
+            v.x = newmark_half(dt, half_dt, a_new[2 * c], u.x, w.x);
+            v.y = newmark_half(dt, half_dt, a_new[2 * c + 1], u.y, w.y);
+            bad |= !isfinite(u.x) || !isfinite(u.y);
+            up[c] = u;
+            hp[c] = w;
+            if (to_va) {
+                vp[c] = v;
+                ap[c] = make_double2(a_new[2 * c], a_new[2 * c + 1]);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            u2[c] = up[c];
+            v2[c] = vp[c];
+            a2[c] = ap[c];
+        }
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            double2 u = u2[c], v = v2[c];
+            bad0 |= !isfinite(u.x) || !isfinite(u.y);
+            newmark_full(dt, half_dt, half_dt_dt, a2[c].x, a_new[2 * c], u.x,
+                         v.x);
+            newmark_full(dt, half_dt, half_dt_dt, a2[c].y, a_new[2 * c + 1],
+                         u.y, v.y);
+            bad |= !isfinite(u.x) || !isfinite(u.y);
+            vp[c] = v;
             ap[c] = make_double2(a_new[2 * c], a_new[2 * c + 1]);
+            up[c] = u;
         }
     }
     if (!GATHER) {

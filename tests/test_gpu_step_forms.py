@@ -6,7 +6,9 @@ for n around the lengths where the form or the graph changes, on a solid with
 receivers of few and of several hundred orders and on a fluid layer with 3D
 coupling and 3D masses (points marched by other kernels).  Where the program
 sets the velocity and the acceleration in between, w follows them: the run
-equals that of a solver that starts from those fields."""
+equals that of a solver that starts from those fields.  And w is what the
+velocity and the acceleration give: a run that goes on from fields read from a
+solver, in another or set again in the same, is the unbroken run bit by bit."""
 import math
 
 import numpy as np
@@ -99,5 +101,43 @@ def test_run_equals_single_steps(case, prec, n):
     c.run(n)
     for f in fields:
         assert np.array_equal(a.get_field(f), c.get_field(f)), f
+    for g in (a, b, c):
+        g.close()
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("case", ["solid", "fluid"])
+@pytest.mark.parametrize("n", [1, 12])
+def test_run_from_saved_fields_equals_unbroken_run(case, prec, n):
+    from axisem3d_amd.solver import GpuSolver
+    m = 14
+    spec = (_solid if case == "solid" else _fluid)(n + m)
+    fields = ["displ", "veloc", "accel"]
+    if case == "fluid":
+        fields += ["fdispl", "fveloc", "faccel"]
+    a, b, c = (GpuSolver(spec, prec) for _ in range(3))
+    rng = np.random.default_rng(8)
+    for f in fields:
+        x = a.get_field(f)
+        x = rng.standard_normal(x.shape) + 1j * rng.standard_normal(x.shape)
+        x *= {"d": 1.0, "v": 1.0 / spec.dt,
+              "a": 1.0 / spec.dt ** 2}[f.lstrip("f")[0]] * 1e-3
+        a.set_field(f, x)
+        b.set_field(f, x)
+    a.run(n + m)
+    b.run(n)
+    for f in fields:
+        x = b.get_field(f)
+        b.set_field(f, x)
+        c.set_field(f, x)
+    c.step = n
+    b.run(m)
+    c.run(m)
+    for g in (b, c):
+        for f in fields:
+            assert np.array_equal(a.get_field(f), g.get_field(f)), f
+        s = a.seismograms()[n:]
+        assert np.abs(s).max() > 0
+        assert np.array_equal(s, g.seismograms()[n:])
     for g in (a, b, c):
         g.close()
