@@ -2345,6 +2345,22 @@ public:
         fluidPoint(PHASE_MARCH);
     }
 
+    void recordKernel(const RecordArgs &rec) {
+        if (rec.nrec <= 0) return;
+        tick(AXS3D_KERNEL_RECORD);
+        launch_record(mStream, rec);
+        tock(AXS3D_KERNEL_RECORD);
+    }
+    // Whether the receivers ride on the step's first element launch: always
+    // but in too many large blocks of the one-kernel form.
+    bool receiversRide(const RecordArgs &rec) const {
+        if (mNumEM > 0 || !mCardBatches.empty() || mFusedGroups.empty())
+            return true;
+        return (int64_t)rec.nrec *
+                   fused_threads<Real>(mFusedGroups.front().nr_max) <=
+               FUSED_RIDER_THREADS;
+    }
+
     // One Newmark step in its bulk form: the element kernels write the
     // element-local forces (the source's among its element's) and sample
     // the receivers from u(t), then one fluid and one solid point kernel
@@ -2367,12 +2383,7 @@ public:
             // 103): record, source (into the first sub-step's forces),
             // launch, then four sub-steps of stiffness, boundaries, mass
             // and update
-            const RecordArgs rec = recordArgs(isample, dev);
-            if (rec.nrec > 0) {
-                tick(AXS3D_KERNEL_RECORD);
-                launch_record(mStream, rec);
-                tock(AXS3D_KERNEL_RECORD);
-            }
+            recordKernel(recordArgs(isample, dev));
             symplecticLaunch();
             for (int isub = 1; isub <= 4; isub++) {
                 if (isub == 1)
@@ -2388,6 +2399,10 @@ public:
             }
         } else {
             h.rec = recordArgs(isample, dev);
+            if (!receiversRide(h.rec)) {
+                recordKernel(h.rec);
+                h.rec = RecordArgs();
+            }
             elementKernel(false, h, sourceArgs(tstep, dev));
             abcKernel();
             fluidPoint(all | PHASE_COUPLE);

@@ -276,15 +276,17 @@ __global__ __launch_bounds__(FusedBlock<Real>::value) void k_cd_fused(
     }
 }
 
+template <typename Real>
+int fused_threads(int nr) {
+    const int want = (NPEM * (nr / 2 + 1) + 63) & ~63;
+    return std::max(128, std::min(want, (int)FusedBlock<Real>::value));
+}
+
 template <typename Real, int MT>
 static void launch_fused_mt(hipStream_t st, const CardArgs<Real> &a,
                             const FusedGroup &g, const StepArgs &h) {
-    // one thread per (point, order) of the largest element, up to the
-    // largest block
-    const int want = (NPEM * (g.nr_max / 2 + 1) + 63) & ~63;
-    const int threads =
-        std::max(128, std::min(want, (int)FusedBlock<Real>::value));
-    const dim3 grid(h.rec.nrec + g.end - g.begin), block(threads);
+    const dim3 grid(h.rec.nrec + g.end - g.begin);
+    const dim3 block(fused_threads<Real>(g.nr_max));
     const size_t lds = fused_lds_bytes<Real>(g.nr_max);
     if (a.nsls == 0)
         hipLaunchKernelGGL((k_cd_fused<Real, 0, MT>), grid, block, lds, st,
@@ -310,6 +312,8 @@ void launch_cd_fused(hipStream_t st, const CardArgs<Real> &a,
     h = StepArgs();
 }
 
+template int fused_threads<float>(int);
+template int fused_threads<double>(int);
 template size_t fused_lds_bytes<float>(int);
 template size_t fused_lds_bytes<double>(int);
 template void launch_cd_fused<float>(hipStream_t, const CardArgs<float> &,

@@ -415,6 +415,20 @@ constexpr int FUSED_NR_CAP = 400;
 constexpr size_t FUSED_LDS_MAX = (size_t)158 << 10;
 constexpr int FUSED_GROUP_MIN = 512;
 constexpr int FUSED_WITH_LARGER_MIN = 256;
+// Its threads per block for a group whose largest element is of nr: one per
+// (point, order), up to the largest block.
+template <typename Real>
+int fused_threads(int nr);
+// Most threads that the receivers' blocks of such a launch may have together;
+// with more of them the receivers take a launch of their own.  A receiver's
+// block is as large as an element's, and takes its place: 256 receivers in
+// blocks of 1024 threads cost 3 us a step, where the launch of their own costs
+// 4 to 7 us, and 0.4 us for each 256 of them.  Us a step, riding against a
+// launch of their own, at 512, 1024 and 4096 receivers: 960 elements of Nr up
+// to 121 (1024 threads) 101 to 104, 107 to 104, 144 to 109; 640 of Nr up to 42
+// (576 threads) 51 to 52, 56 to 53, 81 to 58; 480 of Nr 9 (128 threads) 16.6 to
+// 20.3, 16.8 to 20.8, 21.1 to 25.5.
+constexpr int64_t FUSED_RIDER_THREADS = 512 * 1024;
 // Its dynamic LDS for an element of nr.
 template <typename Real>
 size_t fused_lds_bytes(int nr);

@@ -4,9 +4,10 @@
 // Each of these is a few microseconds of work whose launch costs as much
 // as a small domain's element kernel (about 5 us a launch on the serial
 // path of the step), so none has a launch of its own: the first element
-// kernel of a step runs one extra block per receiver, every element kernel
-// adds the source force where it writes the source element's forces, and
-// the step's number travels through the flag words.
+// kernel of a step runs one extra block per receiver (but see
+// FUSED_RIDER_THREADS), every element kernel adds the source force where it
+// writes the source element's forces, and the step's number travels through
+// the flag words.
 #pragma once
 
 #include "axs3d_common.hpp"

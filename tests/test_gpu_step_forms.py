@@ -8,7 +8,9 @@ coupling and 3D masses (points marched by other kernels).  Where the program
 sets the velocity and the acceleration in between, w follows them: the run
 equals that of a solver that starts from those fields.  And w is what the
 velocity and the acceleration give: a run that goes on from fields read from a
-solver, in another or set again in the same, is the unbroken run bit by bit."""
+solver, in another or set again in the same, is the unbroken run bit by bit.
+Receivers ride on the step's first element launch, or, where that launch has
+large blocks and they are many, take one of their own."""
 import math
 
 import numpy as np
@@ -141,3 +143,45 @@ def test_run_from_saved_fields_equals_unbroken_run(case, prec, n):
         assert np.array_equal(s, g.seismograms()[n:])
     for g in (a, b, c):
         g.close()
+
+
+# one-kernel form: at most 512 x 1024 threads of receivers' blocks ride.  Nr
+# 90: 1024 threads in FP32, 512 in FP64; Nr 9: 128 threads
+@pytest.mark.parametrize("prec,nr,nrec,own", [
+    ("fp32", 90, 512, False), ("fp32", 90, 513, True),
+    ("fp64", 81, 1024, False), ("fp64", 81, 1025, True),
+    ("fp32", 9, 1500, False)])
+def test_many_receivers(prec, nr, nrec, own):
+    from axisem3d_amd import capi
+    from axisem3d_amd.solver import GpuSolver
+    n = 12
+    mesh = preloop.StructuredMesh(np.linspace(0, 4e3, 4),
+                                  np.linspace(0, 3e3, 4))
+    _, prof = preloop.layered_profile(3, 3e3, 0.)
+    sp = preloop.build_domain(mesh, prof, lambda s, z: nr + 0. * s,
+                              courant=0.4 / nr, bound_nr=False)
+    field = preloop.RandomField(5, corr_len=3e3)
+    preloop.make_3d_isotropic(sp, field, None,
+                              np.ones(sp.n_solid_elements, bool))
+    mt = np.array([1.0, 0.7, 0.4, 0.3, 0.2, 0.1]) * 1e15
+    preloop.add_axial_moment_source(sp, 1.7e3, mt, 3 * sp.dt, 1.628, n)
+    s = 4e3 * (np.arange(nrec) + 0.5) / nrec
+    phi = np.linspace(0.0, 6.0, nrec)
+    preloop.add_receivers(sp, s, np.full(nrec, 3e3), phi)
+    g = GpuSolver(sp, prec)
+    assert g.autotune_info()["fused_elements"] == sp.n_solid_elements
+    g.profile(True)
+    g.run(n)
+    assert (g.profile_read(capi.KERNEL_RECORD)[1] > 0) == own
+    sel = np.r_[0:20, nrec // 2, nrec - 20:nrec]
+    preloop.add_receivers(sp, s[sel], np.full(len(sel), 3e3), phi[sel])
+    few = GpuSolver(sp, prec)
+    few.run(n)
+    a, b = g.seismograms()[:, sel], few.seismograms()
+    # the same field; a receiver's sum of 25 points and up to 46 orders in
+    # another order
+    assert np.abs(b).max() > 0
+    assert np.abs(a - b).max() < 25 * 46 * 2.3e-16 * np.abs(
+        few.get_field("displ")).max()
+    for x in (g, few):
+        x.close()
