@@ -2884,6 +2884,10 @@ private:
             const int end = mTypeBegin3D[mt + 1];
             while (w < end && hElemNr[hList3D[w]] > mFusedNrMax) w++;
             if (larger && end - w < FUSED_WITH_LARGER_MIN) w = end;
+            // few large ones leave most of the chip idle, a block each
+            if (end - w < FUSED_FEW && w < end &&
+                fused_lds_bytes<Real>(hElemNr[hList3D[w]]) > FUSED_FEW_LDS)
+                w = end;
             mFusedBegin[mt] = w;
             mNumFused += end - w;
             while (w < end) {

@@ -407,12 +407,25 @@ struct FusedGroup {
 };
 // Largest Nr the one-kernel form can index.
 constexpr int FUSED_NR_CAP = 400;
-// Largest dynamic LDS the one-kernel form takes for an element (one block
-// per CU: faster than the three-kernel form up to there, 960 elements of Nr
-// 11 to 121 take 164 us a step without it, 134 with it up to Nr 90 and 98 up
-// to 121), the fewest elements of a launch group, and of a type next to
-// elements of larger Nr.
+// Largest dynamic LDS the one-kernel form takes for an element: what a CU has,
+// for one block (Nr 168 in FP32, 83 in FP64).  From 64 elements on it is the
+// faster form up to there: us a step of elements of Nr 168 (FP32, CG4), in
+// three kernels against one, 46.5 to 46.9 for 64 elements, 55.5 to 53.1 for
+// 128, 76.7 to 64.5 for 256, 159 to 117 for 512; of Nr 140, 44 to 43, 54 to
+// 50, 70 to 59, 120 to 106; of Nr 72 in FP64, 36 to 30, 48 to 34, 61 to 42,
+// 100 to 71.
 constexpr size_t FUSED_LDS_MAX = (size_t)158 << 10;
+// Fewer elements than this, if some need more than FUSED_FEW_LDS, take the
+// three kernels, which spread an element's 25 points over 5 to 25 blocks: 4,
+// 16 and 32 elements of Nr 125 (FP32, CG4) 30.5, 31.2, 33.1 us a step in three
+// kernels, 37.6, 37.7, 38.5 in one; of Nr 168 30.8, 32.2, 35.5 against 39.9,
+// 40.5, 42.0; of Nr 63 in FP64 26.7, 27.6, 29.0 against 28.9, 28.8, 29.4.
+// Smaller ones are faster in one kernel at any count (Nr 77: 28.4 against
+// 26.5; Nr 52 in FP64 28.5 against 26.7).
+constexpr int FUSED_FEW = 48;
+constexpr size_t FUSED_FEW_LDS = (size_t)112 << 10;
+// The fewest elements of a launch group, and of a type next to elements of
+// larger Nr.
 constexpr int FUSED_GROUP_MIN = 512;
 constexpr int FUSED_WITH_LARGER_MIN = 256;
 // Its threads per block for a group whose largest element is of nr: one per

@@ -23,9 +23,9 @@ pytestmark = pytest.mark.gpu
 STEPS = 30
 
 
-def _spec(nr0, nr1, mtype, att, nsls):
+def _spec(nr0, nr1, mtype, att, nsls, ntheta=3, nrad=2):
     sp = preloop.spherical_regional(
-        ntheta=3, nrad=2, theta_max_deg=3.0, depth=100e3, nu_min=1, nu_max=1,
+        ntheta=ntheta, nrad=nrad, theta_max_deg=3.0, depth=100e3, nu_min=1, nu_max=1,
         nsteps=STEPS, attenuation=att is not None, cg4=att == "cg4",
         nsls=nsls, corr_len=40e3, bound_nr=False)
     s_max = 6371e3 * np.sin(np.radians(3.0))
@@ -86,4 +86,32 @@ def test_small_nr_matches_oracle(prec, tol, nr0, nr1, mtype, att, nsls):
     assert eu < (1e-12 if prec == "fp64" else 1e-4)
     if np.abs(ref).max() > 0:
         assert es < (1e-12 if prec == "fp64" else 1e-4)
+    g.close()
+
+
+# the form each element should take: the LDS holds Nr 168 in FP32 and 83 in
+# FP64; from Nr 120 and 58 (112 KiB) fewer than 48 of a medium take the three
+# kernels
+@pytest.mark.parametrize("prec,nr,ntheta,nrad,fused", [
+    ("fp32", 117, 3, 2, 6), ("fp32", 120, 3, 2, 0), ("fp32", 120, 47, 1, 0),
+    ("fp32", 120, 8, 6, 48), ("fp32", 168, 8, 6, 48), ("fp32", 175, 8, 6, 0),
+    ("fp64", 56, 3, 2, 6), ("fp64", 60, 3, 2, 0), ("fp64", 60, 47, 1, 0),
+    ("fp64", 60, 8, 6, 48), ("fp64", 81, 8, 6, 48), ("fp64", 84, 8, 6, 0)])
+def test_form_by_count_and_size(prec, nr, ntheta, nrad, fused):
+    from axisem3d_amd.solver import GpuSolver
+    sp = _spec(nr, nr, "iso", "cg4", 5, ntheta, nrad)
+    assert set(sp.elem_nr.tolist()) == {nr}
+    o = oracle.Oracle(sp)
+    g = GpuSolver(sp, prec)
+    assert g.autotune_info()["fused_elements"] == fused
+    rng = np.random.default_rng(23)
+    for k in range(2):
+        u = rng.standard_normal((o.nmodes, 3)) + 1j * rng.standard_normal(
+            (o.nmodes, 3))
+        g.set_field("displ", u)
+        g.set_field("stiff", np.zeros_like(u))
+        g.computeStiffness()
+        e = _rel(g.get_field("stiff"), o.stiffness(u))
+        print(f"{sp.n_solid_elements} of Nr {nr} {prec} pass {k}: {e:.2e}")
+        assert e < (1e-13 if prec == "fp64" else 1e-5)
     g.close()

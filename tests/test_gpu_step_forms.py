@@ -146,10 +146,10 @@ def test_run_from_saved_fields_equals_unbroken_run(case, prec, n):
 
 
 # one-kernel form: at most 512 x 1024 threads of receivers' blocks ride.  Nr
-# 90: 1024 threads in FP32, 512 in FP64; Nr 9: 128 threads
+# 90: 1024 threads in FP32; Nr 50: 512 in FP64; Nr 9: 128
 @pytest.mark.parametrize("prec,nr,nrec,own", [
     ("fp32", 90, 512, False), ("fp32", 90, 513, True),
-    ("fp64", 81, 1024, False), ("fp64", 81, 1025, True),
+    ("fp64", 50, 1024, False), ("fp64", 50, 1025, True),
     ("fp32", 9, 1500, False)])
 def test_many_receivers(prec, nr, nrec, own):
     from axisem3d_amd import capi
