@@ -471,11 +471,12 @@ void launch_cd_quad(hipStream_t st, const CardArgs<Real> &a,
 // (c = dp/ds, i alpha p / s, dp/dz), C2R of the three series, K = 1 / rho
 // per slice (Acoustic::strainToStress _3D_CD, Acoustic.hpp:80-92), R2C,
 // computeQuad3 (GradientQuadrature.hpp:234-252) into the fluid
-// element-local forces.  The same three-kernel split as the solids.
+// element-local forces.  The same three-kernel split as the solids.  The
+// potential is contracted in FP64, as in the Fourier-path fluid kernel.
 template <typename Real>
 __global__ __launch_bounds__(CD_EMB_THREADS) void k_cdf_grad(
     FluidCardArgs<Real> a, int em0, int em1) {
-    __shared__ cpx<Real> sP[CD_EMB][NPEM];
+    __shared__ cpx<double> sP[CD_EMB][NPEM];
     __shared__ Real sG[2][NPEM];
     const FluidArgs<Real> &f = a.f;
     const int t = threadIdx.x;
@@ -486,7 +487,7 @@ __global__ __launch_bounds__(CD_EMB_THREADS) void k_cdf_grad(
     const bool active = t < CD_EMB * NPEM && em < em1;
     const int i = ipnt / NPED, j = ipnt - (ipnt / NPED) * NPED;
     int e = 0, alpha = 0;
-    cpx<Real> p = {0, 0};
+    cpx<double> p = {0, 0};
     if (active) {
         const EMItem it = f.em_list[em];
         e = it.elem;
@@ -494,7 +495,7 @@ __global__ __launch_bounds__(CD_EMB_THREADS) void k_cdf_grad(
         const int ip = f.elem_points[e * NPEM + ipnt];
         if (alpha < f.point_nu1[ip]) {
             const double *src = f.chi + (size_t)(f.point_off[ip] + alpha) * 2;
-            p = {(Real)src[0], (Real)src[1]};
+            p = {src[0], src[1]};
         }
         sP[eml][ipnt] = p;
     }
@@ -505,17 +506,20 @@ __global__ __launch_bounds__(CD_EMB_THREADS) void k_cdf_grad(
     load_point_g<Real>(sG, axial, i, j, G);
     PointOps<Real> g{}, q{};
     load_point_ops(f.elem_ops, e, ipnt, g, q);
-    cpx<Real> x = {0, 0}, y = {0, 0};
+    cpx<double> xd = {0, 0}, yd = {0, 0};
 #pragma unroll
     for (int k = 0; k < NPED; k++) {
-        x = cfma(sP[eml][k * NPED + j], G.gxi_col[k], x);
-        y = cfma(sP[eml][i * NPED + k], G.g_col[k], y);
+        xd = cfma(sP[eml][k * NPED + j], (double)G.gxi_col[k], xd);
+        yd = cfma(sP[eml][i * NPED + k], (double)G.g_col[k], yd);
     }
+    const cpx<Real> x = {(Real)xd.re, (Real)xd.im};
+    const cpx<Real> y = {(Real)yd.re, (Real)yd.im};
+    const cpx<Real> pr = {(Real)p.re, (Real)p.im};
     const Real ralpha = (Real)alpha;
     const cpx<Real> dpds = cadd(cmul(x, g.dzdeta), cmul(y, g.dzdxii));
     const cpx<Real> dpdz = cadd(cmul(x, g.dsdeta), cmul(y, g.dsdxii));
     const cpx<Real> ps = (axial && i == 0) ? ialpha(ralpha, dpds)
-                                           : cmul(ialpha(ralpha, p), g.invs);
+                                           : cmul(ialpha(ralpha, pr), g.invs);
     const int nu1 = f.elem_nu1[e];
     cpx<Real> *dst = reinterpret_cast<cpx<Real> *>(a.scratch) + a.scr_off[e] +
                      (size_t)ipnt * scr_row(nu1) + alpha;

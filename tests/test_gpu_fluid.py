@@ -205,3 +205,32 @@ def test_coupling3d_seismograms_match_oracle(prec, tol, layer):
     print(f"3D coupling {layer} {prec}: relative seismogram L2 = {err:.3e}")
     assert err < tol
     assert _rel(chi, o.fdispl) < 10 * tol
+
+
+def test_smooth_potential_in_fp32():
+    """The potential is large next to its differences between GLL points; it
+    is contracted in FP64 whatever the precision mode, in elements of either
+    medium: the FP32 force of a smooth potential is as close to the oracle's
+    in 3D elements as in the same elements taken as 1D."""
+    from axisem3d_amd.solver import GpuSolver
+    err = {}
+    for medium in ("1D", "3D"):
+        sp = _spec("middle")
+        if medium == "3D":
+            preloop.make_fluid3d(sp, np.arange(len(sp.fluid_elem_nr)),
+                                 amp=0.3, seed=5)
+        o = oracle.Oracle(sp)
+        g = GpuSolver(sp, "fp32")
+        # plane waves of 40 elements' length, falling with the order
+        wave = [np.cos(2 * np.pi * (x[0] + 0.7 * x[1]) / 40e3 + 0.3) *
+                np.exp(-np.arange(nr // 2 + 1)) * (1 + 0.5j)
+                for x, nr in zip(sp.fluid_sz, sp.fluid_nr)]
+        chi = np.concatenate(wave)
+        g.set_field("displ", np.zeros((o.nmodes, 3), complex))
+        g.set_field("fdispl", chi)
+        g.set_field("fstiff", np.zeros_like(chi))
+        g.computeStiffness()
+        err[medium] = _rel(g.get_field("fstiff"), o.fluid_stiffness(chi))
+        g.close()
+    print(f"smooth potential, FP32 force: {err}")
+    assert err["3D"] < 1.5 * err["1D"]
