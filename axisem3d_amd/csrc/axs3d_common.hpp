@@ -9,6 +9,7 @@ namespace axs3d {
 constexpr int NPED = 5;    // GLL points per direction (npol = 4)
 constexpr int NPEM = 25;   // GLL points per element
 constexpr int EMB = 10;    // Fourier path: element-modes per 256-thread block
+constexpr int CD_MAX_SLS = 16;  // cardinal path: most standard linear solids
 
 // Complex value; aligned to its size so that one LDS or global access
 // moves both parts.

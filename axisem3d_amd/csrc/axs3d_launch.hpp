@@ -144,11 +144,16 @@ inline size_t stress_lds_bytes(int nr, int count) {
 // owns the same strain pair of several points counts their butterflies
 // together.  As many (up to five, which divide the 25) as leave five blocks'
 // LDS per CU (fifteen waves of the sixteen the registers allow; in FP64 four
-// blocks, twelve waves).
+// blocks, twelve waves), with the kernel's static LDS in it and in whole
+// granules, of which a CU has 128.  384 elements with CG4, us a step, with one
+// point more and four blocks against this: 179 to 175 at Nr 231, 232 to 225 at
+// 288, 299 to 282 at 375, 400 to 402 at 528; without attenuation 312 to 289 at
+// 528.
 template <typename Real>
 inline int stress_points(int nr) {
-    const size_t budget = sizeof(Real) == 4 ? (size_t)32 << 10
-                                            : (size_t)40 << 10;
+    const size_t granule = 1280, blocks = sizeof(Real) == 4 ? 5 : 4;
+    const size_t budget =
+        128 / blocks * granule - 3 * CD_MAX_SLS * sizeof(double);
     int n = 1;
     while (n < 5 && stress_lds_bytes<Real>(nr, n + 1) <= budget) n++;
     return n;

@@ -51,7 +51,6 @@ struct SliceMat {
 // The update is bound by the latency of its loads, which no store may pass:
 // with a fixed count of solids two components' are issued together, then
 // their stores.
-constexpr int CD_MAX_SLS = 16;
 template <typename Real, int NS>
 __device__ __forceinline__ void att_update(const SliceMat<Real> &M, int at,
                                            int nsls, const double *abg,

@@ -63,3 +63,22 @@ def test_stress_blocks_match_oracle(prec, tol, nr0, nr1, mtype, att, nsls):
         print(f"Nr {nr0}..{nr1} {mtype} {att} {prec} pass {k}: {e:.2e}")
         assert e < tol
     g.close()
+
+
+@pytest.mark.parametrize("prec,nr", [
+    ("fp32", 180), ("fp32", 231), ("fp32", 288), ("fp32", 375),
+    ("fp32", 378), ("fp32", 525), ("fp32", 528), ("fp32", 810),
+    ("fp64", 150), ("fp64", 189), ("fp64", 240), ("fp64", 405)])
+def test_blocks_per_cu(prec, nr):
+    """The points of a block leave LDS for five blocks of a CU (four in
+    FP64), the kernel's own arrays included: as the runtime counts them, at Nr
+    on either side of where a block takes one point less."""
+    from axisem3d_amd.solver import GpuSolver
+    sp = _spec(nr, nr, "iso", "cg4", 5)
+    assert set(sp.elem_nr.tolist()) == {nr}
+    g = GpuSolver(sp, prec)
+    info = g.autotune_info()
+    g.close()
+    assert info["fused_elements"] == 0
+    # of the chip's 256 CUs
+    assert info["cardinal_blocks"] >= (5 if prec == "fp32" else 4) * 256
