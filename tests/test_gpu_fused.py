@@ -7,9 +7,11 @@ the source inside such an element.
 Domains: a spherical sector of three by two elements, axial ones among them,
 with element Nr 1 to 5 (single butterflies, even and odd, orders that are
 mean or Nyquist only), a ramp of small Nr with points of fewer orders than
-their element, primes, and a ramp over the largest Nr that fits the LDS of
-either precision, so that neighbouring elements take the two forms; all
-media, with no, CG4 and FULL attenuation of 5 and of 3 solids.
+their element, primes, and ramps over the Nr from which six elements take the
+three kernels; all media, with no, CG4 and FULL attenuation of 5 and of 3
+solids.  Larger ones: 48 elements at the largest Nr of either precision, a
+sector in which the two forms run side by side, and one whose elements make
+two launch groups.  Each asserts how many elements take the one-kernel form.
 
 Tolerances as for the other element kernels: relative 1e-13 (FP64) and 1e-5
 (FP32+FP64) per stage, 1e-12 and 1e-4 over the run."""
@@ -46,6 +48,21 @@ def _spec(nr0, nr1, mtype, att, nsls, ntheta=3, nrad=2):
     return sp
 
 
+def _fused(sp, prec):
+    """How many elements should take the one-kernel form: up to Nr 168 (FP32)
+    or 83 (FP64); of each medium, if there are larger ones in the domain, at
+    least 256, and at least 48 if one of them has Nr 120 (58) or more."""
+    top, big = {"fp32": (168, 120), "fp64": (83, 58)}[prec]
+    nr = np.asarray(sp.elem_nr)
+    n = 0
+    for mt in range(3):
+        q = nr[(np.asarray(sp.elem_mtype) == mt) & (nr <= top)]
+        few = (nr > top).any() and len(q) < 256
+        few |= len(q) < 48 and len(q) > 0 and q.max() >= big
+        n += 0 if few else len(q)
+    return n
+
+
 def _rel(a, b):
     return np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300)
 
@@ -65,6 +82,8 @@ def test_small_nr_matches_oracle(prec, tol, nr0, nr1, mtype, att, nsls):
     sp = _spec(nr0, nr1, mtype, att, max(nsls, 1))
     o = oracle.Oracle(sp)
     g = GpuSolver(sp, prec)
+    assert g.autotune_info()["fused_elements"] == _fused(sp, prec)
+    assert (_fused(sp, prec) > 0) == (nr1 < (190 if prec == "fp32" else 64))
     rng = np.random.default_rng(21)
     for k in range(2):
         u = rng.standard_normal((o.nmodes, 3)) + 1j * rng.standard_normal(
@@ -99,7 +118,10 @@ def test_small_nr_matches_oracle(prec, tol, nr0, nr1, mtype, att, nsls):
     ("fp64", 60, 8, 6, 48), ("fp64", 81, 8, 6, 48), ("fp64", 84, 8, 6, 0)])
 def test_form_by_count_and_size(prec, nr, ntheta, nrad, fused):
     from axisem3d_amd.solver import GpuSolver
-    sp = _spec(nr, nr, "iso", "cg4", 5, ntheta, nrad)
+    # the largest Nr with the media and attenuation of most operands
+    mtype, att, nsls = {168: ("aniso", "full", 5), 81: ("ti", "full", 3)}.get(
+        nr, ("iso", "cg4", 5))
+    sp = _spec(nr, nr, mtype, att, nsls, ntheta, nrad)
     assert set(sp.elem_nr.tolist()) == {nr}
     o = oracle.Oracle(sp)
     g = GpuSolver(sp, prec)
@@ -115,3 +137,46 @@ def test_form_by_count_and_size(prec, nr, ntheta, nrad, fused):
         print(f"{sp.n_solid_elements} of Nr {nr} {prec} pass {k}: {e:.2e}")
         assert e < (1e-13 if prec == "fp64" else 1e-5)
     g.close()
+
+
+def _stages(sp, prec, seed):
+    """Two stages against the oracle; the launches of the one-kernel form."""
+    from axisem3d_amd import capi
+    from axisem3d_amd.solver import GpuSolver
+    o = oracle.Oracle(sp)
+    g = GpuSolver(sp, prec)
+    fused = g.autotune_info()["fused_elements"]
+    assert fused == _fused(sp, prec)
+    g.profile(True)
+    rng = np.random.default_rng(seed)
+    for k in range(2):
+        u = rng.standard_normal((o.nmodes, 3)) + 1j * rng.standard_normal(
+            (o.nmodes, 3))
+        g.set_field("displ", u)
+        g.set_field("stiff", np.zeros_like(u))
+        g.computeStiffness()
+        e = _rel(g.get_field("stiff"), o.stiffness(u))
+        print(f"{fused} of {sp.n_solid_elements} {prec} pass {k}: {e:.2e}")
+        assert e < (1e-13 if prec == "fp64" else 1e-5)
+    n = [g.profile_read(k)[1] for k in (capi.KERNEL_CD_FUSED,
+                                        capi.KERNEL_CD_STRESS)]
+    g.close()
+    return fused, n[0] / 2, n[1] / 2
+
+
+@pytest.mark.parametrize("prec,nr1", [("fp32", 200), ("fp64", 100)])
+def test_two_forms_side_by_side(prec, nr1):
+    sp = _spec(9, nr1, "ti", "cg4", 5, 33, 10)
+    fused, one, three = _stages(sp, prec, 24)
+    assert 256 <= fused < sp.n_solid_elements
+    assert one == 1 and three >= 1
+
+
+# groups of at least 512: the second begins where two of its elements fit the
+# LDS of one of the first's largest
+@pytest.mark.parametrize("prec,nr1", [("fp32", 120), ("fp64", 81)])
+def test_two_launch_groups(prec, nr1):
+    sp = _spec(8, nr1, "iso", None, 0, 75, 20)
+    fused, one, three = _stages(sp, prec, 25)
+    assert fused == sp.n_solid_elements
+    assert one == 2 and three == 0

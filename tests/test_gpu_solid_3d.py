@@ -124,9 +124,8 @@ def _run(spec, prec, nsteps):
 
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
 def test_batching_does_not_change_results(prec, monkeypatch):
-    """A 50 KiB scratch splits the 3D elements into many batches (a few
-    elements each); the kernels see the same operands, so the fields are
-    bitwise those of the default (autotuned) batches."""
+    """The scratch budget is no concern of elements of small Nr, which take
+    the one-kernel form: the fields are bitwise those of the default."""
     nsteps = 60
     spec = _spec(nsteps)
     out = []
@@ -137,6 +136,7 @@ def test_batching_does_not_change_results(prec, monkeypatch):
             monkeypatch.setenv("AXS3D_CARD_SCRATCH_MB", mib)
         g = _solver(spec, prec)
         info = g.autotune_info()
+        assert info["fused_elements"] == spec.n_solid_elements
         g.run(nsteps)
         out.append((g.get_field("displ"), g.seismograms(), info))
         g.close()
@@ -145,3 +145,45 @@ def test_batching_does_not_change_results(prec, monkeypatch):
     assert np.array_equal(out[0][0], out[1][0])
     assert np.array_equal(out[0][1], out[1][1])
 
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_batches_of_the_three_kernels_do_not_change_results(prec,
+                                                            monkeypatch):
+    """24 elements of Nr 170 to 420, odd and even, of three media, in one
+    batch a medium, in batches of a few elements (1 MiB of scratch) and of one
+    (50 KiB): the kernels see the same operands, so the fields are the same
+    bit by bit.  The number of batches is that of the gradient's launches."""
+    from axisem3d_amd import capi
+    nsteps = 12
+    sp = preloop.spherical_regional(
+        ntheta=6, nrad=4, theta_max_deg=6.0, depth=200e3, nu_min=85,
+        nu_max=210, nsteps=nsteps, corr_len=80e3, bound_nr=False)
+    sp._courant /= 100.0
+    E = sp.n_solid_elements
+    preloop.make_media(sp, (np.arange(E) % 3).astype(np.uint8),
+                       field=sp._field, mask3d=np.ones(E, bool),
+                       att=sp._att_in, seed=4)
+    preloop.finish_regional(sp, nsteps, src_depth=60e3, f_peak=1.0,
+                            n_receivers=3, theta_max_deg=6.0)
+    nr = sp.elem_nr
+    assert nr.min() > 168 and len(set((nr % 2).tolist())) == 2
+    out, batches = [], []
+    for mib in ("4096", "1", "0.05"):
+        monkeypatch.setenv("AXS3D_CARD_SCRATCH_MB", mib)
+        g = _solver(sp, prec)
+        assert g.autotune_info()["fused_elements"] == 0
+        g.profile(True)
+        rng = np.random.default_rng(6)
+        for f in ("displ", "veloc"):
+            x = rng.standard_normal((g.nmodes, 3)) + \
+                1j * rng.standard_normal((g.nmodes, 3))
+            g.set_field(f, 1e-3 * x / (sp.dt if f == "veloc" else 1.0))
+        g.run(nsteps)
+        out.append((g.get_field("displ"), g.seismograms()))
+        batches.append(g.profile_read(capi.KERNEL_CD_GRAD)[1] / nsteps)
+        g.close()
+    assert batches[0] == 3 and 6 <= batches[1] < E and batches[2] == E
+    assert np.abs(out[0][1]).max() > 0
+    for x in out[1:]:
+        assert np.array_equal(out[0][0], x[0])
+        assert np.array_equal(out[0][1], x[1])

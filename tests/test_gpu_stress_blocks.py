@@ -5,7 +5,9 @@ memory enters the second), against the FP64 oracle.
 The ranges of Nr are those in which a block takes five, four, three, two and
 one points in either precision, each with odd Nr among them, so that the last
 block of an element is short (25 = 12 x 2 + 1 = 8 x 3 + 1 = 6 x 4 + 1) and the
-sixteen bytes a lane reads or writes end on a row's padding.
+sixteen bytes a lane reads or writes end on a row's padding (in FP32 the
+lowest range, 84 to 110, takes the one-kernel form; the others assert that
+none does).
 
 Tolerances as for the other element kernels: relative 1e-13 (FP64) and 1e-5
 (FP32+FP64)."""
@@ -51,6 +53,9 @@ def test_stress_blocks_match_oracle(prec, tol, nr0, nr1, mtype, att, nsls):
     sp = _spec(nr0, nr1, mtype, att, max(nsls, 1))
     o = oracle.Oracle(sp)
     g = GpuSolver(sp, prec)
+    one = prec == "fp32" and nr1 <= 110
+    assert g.autotune_info()["fused_elements"] == (
+        sp.n_solid_elements if one else 0)
     rng = np.random.default_rng(22)
     for k in range(2):
         u = rng.standard_normal((o.nmodes, 3)) + 1j * rng.standard_normal(

@@ -27,6 +27,20 @@ def _solid3d_att():
     return spec
 
 
+def _solid3d_large():
+    # 96 elements of Nr above 1000: 60 MiB of rows and more, of a static
+    # scratch of 64 (batches in FP64)
+    spec = preloop.spherical_regional(
+        ntheta=12, nrad=8, theta_max_deg=6.0, depth=300e3, nu_min=550,
+        nu_max=600, nsteps=50, n_receivers=3, attenuation=True, cg4=True,
+        corr_len=80e3, bound_nr=False)
+    spec._build_3d(np.ones(spec.n_solid_elements, bool))
+    preloop.finish_regional(spec, 50, src_depth=60e3, f_peak=0.5,
+                            n_receivers=3, theta_max_deg=6.0)
+    assert spec.elem_nr.min() > 1000
+    return spec
+
+
 def _fluid3d():
     # a fluid layer inside a solid, half the fluid elements 3D
     mesh = preloop.StructuredMesh(np.linspace(0, 4e3, 5),
@@ -81,6 +95,18 @@ def _call_both(ga, gb):
         assert np.abs(a).max() > 0
         out.append((name, a, b))
     return out
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_static_scratch_of_the_three_kernels(prec):
+    """Elements too large for the one-kernel form, which needs no scratch."""
+    a, b = _pair(_solid3d_large(), prec, 13)
+    assert b.autotune_info()["fused_elements"] == 0
+    for _ in range(2):
+        for name, x, y in _call_both(a, b):
+            assert np.array_equal(x, y), (name, np.abs(x - y).max())
+    for g in (a, b):
+        g.close()
 
 
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
