@@ -33,6 +33,16 @@ METRIC = ("GLL-point*mode updates/s, FP32-batched vs FP64 plain at <=1e-4 "
           "seismogram L2")
 UNIT = "GLL-point*mode updates/s"
 HBM_PEAK_GBS = 8000.0
+# The library replays its steps in graphs of eight, captured in the first run
+# with so many between its first and its last step.
+GRAPH_STEPS = 8
+CAPTURE_RUN = GRAPH_STEPS + 2
+
+
+def replay_run(steps):
+    """A run of at least `steps` steps that is replays but for its last step,
+    which writes the velocity and the acceleration."""
+    return -(-steps // GRAPH_STEPS) * GRAPH_STEPS + 1
 
 
 def log(msg):
@@ -134,7 +144,14 @@ def build_workload(name, nsteps):
     return spec, cfg
 
 
-def bytes_per_step(spec, real, fused_nr=0):
+def marches_half(spec):
+    """Whether a run marches displacement and w = v + dt/2 a (Newmark without
+    absorbing boundaries) in place of u, v and a."""
+    return (getattr(spec, "time_scheme", "newmark") == "newmark" and
+            not getattr(spec, "_abc_abi", None))
+
+
+def bytes_per_step(spec, real, fused_nr=0, run_steps=0):
     """Algorithmic HBM bytes of one step, by kernel: every array touched
     once, intermediates (the cardinal scratch, the element-local forces'
     read by the point kernel aside) on chip.
@@ -150,9 +167,10 @@ def bytes_per_step(spec, real, fused_nr=0):
       integral-factor rows.
     cd_fused: the same three of the 3D elements with Nr <= fused_nr,
       which run as one kernel.
-    point: element forces read, u, v, a read+written (FP64), per-point
-      data: the plain Newmark update's (a run of several steps marches two
-      fields and moves 96 B less)."""
+    point: element forces read, per-point data, and the state read and
+      written (FP64): u, v, a in the plain Newmark update; u and w in a run
+      of run_steps steps that marches them, whose last step writes v and a
+      too."""
     nupd = spec.n_updates_per_step()
     E, U = spec.n_solid_elements, spec.n_solid_points
     nr = spec.elem_nr.astype(np.int64)
@@ -186,7 +204,10 @@ def bytes_per_step(spec, real, fused_nr=0):
     n1 = int((~is3d).sum())
     fr = (nupd - updf - upd3) * (48 + 6 * real) + n1 * (
         10 * 25 * real + 25 * 4 + 1 + 25 * real * 2)
-    point = nupd * (6 * real + 6 * 48 + 4) + U * (4 + 4 + 4 + 1 + 8 + 16)
+    state = 6 * 48
+    if run_steps > 0 and marches_half(spec):
+        state = 4 * 48 + 2 * 48 / run_steps
+    point = nupd * (6 * real + state + 4) + U * (4 + 4 + 4 + 1 + 8 + 16)
     return {"fr": int(fr), "cd_grad": int(grad), "cd_stress": int(stress),
             "cd_quad": int(quad), "cd_fused": int(sum(f3)),
             "point": int(point)}
@@ -252,18 +273,24 @@ def pmc_traffic(kernel, workload):
     return (fetch_kib * fetch_fac + write_kib * write_fac) * 1024.0
 
 
+def bench_steps(steps, warmup):
+    """Steps of the timed legs of a precision: warm-up, launched steps, the
+    run that captures, replayed steps."""
+    return warmup + steps + CAPTURE_RUN + replay_run(steps)
+
+
 def time_gpu(spec, prec, steps, warmup, graph=False, total=0):
     """Times `steps` steps launched kernel by kernel with HIP events around
     every kernel (the per-kernel averages come from these same steps);
-    with graph, then the same number of steps as replays of the captured
-    step graph, without events.  With total, the run then goes on
+    with graph, then a run of replays of the captured steps, without events,
+    after one that captures them.  With total, the run then goes on
     (untimed) to `total` steps from rest, and the seismograms of all of
     them are returned (the accuracy leg)."""
     from axisem3d_amd import capi
     from axisem3d_amd.solver import GpuSolver
     t0 = time.perf_counter()
     g = GpuSolver(spec, prec,
-                  max_samples=max(total, 2 * steps + warmup + 1))
+                  max_samples=max(total, bench_steps(steps, warmup)))
     tune = g.autotune_info()
     log(f"{prec}: set-up {time.perf_counter() - t0:.1f} s, "
         f"{g.nmodes} point-modes, autotune {tune}")
@@ -280,13 +307,15 @@ def time_gpu(spec, prec, steps, warmup, graph=False, total=0):
     log(f"{prec}: {steps} steps in {t1 - t0:.3f} s")
     prof["autotune"] = tune
     if graph:
-        g.run(1)    # captures the step graph outside the timed region
+        g.run(CAPTURE_RUN)      # the capture, outside the timed region
         g.synchronize()
+        n = replay_run(steps)
         t2 = time.perf_counter()
-        g.run(steps)
+        g.run(n)
         g.synchronize()
         prof["graph_s"] = time.perf_counter() - t2
-        log(f"{prec}: {steps} graph replays in {prof['graph_s']:.3f} s")
+        log(f"{prec}: {n} steps, {n - 1} of them replayed, in "
+            f"{prof['graph_s']:.3f} s")
     if total > g.step:
         t3 = time.perf_counter()
         g.run(total - g.step)
@@ -415,8 +444,9 @@ def accuracy_leg(spec, seis32, seis64):
 
 def batched_extras(spec, seis32, seis64, steps, warmup, t_batch):
     """Per-instance seismogram L2 of FP32+FP64 against FP64, and the time
-    of the same instances run one after the other, each alone (graph
-    replays, against the batch's graph replays t_batch)."""
+    of the same instances run one after the other, each alone (`steps`
+    steps as replays after a run that captures them, as the batch's
+    t_batch)."""
     from axisem3d_amd.solver import GpuSolver
     out = {"seismogram_rel_l2_vs_fp64": [], "alone_ms_per_step": []}
     for i, (_, _, (r0, r1)) in enumerate(spec._instances):
@@ -460,9 +490,10 @@ def adjoint_bench(a):
     sp = adjoint.with_model(spec, *model)
     g = GpuSolver(sp, "fp32", max_samples=nsteps)
     g.run(nsteps)          # warm-up of the forward (graph capture)
+    for f in ("displ", "veloc", "accel"):
+        g.set_field(f, np.zeros((g.nmodes, 3), complex))
+    g.step = 0
     g.synchronize()
-    g.close()
-    g = GpuSolver(sp, "fp32", max_samples=nsteps)
     t0 = time.perf_counter()
     g.run(nsteps)
     g.synchronize()
@@ -509,11 +540,11 @@ def main():
         adjoint_bench(a)
         return
     from axisem3d_amd import capi
-    # warm-up, timed steps, one capture step and the graph replays; both
-    # precisions then run on to the accuracy leg's step count
-    acc = 0 if a.no_fp64 else max(a.accuracy_steps, 2 * a.steps + a.warmup
-                                  + 1)
-    nsteps = max(2 * a.steps + a.warmup + 1, acc)
+    # the timed legs; both precisions then run on to the accuracy leg's step
+    # count
+    nsteps = bench_steps(a.steps, a.warmup)
+    acc = 0 if a.no_fp64 else max(a.accuracy_steps, nsteps)
+    nsteps = max(nsteps, acc)
     t0 = time.perf_counter()
     spec, cfg = build_workload(a.workload, nsteps)
     log(f"workload built in {time.perf_counter() - t0:.1f} s: "
@@ -548,7 +579,7 @@ def main():
              capi.KERNEL_RECORD: "receivers"}
     tune32 = prof32.pop("autotune")
     b = bytes_per_step(spec, 4, tune32["fused_nr_max"]
-                       if tune32["fused_elements"] else 0)
+                       if tune32["fused_elements"] else 0, a.steps)
     # algorithmic bytes per step of each timed group
     byts = {capi.KERNEL_STIFFNESS: b["fr"],
             capi.KERNEL_STIFFNESS_3D: b["cd_grad"] + b["cd_stress"] +
@@ -569,7 +600,7 @@ def main():
             "avg_us": ms / cnt * 1e3,
             "bytes_per_launch": byts[k] / per_step,
             "achieved_GBs": byts[k] / (ms / a.steps * 1e-3) / 1e9}
-    tg = prof32.pop("graph_s")
+    tg, ng = prof32.pop("graph_s"), replay_run(a.steps)
     if out_64 is not None:
         prof64.pop("autotune")
     # dominant single kernel (the cardinal group is three kernels)
@@ -604,14 +635,16 @@ def main():
                           "frac": step_bytes / (t32 / a.steps) / 1e9 /
                           HBM_PEAK_GBS},
         "kernels": kernels,
-        "graph_replay": {"ms_per_step": tg / a.steps * 1e3,
-                         "value": nupd * a.steps / tg},
+        "graph_replay": {"steps": ng, "replayed_steps": ng - 1,
+                         "ms_per_step": tg / ng * 1e3,
+                         "value": nupd * ng / tg},
         "autotune": tune32,
     }
     if a.workload == "batched":
         out["per_instance"] = batched_extras(spec, seis32,
                                              seis64 if out_64 else None,
-                                             a.steps, a.warmup, tg)
+                                             ng, max(a.warmup, CAPTURE_RUN),
+                                             tg)
     if not a.no_cpu:
         t0 = time.perf_counter()
         out["cpu_baseline"] = cpu_baseline(spec, a.cpu_seconds, a.workload)

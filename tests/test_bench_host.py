@@ -32,6 +32,28 @@ def test_bytes_per_step_counts_each_array_once():
     assert b["cd_grad"] == b["cd_stress"] == b["cd_quad"] == 0
     assert b["point"] >= nupd * (6 * 4 + 6 * 48)
     assert b["fr"] > nupd * 48
+    # a run marches u and w = v + dt/2 a, and writes v and a in its last step;
+    # with absorbing boundaries, or in the symplectic scheme, it does not
+    r = bench.bytes_per_step(sp, 4, run_steps=20)
+    assert b["point"] - r["point"] == nupd * 2 * 48 - nupd * 2 * 48 // 20
+    sp.time_scheme = "symplectic"
+    assert bench.bytes_per_step(sp, 4, run_steps=20) == b
+    sp.time_scheme = "newmark"
+    sp._abc_abi = {"sponge_solid": {0: [1.0]}}
+    assert bench.bytes_per_step(sp, 4, run_steps=20) == b
+
+
+def test_the_timed_replays_are_replays():
+    """Eight steps a graph: the run that captures is long enough for one
+    whatever came before it (the first step may form w, the last writes v and
+    a), and in the timed one all but the last step are replayed."""
+    import bench
+    assert bench.CAPTURE_RUN - 2 == bench.GRAPH_STEPS == 8
+    for steps in (1, 7, 8, 9, 20, 60):
+        n = bench.replay_run(steps)
+        assert n > steps and (n - 1) % bench.GRAPH_STEPS == 0
+        assert n - 1 < steps + bench.GRAPH_STEPS
+        assert bench.bench_steps(steps, 5) == 5 + steps + bench.CAPTURE_RUN + n
 
 
 def test_profile_lookups():
