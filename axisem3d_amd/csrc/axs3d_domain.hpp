@@ -165,7 +165,7 @@ public:
     // bulk
     void solve(int step_begin, int nsteps);
     void setRecordOrigin(int step0) { mRecordStep0 = step0; }
-    // replay a captured step graph in solve (default) or launch eagerly
+    // replay the captured steps in solve (default) or launch eagerly
     void useGraph(bool on) { mUseGraph = on; }
     void readSeismograms(double *out, int nsamples);
 

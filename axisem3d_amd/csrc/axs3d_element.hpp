@@ -14,6 +14,12 @@ namespace axs3d {
 
 constexpr int STIFF_BLOCK = 256;
 
+// CG4 attenuation points (1,1),(1,3),(3,1),(3,3) (AttBuilder.cpp:141-147).
+__device__ __forceinline__ int att_slot(int p, int npa) {
+    if (npa == NPEM) return p;
+    return p == 6 ? 0 : p == 8 ? 1 : p == 16 ? 2 : p == 18 ? 3 : -1;
+}
+
 template <typename Real>
 struct PointOps {                // inverse-Jacobian entries and 1/s
     Real dsdxii, dsdeta, dzdxii, dzdeta, invs;

@@ -30,12 +30,6 @@
 
 namespace axs3d {
 
-// CG4 attenuation points (1,1),(1,3),(3,1),(3,3) (AttBuilder.cpp:141-147).
-__device__ __forceinline__ int att_slot_fr(int p, int npa) {
-    if (npa == NPEM) return p;
-    return p == 6 ? 0 : p == 8 ? 1 : p == 16 ? 2 : p == 18 ? 3 : -1;
-}
-
 // SLS memory per Fourier order with 1D moduli (AttenuationFull/CG4::apply,
 // AttenuationCG4.hpp:312-330, Attenuation.hpp:92-140): sigma -= sum_l m_l;
 // m_l = alpha_l m_l + beta_l ds_old; ds = iso(dlambda, dmu)(eps); m_l +=
@@ -223,7 +217,7 @@ __global__ __launch_bounds__(STIFF_BLOCK) void k_solid_stiff_fr(
                 eps, [&](int k) { return mat[k * NPEM]; }, sig);
         }
         if constexpr (ATT != ATT_NONE) {
-            const int qa = att_slot_fr(ipnt, a.npa);
+            const int qa = att_slot(ipnt, a.npa);
             if (qa >= 0) {
                 const Real *dlm = a.att1d + (size_t)e * 2 * a.npa + qa;
                 cpx<Real> dsn[6];
@@ -253,7 +247,7 @@ __global__ __launch_bounds__(STIFF_BLOCK) void k_solid_stiff_fr(
             *ds = dsn;
         }
         __syncthreads();
-        const int qa = att_slot_fr(ipnt, 4);
+        const int qa = att_slot(ipnt, 4);
         if (active && qa >= 0)
 #pragma unroll
             for (int d = 0; d < 6; d++) {

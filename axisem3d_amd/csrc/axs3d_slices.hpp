@@ -8,12 +8,6 @@
 
 namespace axs3d {
 
-// CG4 attenuation points (1,1),(1,3),(3,1),(3,3) (AttBuilder.cpp:141-147).
-__device__ __forceinline__ int att_slot(int p, int npa) {
-    if (npa == NPEM) return p;
-    return p == 6 ? 0 : p == 8 ? 1 : p == 16 ? 2 : p == 18 ? 3 : -1;
-}
-
 // Per-slice operands of an element: its base addresses, the same for the
 // whole block (they stay in scalar registers), and the lane's place in a
 // component's row: parameter c of slice k at point p sits at par[c * ps + p

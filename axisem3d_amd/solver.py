@@ -297,7 +297,7 @@ class GpuSolver:
         self.step += nsteps
 
     def use_graph(self, enable=True):
-        """Replay one captured step graph per step in run() (the default),
+        """Replay graphs of several captured steps in run() (the default),
         or launch every kernel from the host."""
         self._chk(self.lib.axs3d_set_graph(self.ctx, int(bool(enable))),
                   "set_graph")

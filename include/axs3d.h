@@ -67,7 +67,11 @@ enum axs3d_field {
 enum axs3d_kernel_id {
     AXS3D_KERNEL_STIFFNESS = 0,   /* Fourier-path (1D) element stiffness */
     AXS3D_KERNEL_POINT = 1,       /* fused BC/mass/Newmark point update  */
+    /* axs3d_apply_sources; within a run the source is part of the element
+     * kernels and this reads zero */
     AXS3D_KERNEL_SOURCE = 2,
+    /* axs3d_record, the symplectic scheme, and runs whose receivers have a
+     * launch of their own; elsewhere they are part of the element kernels */
     AXS3D_KERNEL_RECORD = 3,
     AXS3D_KERNEL_STIFFNESS_3D = 4,/* cardinal-path (3D) element stiffness */
     AXS3D_KERNEL_FLUID_STIFFNESS = 5, /* fluid element stiffness       */
@@ -437,7 +441,11 @@ int axs3d_check_stability(axs3d_ctx *ctx, int tstep);
 /* NewmarkTimeScheme::solve (src/core/time/NewmarkTimeScheme.cpp:18-131)
  * over steps [step_begin, step_begin + nsteps), recording every step into
  * the seismogram buffer at sample (tstep - record_step0).  The
- * BC-after/mass/Newmark phases run as one fused kernel. */
+ * BC-after/mass/Newmark phases run as one fused kernel.  A run that goes on
+ * from the displacement, velocity and acceleration (and the fluid's) that
+ * axs3d_get_field gave after an earlier one, in the same context or set into
+ * another, takes bitwise the steps of one unbroken run, without attenuation
+ * (whose memory variables no call reads). */
 int axs3d_run(axs3d_ctx *ctx, int step_begin, int nsteps);
 int axs3d_set_record_origin(axs3d_ctx *ctx, int record_step0);
 /* Launch form of axs3d_run, no counterpart in the reference (its steps are
